@@ -1,0 +1,409 @@
+"""Performance cases: the work a user of cm1_amd has it do.
+
+Two kinds of program use the library: a model run (large steps of one model
+or of a batched ensemble, the state resident on the GPU) and the training and
+use of the learned Kessler surrogate.  A case is one pass of such a program's
+inner loop.
+
+Stepping cases come in the two ways a host holds the state:
+
+* ``out = "host"``: the driver advances the model by some steps and fetches
+  the prognostic fields (history output, plotting);
+* ``out = "device"``: a program that works on the state on the GPU, between
+  steps, through the addresses ``cm1g_field_ptr`` hands out (asked for again
+  after every step, as the interface requires), here as torch tensors.
+
+Initial states are made on the GPU from the seed: the Weisman-Klemp
+supercell environment with storms that already hold cloud water, rain and
+updraughts, so that every process of the Kessler branch acts, or the dry
+convective boundary layer with its tracers and, where the subgrid turbulence
+is on, a mixed layer that is already turbulent.
+"""
+import ctypes as C
+import math
+
+import numpy as np
+import torch
+
+from cm1_amd import _native as N
+from cm1_amd import init, model, surrogate, workloads
+
+DEV = "cuda"
+
+
+# --------------------------------------------------------------------- cases
+def _storm(name, ni, nj, nk, steps, out, **kw):
+    c = dict(name=name, kind="storm", ni=ni, nj=nj, nk=nk, steps=steps, out=out, stretch=False, bc=2,
+             psolver=3, weno=0, npt=0, rdamp=0, net=False)
+    c.update(kw)
+    return c
+
+
+def _cbl(name, ni, nj, nk, steps, out, npt=6, turb=True, impl=True):
+    return dict(name=name, kind="cbl", ni=ni, nj=nj, nk=nk, steps=steps, out=out, npt=npt, turb=turb,
+                impl=impl)
+
+
+def listed():
+    return [
+        # the largest run: the 1024 x 1024 x 96 supercell on the stretched
+        # grid that the framework's benchmark steps
+        _storm("storm_1024x1024x96", 1024, 1024, 96, 1, "device", stretch=True),
+        # an ordinary regional run whose sizes fit no tile
+        _storm("storm_301x227x63", 301, 227, 63, 8, "host", rdamp=1),
+        # the 64 x 64 x 40 supercell, 1 km: the first case a user runs, small
+        # enough that launches and latency decide
+        _storm("storm_64x64x40", 64, 64, 40, 20, "host"),
+        # the other options in earnest: doubly periodic sides, WENO5 scalar
+        # advection, the explicit acoustic solver, tracers
+        _storm("storm_periodic_weno_192x160x48", 192, 160, 48, 4, "device", bc=1, psolver=2, weno=1, npt=2),
+        # the supercell with the learned Kessler surrogate in its step
+        _storm("storm_surrogate_256x256x64", 256, 256, 64, 4, "device", net=True),
+        # large-eddy simulation of the dry convective boundary layer: subgrid
+        # turbulence, six tracers, WENO5
+        _cbl("cbl_512x512x128", 512, 512, 128, 1, "device"),
+        # the same on a test-sized grid
+        _cbl("cbl_64x48x40", 64, 48, 40, 10, "host"),
+        # an ensemble of members that each leave the chip mostly idle, and one
+        # whose members do not
+        dict(name="ensemble_32_small", kind="ensemble", members=32, small=True, steps=4),
+        dict(name="ensemble_8", kind="ensemble", members=8, small=False, steps=2),
+        # surrogate training: one minibatch of the trainer's default size,
+        # forward and backward
+        dict(name="surrogate_grad_65536", kind="grad", rows=65536),
+        # surrogate inference on a large batch, and on a handful of columns
+        dict(name="surrogate_forward_4194304", kind="forward", rows=4194304),
+        dict(name="surrogate_forward_1000", kind="forward", rows=1000),
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(["storm", "storm", "storm", "cbl", "ensemble", "grad", "forward"])
+    if kind == "grad":
+        return dict(kind="grad", rows=_log_int(rng, 512, 262144))
+    if kind == "forward":
+        return dict(kind="forward", rows=_log_int(rng, 100, 4194304))
+    if kind == "ensemble":
+        small = rng.random() < 0.5
+        return dict(kind="ensemble", members=rng.randint(3, 48) if small else rng.randint(2, 10), small=small,
+                    steps=rng.randint(1, 4))
+    if kind == "cbl":
+        ni, nj, nk = _log_int(rng, 24, 512), _log_int(rng, 24, 512), rng.randint(24, 128)
+        steps = 1 if ni * nj * nk > 2000000 else rng.randint(2, 8)
+        out = "device" if steps == 1 else rng.choice(["host", "device"])
+        c = _cbl("", ni, nj, nk, steps, out, npt=rng.randint(0, 6), turb=rng.random() < 0.7,
+                 impl=rng.random() < 0.7)
+    else:
+        ni, nj = _log_int(rng, 24, 800), _log_int(rng, 24, 800)
+        stretch = rng.random() < 0.25
+        nk = 96 if stretch else rng.randint(20, 90)
+        steps = 1 if ni * nj * nk > 4000000 else rng.randint(2, 10)
+        out = "device" if steps == 1 else rng.choice(["host", "device"])
+        psolver = 2 if rng.random() < 0.2 else 3
+        c = _storm("", ni, nj, nk, steps, out, stretch=stretch, bc=rng.choice([1, 2, 2]), psolver=psolver,
+                   weno=rng.choice([0, 0, 0, 1, 2]), npt=rng.choice([0, 0, 1, 3]), rdamp=rng.choice([0, 1]),
+                   net=rng.random() < 0.15)
+    c.pop("name")
+    return c
+
+
+# -------------------------------------------------------------------- states
+class _View:
+    """A device field as an object torch takes without copying; it keeps the
+    model that owns the memory alive."""
+
+    def __init__(self, owner, ptr, n):
+        self.owner = owner
+        self.__cuda_array_interface__ = dict(shape=(n,), typestr="<f4", data=(ptr, False), version=3, strides=None)
+
+
+def _field(m, name):
+    """The whole padded box of a field as a (pz, py, px) tensor on the GPU."""
+    p = C.c_void_p()
+    N.check(m.L.cm1g_field_ptr(m.h, N.FID[name], C.byref(p)), "cm1g_field_ptr")
+    return torch.as_tensor(_View(m, p.value, m.px * m.py * m.pz), device=DEV).view(m.pz, m.py, m.px)
+
+
+def _inside(m, name, stag=None):
+    """The part of a device field that its loops cover (i = 1..ni, plus the
+    last face along a staggered direction)."""
+    ei, ej, ek = stag == "u", stag == "v", stag == "w"
+    return _field(m, name)[1:m.nk + 1 + ek, 3:m.nj + 3 + ej, 32:m.ni + 32 + ei]
+
+
+def _generator(seed):
+    g = torch.Generator(device=DEV)
+    g.manual_seed(int(seed))
+    return g
+
+
+def _load(m, boxes, on_device):
+    """Initial fields, logical boxes (nk+3, nj+7, ni+7), into the model."""
+    if on_device:
+        for name, a in boxes.items():
+            _field(m, name)[:, :, 29:29 + m.ni + 7] = a
+        torch.cuda.synchronize()
+    else:
+        for name, a in boxes.items():
+            m.put(name, a.cpu().numpy())
+    m.getset(True)
+
+
+def _storm_model(ni, nj, nk, seed, *, stretch=False, bc=2, psolver=3, weno=0, npt=0, rdamp=0, on_device=False,
+                 umax=25.0, qv_scale=1.0):
+    """A supercell environment with a few mature storms."""
+    if stretch:
+        dx, dz, dt, nsound, st = 250.0, workloads.CONFIG1_DZ, 1.5, 8, workloads.CONFIG1_STRETCH
+    else:
+        dx, dz, dt, nsound, st = 1000.0, 20000.0 / nk, 4.0, 6, None
+    if psolver == 2:
+        nsound = 0  # the explicit solver's count follows from the smallest spacing
+    cols, dzn = init.vertical_grid(nk, dz, st)
+    cols.update(init.wk_sounding(cols["zh"], nk, qv_scale=qv_scale))
+    cols["u0"] = init.wind_iwnd4(cols["zh"], nk, umax)
+    cfg = model.make_config(ni=ni, nj=nj, nk=nk, wbc=bc, ebc=bc, sbc=bc, nbc=bc, psolver=psolver,
+                            advwenos=weno, advwenov=0, nsound=nsound, npt=npt, dx=dx, dy=dx, dz=dzn, dt=dt,
+                            irdamp=rdamp, zd=15000.0, min_dz=init.min_dz(cols["zf"], nk) if st else dzn)
+    m = model.Model(cfg)
+    m.set_columns(cols)
+    g = _generator(seed)
+    box = (nk + 3, nj + 7, ni + 7)
+    k, j, i = slice(1, nk + 1), slice(3, nj + 3), slice(3, ni + 3)
+    col = lambda n: torch.from_numpy(cols[n][:nk + 3].copy()).to(DEV)[:, None, None]  # noqa: E731
+    noise = lambda amp: (torch.rand((nk, nj, ni), device=DEV, generator=g) * 2.0 - 1.0) * amp  # noqa: E731
+    zh = torch.from_numpy(cols["zh"][1:nk + 1].copy()).to(DEV)[:, None, None]
+    x = torch.arange(ni, device=DEV, dtype=torch.float32)[None, None, :]
+    y = torch.arange(nj, device=DEV, dtype=torch.float32)[None, :, None]
+    # storms: one per 60 x 60 km or so, warm, moist and rising, cloud in the
+    # middle levels and rain below and around
+    core = torch.zeros((nk, nj, ni), device=DEV)
+    rain = torch.zeros((nk, nj, ni), device=DEV)
+    for _ in range(max(1, min(12, int(ni * nj * dx * dx / 3.6e9) + 1))):
+        px, py, pr = torch.rand(3, device=DEV, generator=g).tolist()
+        cx, cy, r = (0.15 + 0.7 * px) * ni, (0.15 + 0.7 * py) * nj, min((6.0 + 4.0 * pr) * 1000.0 / dx, 0.25 * min(ni, nj))
+        h2 = ((x - cx) / r) ** 2 + ((y - cy) / r) ** 2
+        core = torch.maximum(core, torch.clamp(1.0 - h2 - ((zh - 4500.0) / 4000.0) ** 2, min=0.0))
+        h2 = ((x - cx - 0.3 * r) / (1.3 * r)) ** 2 + ((y - cy) / (1.3 * r)) ** 2
+        rain = torch.maximum(rain, torch.clamp(1.0 - h2 - ((zh - 2500.0) / 3500.0) ** 2, min=0.0))
+    f = {}
+    f["ua"] = col("u0").expand(box).contiguous()
+    f["ua"][k, j, i] += noise(0.2)
+    f["va"] = torch.zeros(box, device=DEV)
+    f["va"][k, j, i] = noise(0.2)
+    f["wa"] = torch.zeros(box, device=DEV)
+    f["wa"][2:nk + 1, j, i] = 12.0 * core[1:] * (1.0 + noise(0.1)[1:])
+    f["tha"] = torch.zeros(box, device=DEV)
+    f["tha"][k, j, i] = 2.5 * core + noise(0.1)
+    f["qa0"] = col("qv0").expand(box).contiguous()
+    f["qa0"][k, j, i] *= 1.0 + 0.25 * core + noise(0.01)
+    f["qa1"] = torch.zeros(box, device=DEV)
+    f["qa1"][k, j, i] = 2.0e-3 * core
+    f["qa2"] = torch.zeros(box, device=DEV)
+    f["qa2"][k, j, i] = 3.0e-3 * rain
+    for t in range(npt):
+        f[f"pta{t}"] = torch.zeros(box, device=DEV)
+        f[f"pta{t}"][k, j, i] = torch.where(zh < 1000.0 * (t + 1), 1.0, 0.0) * (1.0 + noise(0.05))
+    _load(m, f, on_device)
+    return m
+
+
+def _cbl_model(ni, nj, nk, seed, *, npt, turb, impl, on_device):
+    """The dry convective boundary layer (20 m, doubly periodic)."""
+    cols, dzn = init.vertical_grid(nk, 20.0, None)
+    cols.update(init.cbl_sounding(cols["zh"], nk))
+    cols["u0"] = np.zeros(nk + 3, np.float32)
+    cols["u0"][1:nk + 1] = 10.0
+    cfg = model.make_config(ni=ni, nj=nj, nk=nk, wbc=1, ebc=1, sbc=1, nbc=1, imoist=0, ptype=0, psolver=2,
+                            advwenos=1, advwenov=0, nsound=0, npt=npt, dx=20.0, dy=20.0, dz=dzn, dt=0.25)
+    m = model.Model(cfg)
+    m.set_columns(cols)
+    if turb:
+        m.set_turbulence(**dict(workloads.CBL_TURB, doimpl=int(impl)))
+    g = _generator(seed)
+    box = (nk + 3, nj + 7, ni + 7)
+    k, j, i = slice(1, nk + 1), slice(3, nj + 3), slice(3, ni + 3)
+    zh = torch.from_numpy(cols["zh"][1:nk + 1].copy()).to(DEV)[:, None, None]
+    zf = torch.from_numpy(cols["zf"][1:nk + 1].copy()).to(DEV)[:, None, None]
+    noise = lambda amp: (torch.rand((nk, nj, ni), device=DEV, generator=g) * 2.0 - 1.0) * amp  # noqa: E731
+    mixed = torch.clamp(1.0 - zh / 1000.0, min=0.0)
+    f = {}
+    f["ua"] = torch.zeros(box, device=DEV)
+    f["ua"][1:nk + 1] = 10.0
+    f["ua"][k, j, i] += noise(0.5) * mixed
+    f["va"] = torch.zeros(box, device=DEV)
+    f["va"][k, j, i] = noise(0.5) * mixed
+    f["tha"] = torch.zeros(box, device=DEV)
+    f["tha"][k, j, i] = noise(0.1) * (zh < 500.0)
+    x = torch.arange(ni, device=DEV, dtype=torch.float32)[None, None, :]
+    y = torch.arange(nj, device=DEV, dtype=torch.float32)[None, :, None]
+    for t in range(npt):
+        cx, cy, cz = torch.rand(3, device=DEV, generator=g).tolist()
+        r2 = ((x - (0.2 + 0.6 * cx) * ni) ** 2 + (y - (0.2 + 0.6 * cy) * nj) ** 2) * 400.0
+        r2 = r2 + (zh - (0.2 + 0.4 * cz) * nk * 20.0) ** 2
+        f[f"pta{t}"] = torch.zeros(box, device=DEV)
+        f[f"pta{t}"][k, j, i] = torch.exp(-0.5 * r2 / 200.0 ** 2)
+    if turb:
+        f["tkea"] = torch.zeros(box, device=DEV)
+        f["tkea"][k, j, i] = 0.4 * torch.clamp(1.0 - zf / 1000.0, min=0.0) * (1.0 + noise(0.5)) * (zf > 0.0)
+    _load(m, f, on_device)
+    return m
+
+
+def _outputs(case):
+    """The fields of a model's state that a pass returns, with staggering."""
+    out = [("ua", "u"), ("va", "v"), ("wa", "w"), ("tha", None), ("ppi", None), ("rho", None), ("prs", None)]
+    if case["kind"] != "cbl":
+        out += [("qa0", None), ("qa1", None), ("qa2", None)]
+    out += [(f"pta{t}", None) for t in range(case.get("npt", 0))]
+    if case.get("turb"):
+        out += [("tkea", "w")]
+    return out
+
+
+def _net_inputs(rows, seed):
+    g = _generator(seed)
+    return torch.randn((rows, 8), device=DEV, generator=g), g
+
+
+def _params(seed, scale=1.0):
+    """Weights of the 8-128-128-128-4 network as a training run meets them
+    (scaled normal weights, small biases), flat as Net.set_params takes them."""
+    rng = np.random.default_rng(seed)
+    parts = []
+    for fin, fout in ((8, 128), (128, 128), (128, 128), (128, 4)):
+        parts.append(rng.standard_normal(fin * fout) * scale * math.sqrt(2.0 / fin))
+        parts.append(rng.standard_normal(fout) * 0.05)
+    return np.concatenate(parts).astype(np.float32)
+
+
+def prepare(case, seed):
+    kind = case["kind"]
+    if kind == "storm":
+        m = _storm_model(case["ni"], case["nj"], case["nk"], seed, stretch=case["stretch"], bc=case["bc"],
+                         psolver=case["psolver"], weno=case["weno"], npt=case["npt"], rdamp=case["rdamp"],
+                         on_device=case["out"] == "device")
+        s = dict(case=case, m=m, outputs=_outputs(case))
+        if case["net"]:
+            net = surrogate.Net(seed=1)
+            net.set_params(_params(seed, 0.7))
+            # T, p, rho, qv, qc, qr, dt, z/ztop and the changes of theta, qv,
+            # qc, qr: means, deviations, then the trusted range
+            net.set_norm(np.array([270.0, 6.0e4, 0.8, 8.0e-3, 5.0e-4, 1.0e-3, 4.0, 0.3,
+                                   25.0, 2.0e4, 0.3, 5.0e-3, 5.0e-4, 1.0e-3, 1.0, 0.25,
+                                   -1.0e-2, 1.0e-6, -2.0e-5, 2.0e-5, 1.0e-2, 2.0e-6, 4.0e-5, 4.0e-5] +
+                                  [-40.0] * 8 + [40.0] * 8, np.float32))
+            surrogate.use(m, net)
+            s["net"] = net
+        return s
+    if kind == "cbl":
+        m = _cbl_model(case["ni"], case["nj"], case["nk"], seed, npt=case["npt"], turb=case["turb"],
+                       impl=case["impl"], on_device=case["out"] == "device")
+        return dict(case=case, m=m, outputs=_outputs(case))
+    if kind == "ensemble":
+        shapes = workloads.ensemble_small_shapes(case["members"]) if case["small"] else \
+            workloads.ensemble_shapes(case["members"])
+        ms = [_storm_model(ni, nj, nk, 1000 * seed + n, umax=umax, qv_scale=qvs, on_device=True)
+              for n, (ni, nj, nk, qvs, umax, _) in enumerate(shapes)]
+        return dict(case=case, ms=ms, ens=model.Ensemble(ms), outputs=_outputs(case))
+    net = surrogate.Net(seed=1)
+    net.set_params(_params(seed))
+    x, g = _net_inputs(case["rows"], seed)
+    s = dict(case=case, net=net, x=x)
+    if kind == "grad":
+        # targets: smooth in the inputs, with scatter
+        s["t"] = (torch.tanh(x[:, :4]) + 0.3 * x[:, 4:] * x[:, :4] +
+                  0.1 * torch.randn((case["rows"], 4), device=DEV, generator=g)).contiguous()
+    return s
+
+
+def run(s):
+    case = s["case"]
+    kind = case["kind"]
+    if kind == "forward":
+        return s["net"].forward(s["x"])
+    if kind == "grad":
+        loss, grad = s["net"].loss_grad(s["x"], s["t"], want_grad=True)
+        return dict(loss=loss, grad=grad)
+    if kind == "ensemble":
+        s["ens"].step(case["steps"])
+        s["ens"].sync()
+        # the members' states side by side, for the ensemble's statistics
+        return {name: torch.cat([_inside(m, name, st).reshape(-1) for m in s["ms"]]) for name, st in s["outputs"]}
+    s["m"].step(case["steps"])
+    if case["out"] == "device":
+        return {name: _inside(s["m"], name, st) for name, st in s["outputs"]}
+    return {name: s["m"].interior(name, st) for name, st in s["outputs"]}
+
+
+def work(case):
+    """Bytes: what a step cannot keep on the chip.  Every Runge-Kutta stage
+    reads and writes each prognostic field and reads its step-start value and
+    forcing; every acoustic substep reads and writes u, v, w, pi', reads the
+    previous damping term, four tendencies and three coefficients, and
+    accumulates three averages.  Flops: the fifth-order fluxes (three per
+    scalar and momentum cell) and the acoustic update; about three times as
+    many per flux with WENO5."""
+    kind = case["kind"]
+    if kind in ("grad", "forward"):
+        weights = 8 * 128 + 2 * 128 * 128 + 128 * 4
+        n = case["rows"]
+        if kind == "grad":
+            return {"bytes": 4.0 * (n * 12 + 2 * (weights + 388)), "flops": 6.0 * n * weights}
+        return {"bytes": 4.0 * (n * 12 + weights + 388), "flops": 2.0 * n * weights}
+
+    def step(cells, nscalar, nsound, weno):
+        nsub = -(-nsound // 3) + nsound // 2 + nsound
+        fields = 3 * 4 * (4 + nscalar) + nsub * (8 + 1 + 4 + 3 + 6)
+        flops = 3 * (3 + nscalar) * 120 * (2.0 if weno else 1.0) + nsub * 70
+        return 4.0 * cells * fields, 1.0 * cells * flops
+
+    if kind == "ensemble":
+        shapes = workloads.ensemble_small_shapes(case["members"]) if case["small"] else \
+            workloads.ensemble_shapes(case["members"])
+        b, f = step(sum(s[0] * s[1] * s[2] for s in shapes), 4, 6, False)
+    elif kind == "cbl":
+        b, f = step(case["ni"] * case["nj"] * case["nk"], 1 + case["npt"] + int(case["turb"]), 10, True)
+    else:
+        nsound = 8 if case["stretch"] else 6
+        b, f = step(case["ni"] * case["nj"] * case["nk"], 4 + case["npt"], nsound, case["weno"] == 1)
+    return {"bytes": b * case["steps"], "flops": f * case["steps"]}
+
+
+def _forward64(p, x):
+    """Pre-activations and activations of the network in 64 bits."""
+    o, a, keep = 0, x.double(), []
+    for n, (fin, fout) in enumerate(((8, 128), (128, 128), (128, 128), (128, 4))):
+        w = p[o:o + fin * fout].view(fin, fout)
+        b = p[o + fin * fout:o + fin * fout + fout]
+        o += fin * fout + fout
+        z = a @ w + b
+        keep.append((a, w, z))
+        a = z * torch.sigmoid(z) if n < 3 else z
+    return a, keep
+
+
+def exact(case, seed):
+    """The surrogate's forward pass and gradients in 64 bits.  A large step
+    has no closed value to give: in 64 bits the model is another
+    discretisation's whole integration, a program of the library's own size."""
+    if case["kind"] not in ("grad", "forward"):
+        return None
+    s = {"case": case}
+    p = torch.from_numpy(_params(seed).astype(np.float64)).to(DEV)
+    x, g = _net_inputs(case["rows"], seed)
+    if case["kind"] == "forward":
+        return torch.cat([_forward64(p, part)[0] for part in x.split(1 << 18)])
+    s["t"] = torch.tanh(x[:, :4]) + 0.3 * x[:, 4:] * x[:, :4] + \
+        0.1 * torch.randn((case["rows"], 4), device=DEV, generator=g)
+    p.requires_grad_(True)
+    total = torch.zeros((), dtype=torch.float64, device=DEV)
+    count = 4.0 * case["rows"]
+    for xp, tp in zip(x.split(1 << 16), s["t"].split(1 << 16)):
+        part = ((_forward64(p, xp)[0] - tp.double()) ** 2).sum() / count
+        part.backward()
+        total += part.detach()
+    return dict(loss=float(total), grad=p.grad.cpu().numpy())
