@@ -94,15 +94,15 @@ def draw(rng):
     if kind == "cbl":
         ni, nj, nk = _log_int(rng, 24, 512), _log_int(rng, 24, 512), rng.randint(24, 128)
         steps = 1 if ni * nj * nk > 2000000 else rng.randint(2, 8)
-        out = "device" if steps == 1 else rng.choice(["host", "device"])
+        out = "device" if steps == 1 or nj * nk > 15000 else rng.choice(["host", "device"])
         c = _cbl("", ni, nj, nk, steps, out, npt=rng.randint(0, 6), turb=rng.random() < 0.7,
                  impl=rng.random() < 0.7)
     else:
-        ni, nj = _log_int(rng, 24, 800), _log_int(rng, 24, 800)
+        ni, nj = _log_int(rng, 24, 640), _log_int(rng, 24, 640)
         stretch = rng.random() < 0.25
         nk = 96 if stretch else rng.randint(20, 90)
         steps = 1 if ni * nj * nk > 4000000 else rng.randint(2, 10)
-        out = "device" if steps == 1 else rng.choice(["host", "device"])
+        out = "device" if steps == 1 or nj * nk > 15000 else rng.choice(["host", "device"])
         psolver = 2 if rng.random() < 0.2 else 3
         c = _storm("", ni, nj, nk, steps, out, stretch=stretch, bc=rng.choice([1, 2, 2]), psolver=psolver,
                    weno=rng.choice([0, 0, 0, 1, 2]), npt=rng.choice([0, 0, 1, 3]), rdamp=rng.choice([0, 1]),
