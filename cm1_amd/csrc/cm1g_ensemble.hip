@@ -117,11 +117,21 @@ static int ens_build(cm1g_ensemble *e, cm1g_ensemble::Graph &g) {
   auto restore = [&]() {
     for (int i = 0; i < n; i++) set_field_map(e->mem[i], g.before[i]);
   };
+  int plan_nk = 0;
+  long plan_tiles = 0;
+  for (const auto *m : e->mem) {
+    plan_nk = std::max(plan_nk, m->P.nk);
+    plan_tiles += (long)((m->P.ni + 63) / 64) * m->P.nj;
+  }
   for (int i = 0; i < n; i++) {
     cm1g_model *m = e->mem[i];
     m->rec = &recs[i];
+    m->plan_nk = plan_nk;
+    m->plan_tiles = plan_tiles;
     const int rc = step_body(m);
     m->rec = nullptr;
+    m->plan_nk = 0;
+    m->plan_tiles = 0;
     if (rc) {
       restore();
       return rc;

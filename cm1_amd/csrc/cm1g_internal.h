@@ -103,6 +103,12 @@ struct cm1g_model {
   // the a-arrays in their place), or until unswap() copies them back for a
   // caller that reads them
   int swapped;
+  // while an ensemble records this member's step: the most levels and the
+  // column tiles (64 columns x 1 row) of all its members, so that every
+  // member chooses the same kernels and workgroup sizes (0 otherwise: the
+  // model's own)
+  int plan_nk;
+  long plan_tiles;
   // non-null while an ensemble records this member's step: launches are
   // appended here instead of run
   std::vector<struct LaunchRec> *rec;
@@ -197,7 +203,7 @@ struct BatchSlot {
 
 template <int NT, class F>
 __global__ void __launch_bounds__(NT) k_one(F f) {
-  f((int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
+  [[clang::always_inline]] f((int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
 }
 
 // The member search and functor call of k_many (below).
@@ -219,8 +225,12 @@ __device__ __forceinline__ void many_body(const F *__restrict__ fs, const BatchS
   const int gy = __builtin_amdgcn_readfirstlane(slots[lo].gy);
   const int l = b - start;
   if (l >= n) return;  // padding up to the next member's start
-  const F f = fs[lo];    // read before the functor stores anything
-  f(l % gx, (l / gx) % gy, l / (gx * gy));
+  // the functor does not change while the launch runs: through the constant
+  // address space its members are read where they are used, with scalar
+  // loads, across stores and barriers (as a kernel's own arguments are)
+  typedef const __attribute__((address_space(4))) F CF;
+  const F &f = *(const F *)(CF *)(uintptr_t)(fs + lo);
+  [[clang::always_inline]] f(l % gx, (l / gx) % gy, l / (gx * gy));
 }
 
 template <int NT, class F>
@@ -235,7 +245,7 @@ __global__ void __launch_bounds__(NT) k_many(const F *__restrict__ fs, const Bat
 // partly filled last round is left.
 template <int NT, int W, class F>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_one_w(F f) {
-  f((int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
+  [[clang::always_inline]] f((int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
 }
 template <int NT, int W, class F>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W)))

@@ -50,6 +50,14 @@ struct SubArgs {
   const float *coef;
   int first;
   int nring;                      // trailing workgroups that do the averaging ring
+  // The averages take in u, v, w of two substeps at a time: substep n - 1's
+  // values are substep n's input, so every other substep leaves rru, rrv,
+  // rrw alone (no read, no write) and the next one adds both values, in the
+  // order of the substeps.  fold: this substep updates the averages; pair:
+  // with the previous substep's values too; init: they start here.
+  int fold, pair, init;
+  const float *wRp;               // the wR of the previous substep
+  float *ppx;                     // last substep of the last stage: the damping term
 };
 
 // new u at (i,j,k): radiative open-boundary update (ssopenbcw/e,
@@ -86,20 +94,42 @@ __device__ __forceinline__ float sub_v(const KP &P, const SubArgs &a, int i, int
   return v + dtv * (a.vten[c] - a.tem2 * (a.ppdX[c] - a.ppdX[cs]) * P.vf[j + 2] * (a.thv[c] + a.thv[cs]));
 }
 
-// store a new u (v) and fold it into the substep average (src/sound.F:806-835)
+// the running average r (rru, rrv) with the previous substep's value x0 and
+// this one's x (src/sound.F:806-835)
+__device__ __forceinline__ float avg_uv(const SubArgs &a, float r, float x0, float x) {
+  if (a.pair) r = r + x0;
+  return a.last ? (r + x) * a.tavg : r + x;
+}
+// store a new u (v) and fold it into the substep average
 __device__ __forceinline__ void put_u(const SubArgs &a, int c, float u) {
+  if (a.fold) a.rru[c] = avg_uv(a, a.init ? 0.0f : a.rru[c], a.uX[c], u);
   a.uY[c] = u;
-  const float r = a.first ? 0.0f : a.rru[c];
-  a.rru[c] = a.last ? (r + u) * a.tavg : r + u;
 }
 __device__ __forceinline__ void put_v(const SubArgs &a, int c, float v) {
+  if (a.fold) a.rrv[c] = avg_uv(a, a.init ? 0.0f : a.rrv[c], a.vX[c], v);
   a.vY[c] = v;
-  const float r = a.first ? 0.0f : a.rrv[c];
-  a.rrv[c] = a.last ? (r + v) * a.tavg : r + v;
 }
-__device__ __forceinline__ void put_w_avg(const SubArgs &a, int c, float w) {
-  const float r = a.first ? a.wa[c] * a.beta : a.rrw[c];
+// w on the ring, where the step does not change it
+__device__ __forceinline__ void put_w_ring(const SubArgs &a, int c) {
+  if (!a.fold) return;
+  float r = a.init ? a.wa[c] * a.beta : a.rrw[c];
+  if (a.pair) r = r + a.wRp[c];
+  const float w = a.wR[c];
   a.rrw[c] = a.last ? (r + w * a.alph) * a.tavg : r + w;
+}
+
+// The one-point halo fill of an interior value (BC_P, src/bc.F:372-520) by
+// the point that owns it: the copies of (i,j) outside the domain, corners
+// included (the reference fills west/east, then south/north over the filled
+// columns, so a corner holds the value of the interior point both map to).
+__device__ __forceinline__ void put_p_halo(const KP &P, float *p, int i, int j, int k, float v) {
+  const bool w = (i == 1), e = (i == P.ni), s = (j == 1), n = (j == P.nj);
+  if (!(w || e || s || n)) return;
+  const int xi = w ? (P.ebc == 1 ? P.ni + 1 : 0) : (P.wbc == 1 ? 0 : P.ni + 1);
+  const int xj = s ? (P.nbc == 1 ? P.nj + 1 : 0) : (P.sbc == 1 ? 0 : P.nj + 1);
+  if (w || e) p[IXD(P, xi, j, k)] = v;
+  if (s || n) p[IXD(P, i, xj, k)] = v;
+  if ((w || e) && (s || n)) p[IXD(P, xi, xj, k)] = v;
 }
 
 // The averaging ring of one substep: u and v on the faces i = ni+1 and
@@ -124,7 +154,7 @@ __device__ __forceinline__ void sound_ring_point(const KP &P, const SubArgs &a, 
   const int c = IXD(P, i, j, k);
   put_u(a, c, sub_u(P, a, i, j, k));
   put_v(a, c, sub_v(P, a, i, j, k));
-  put_w_avg(a, c, a.wR[c]);
+  put_w_ring(a, c);
 }
 
 // Operands of one level of the upward sweep of sound_sub (raw loads).
@@ -146,8 +176,8 @@ __device__ __forceinline__ void sub_load(const KP &P, const SubArgs &a, int c, i
   L.pdc = a.ppdX[c]; L.pdw = a.ppdX[c - 1]; L.pde = a.ppdX[c + 1]; L.pds = a.ppdX[c - px];
   L.pdn = a.ppdX[c + px];
   L.thc = a.thv[c]; L.thw = a.thv[c - 1]; L.the = a.thv[c + 1]; L.ths = a.thv[c - px]; L.thn = a.thv[c + px];
-  L.rruc = a.first ? 0.0f : a.rru[c];
-  L.rrvc = a.first ? 0.0f : a.rrv[c];
+  L.rruc = (!a.fold || a.init) ? 0.0f : a.rru[c];
+  L.rrvc = (!a.fold || a.init) ? 0.0f : a.rrv[c];
   L.paw = a.piadv[c - 1]; L.pae = a.piadv[c + 1]; L.pas = a.piadv[c - px]; L.pan = a.piadv[c + px];
   L.pa_p = a.piadv[c + pxy];
   L.ppterm = a.ppterm[c]; L.ppten = a.ppten[c]; L.wten = a.wten[c]; L.pp_c = a.ppR[c];
@@ -270,9 +300,11 @@ __device__ __forceinline__ void sound_sub(const KP &P, const SubArgs &a, const C
     }
     // ---- stores
     a.uY[c] = un0;
-    a.rru[c] = a.last ? (rruc + un0) * a.tavg : rruc + un0;
     a.vY[c] = vn0;
-    a.rrv[c] = a.last ? (rrvc + vn0) * a.tavg : rrvc + vn0;
+    if (a.fold) {
+      a.rru[c] = avg_uv(a, rruc, uXc, un0);
+      a.rrv[c] = avg_uv(a, rrvc, vXc, vn0);
+    }
     a.fpk[c] = fpk;
     // d1 depends only on the stage's fixed coefficients (thv, piadv,
     // ppterm, dts): stored on the first substep, read on the others
@@ -299,7 +331,12 @@ __device__ __forceinline__ void sound_sub(const KP &P, const SubArgs &a, const C
   // operands of the current level
   float q_d1 = 0.0f, q_d2 = 0.0f;
   float q_pp = a.ppR[c], q_fpk = a.fpk[c], q_pm = a.piadv[c - pxy], q_term = a.ppterm[c];
-  float q_rrw = a.first ? a.wa[c] * a.beta : a.rrw[c];
+  auto rrw_of = [&](int cc) -> float {  // the w average before this substep's w
+    if (!a.fold) return 0.0f;
+    const float r = a.init ? a.wa[cc] * a.beta : a.rrw[cc];
+    return a.pair ? r + a.wR[cc] : r;
+  };
+  float q_rrw = rrw_of(c);
   for (int k = nk; k >= 1; k--, c -= pxy) {
     const float p_old = q_pp, fk = q_fpk, pa_m2 = q_pm, pterm = q_term, rrwc = q_rrw;
     float wk;
@@ -321,7 +358,7 @@ __device__ __forceinline__ void sound_sub(const KP &P, const SubArgs &a, const C
       q_fpk = a.fpk[cb];
       q_pm = a.piadv[cb - pxy];
       q_term = a.ppterm[cb];
-      q_rrw = a.first ? a.wa[cb] * a.beta : a.rrw[cb];
+      q_rrw = rrw_of(cb);
     }
     const float *cf = a.coef + 8 * k;
     const float tem = cf[0], r1 = cf[1], r2 = cf[2];
@@ -334,13 +371,338 @@ __device__ __forceinline__ void sound_sub(const KP &P, const SubArgs &a, const C
     const float d = a.kdiv * (pn - p_old);
     if (k >= 2 || a.wR != a.w3d) a.w3d[c] = wk;
     a.pp3d[c] = pn;
-    if (a.last) a.dum1[c] = d;
+    if (a.ppx) a.ppx[c] = d;
     a.ppdY[c] = pn + d;
-    a.rrw[c] = a.last ? (rrwc + wk * alph) * a.tavg : rrwc + wk;
+    if (!a.last) put_p_halo(P, a.ppdY, i, j, k, pn + d);
+    if (a.fold) a.rrw[c] = a.last ? (rrwc + wk * alph) * a.tavg : rrwc + wk;
     w_above = wk;
     pa_p = pa_c2;
     pa_c2 = pa_m2;
   }
+}
+
+// ------------------------------------------------- acoustic substep, slabs
+// The same substep with a workgroup per 64 columns of one row and NW
+// wavefronts that each own L consecutive levels of those columns, so that
+// what the vertical solve carries from its upward to its downward sweep
+// stays on the chip (the solver's terms in registers, the pi coefficients
+// and the old pi' in LDS) instead of going through fpk, dum2 and a second
+// read of pi', ppterm and piadv.  Per column and substep that leaves 13
+// arrays read (12 on a stage's first substep) and 5 written, plus the
+// averages on every other substep.
+//   1. every wavefront advances u, v and forms fpk and the solver's terms of
+//      its levels;
+//   2. the tridiagonal recurrences run up, then down the column, wavefront
+//      after wavefront, in the reference's order (the values are exactly
+//      those of one thread marching the column);
+//   3. every wavefront updates pi' and the w average of its levels.
+//
+// Bound by memory: at 1024 x 1024 x 96, 2.03 ms a substep against 2.93 ms
+// for sound_sub; 7.5 + 2.8 GB to and from memory (10.7 + 4.2 before), 5.0
+// TB/s, what a plain copy reaches.  On small grids a column's levels are in
+// flight together instead of one after the other: 256 x 256 x 64 104 us
+// against 201, 64 x 64 x 40 see slab_variant.  12 levels per wavefront is
+// the most that 128 registers hold (two workgroups of 8 wavefronts per CU):
+// 6 and 8 levels (one workgroup of 16 or 12) 2.50 and 2.48 ms, 16 levels
+// 3.04 ms; loading the next level's centre values ahead, paid for with a
+// second read of dum1, 2.11 ms.
+//
+// The horizontal metrics uh, uf, vh, vf of sound_sub are all 1 (cm1g_create
+// sets no other), and a product with 1 changes no value: left out here.
+// Loads and stores at a byte offset: fields are below 4 GiB (slab_variant
+// checks it), so one 32-bit offset per point serves every array, with the
+// array's base in scalar registers.
+__device__ __forceinline__ float ldo(const float *p, unsigned o) { return *(const float *)((const char *)p + o); }
+__device__ __forceinline__ void sto(float *p, unsigned o, float v) { *(float *)((char *)p + o) = v; }
+
+struct SlabGrid {
+  int nt, gx, per, nj, nw;  // tiles (64 columns x 1 row), tiles along i, tiles per XCD, rows, wavefronts
+};
+// Tiles are walked row by row in strips of this many tiles along i, a strip
+// after the other, so that a tile's neighbours along i and j run on its XCD
+// at about the same time and find each other's lines in its L2.  Measured at
+// 1024 x 1024 x 96: strips of 1, 2, 4, 8 and 16 tiles 2.26, 2.09, 2.05, 2.02
+// and 2.04 ms per substep (4.62e6 KB fetched with 16, 3.65e6 with 4).
+constexpr int SLAB_STRIP = 8;
+
+template <int L, int CAP, bool FIRST>
+__device__ __forceinline__ void sound_slab(const KP &P, const SubArgs &a, const SlabGrid &sg, int bx) {
+  __shared__ float sA[CAP][64], sB[CAP][64], sP[CAP][64];  // pk1 + qk, pk2 - qk, old pi'
+  __shared__ float h0[CAP / L][64], h1[CAP / L][64];       // hand-over between wavefronts
+  const int nmain = sg.per * NXCD;
+  if (bx >= nmain) {
+    const int npts = P.ni + P.nj + 1;
+    const int t = (bx - nmain) * (int)blockDim.x + (int)threadIdx.x;
+    if (t < npts * P.nk) sound_ring_point(P, a, t % npts, 1 + t / npts);
+    return;
+  }
+  const int t = (bx % NXCD) * sg.per + bx / NXCD;
+  if (t >= sg.nt) return;
+  const int ni = P.ni, nj = P.nj, nk = P.nk;
+  const int lane = (int)threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int strip = t / (SLAB_STRIP * sg.nj), t2 = t - strip * SLAB_STRIP * sg.nj;
+  const int wid = min(SLAB_STRIP, sg.gx - strip * SLAB_STRIP);
+  const int j = 1 + t2 / wid;
+  const int iraw = 1 + (strip * SLAB_STRIP + t2 % wid) * 64 + lane;
+  const bool on = iraw <= ni;
+  const int i = on ? iraw : ni;  // lanes past the row's end follow its last column and store nothing
+  const float dts = a.dts, rdx = P.rdx, rdy = P.rdy;
+  const float alph = a.alph, beta = a.beta, asq = a.asq, smeps = P.K.smeps;
+  // sides whose radiative update falls on this column; bw, be vary along the
+  // wavefront, bs, bn do not (one row)
+  const bool bw = a.opw && i == 1, be = a.ope && i == ni, bs = a.ops && j == 1, bn = a.opn && j == nj;
+  const bool edge = bs || bn || __builtin_amdgcn_ballot_w64(bw || be) != 0ULL;
+  const unsigned pxB = 4u * (unsigned)P.px, pxyB = 4u * (unsigned)P.pxy;
+  const int k0 = 1 + wv * L;
+  const unsigned c0 = 4u * (unsigned)IXD(P, i, j, k0);
+  float sv[L], aa[L], rr[L], d1[L], dd[L];
+  // the first level's terms that need the level below, kept for after the
+  // wavefronts have met
+  float mm0 = 0.0f, A0 = 0.0f, B0 = 0.0f, p0 = 0.0f, w0 = 0.0f, wt0 = 0.0f, d1m = 0.0f;
+  float w_bot = 0.0f, w_top1 = 0.0f;
+  if (k0 <= nk) {
+    // dts times the masks dtu0, dtv0 at (i,j), (i+1,j), (i,j), (i,j+1): zero
+    // on the faces of a non-periodic side (src/param.F:9182-9218)
+    const float dtu_c = (P.ibw && i == 1) ? 0.0f : dts, dtu_e = (P.ibe && i == ni) ? 0.0f : dts;
+    const float dtv_c = (P.ibs && j == 1) ? 0.0f : dts, dtv_n = (P.ibn && j == nj) ? 0.0f : dts;
+    const float tem1 = a.tem1, tem2 = a.tem2, temx = a.temx, temy = a.temy;
+    unsigned c = c0;
+    float pa_m = ldo(a.piadv, c - pxyB), pa_c = ldo(a.piadv, c), th_m = ldo(a.thv, c - pxyB);
+    float w_c = ldo(a.wR, c);
+    if (!FIRST && k0 >= 3) d1m = ldo(a.dum1, c - pxyB);
+    float A_m = 0.0f, B_m = 0.0f, s_m = 0.0f, pp_m = 0.0f;
+#pragma unroll
+    for (int l = 0; l < L; l++, c += pxyB) {
+      const int k = k0 + l;
+      if (k > nk) break;
+      const unsigned cN = c + pxB, cS = c - pxB, cU = c + pxyB;
+      const float uXc = ldo(a.uX, c), utc = ldo(a.uten, c), vXc = ldo(a.vX, c), vtc = ldo(a.vten, c), pdc = ldo(a.ppdX, c), thc = ldo(a.thv, c);
+      const float ppterm = ldo(a.ppterm, c), ppten = ldo(a.ppten, c), wten = ldo(a.wten, c), pp_c = ldo(a.ppR, c);
+      const float uXe = ldo(a.uX, c + 4u), ute = ldo(a.uten, c + 4u);
+      const float vXn = ldo(a.vX, cN), vtn = ldo(a.vten, cN);
+      const float pdw = ldo(a.ppdX, c - 4u), pde = ldo(a.ppdX, c + 4u);
+      const float pds = ldo(a.ppdX, cS), pdn = ldo(a.ppdX, cN);
+      const float thw = ldo(a.thv, c - 4u), the = ldo(a.thv, c + 4u);
+      const float ths = ldo(a.thv, cS), thn = ldo(a.thv, cN);
+      const float paw = ldo(a.piadv, c - 4u), pae = ldo(a.piadv, c + 4u);
+      const float pas = ldo(a.piadv, cS), pan = ldo(a.piadv, cN), pa_p = ldo(a.piadv, cU);
+      const float w_p = (k == nk) ? ldo(a.w3d, cU) : ldo(a.wR, cU);
+      float rruc = 0.0f, rrvc = 0.0f;
+      if (a.fold && !a.init) {
+        rruc = ldo(a.rru, c);
+        rrvc = ldo(a.rrv, c);
+      }
+      float d1c = 0.0f;
+      if (!FIRST && k >= 2 && k < nk) d1c = ldo(a.dum1, c);
+      // ---- u, v (ssopenbc* then src/sound.F:307-345)
+      float uo0 = uXc, uo1 = uXe, vo0 = vXc, vo1 = vXn;
+      if (edge) {
+        if (bw) uo0 = uo0 + dts * (-a.radbcw[(j + 2) + k * P.py] * (uXe - uo0) * rdx + utc);
+        if (be) uo1 = uo1 + dts * (-a.radbce[(j + 2) + k * P.py] * (uo1 - uXc) * rdx + ute);
+        if (bs) vo0 = vo0 + dts * (-a.radbcs[(i + 2) + k * P.px] * (vXn - vo0) * rdy + vtc);
+        if (bn) vo1 = vo1 + dts * (-a.radbcn[(i + 2) + k * P.px] * (vo1 - vXc) * rdy + vtn);
+      }
+      const float un0 = uo0 + dtu_c * (utc - tem1 * (pdc - pdw) * (thc + thw));
+      const float un1 = uo1 + dtu_e * (ute - tem1 * (pde - pdc) * (the + thc));
+      const float vn0 = vo0 + dtv_c * (vtc - tem2 * (pdc - pds) * (thc + ths));
+      const float vn1 = vo1 + dtv_n * (vtn - tem2 * (pdn - pdc) * (thn + thc));
+      // ---- coefficients (src/sound.F:117-180)
+      const float *cf = a.coef + 8 * k;
+      const float tem = cf[0], r1 = cf[1], r2 = cf[2], temm = cf[3];
+      const float c1a = cf[4], c1b = cf[5], c2a = cf[6], c2b = cf[7];
+      const float qk = tem * ppterm;
+      const float pk2 = (k == nk) ? 0.0f : r2 * (-c2b * pa_p + (1.0f - c1b) * pa_c);
+      const float pk1 = (k == 1) ? 0.0f : r1 * (+c1a * pa_m + (c2a - 1.0f) * pa_c);
+      const float mm = temm * (c2a * thc + c1a * th_m);
+      const float A = pk1 + qk, B = pk2 - qk;
+      // ---- explicit pi forcing
+      float div = (un1 - un0) * rdx + (vn1 - vn0) * rdy;
+      if (fabsf(div) < smeps) div = 0.0f;
+      const float fpk = dts * (ppten - ppterm * div) +
+                        (-(un0 * (pa_c - paw) + un1 * (pae - pa_c)) * temx -
+                         (vn0 * (pa_c - pas) + vn1 * (pan - pa_c)) * temy) +
+                        beta * (w_c * (pk1 + qk) + w_p * (pk2 - qk));
+      const float s = pp_c + fpk;
+      sA[k - 1][lane] = A;
+      sB[k - 1][lane] = B;
+      sP[k - 1][lane] = pp_c;
+      // ---- terms of the Thomas forward sweep
+      if (l == 0) {
+        mm0 = mm;
+        A0 = A;
+        B0 = B;
+        p0 = pp_c;
+        w0 = w_c;
+        wt0 = wten;
+      } else {
+        aa[l] = -asq * (+mm * A_m);
+        const float cc = -asq * (-mm * B);
+        const float bb = 1.0f - asq * (+mm * (-A + B_m));
+        const float fwk = dts * wten + beta * (-mm * (pp_c - pp_m));
+        dd[l] = w_c + fwk + alph * (-mm * (s - s_m));
+        if (FIRST) {
+          rr[l] = bb;
+          d1[l] = cc;
+        } else {
+          // d1 is fixed over a stage: its first substep stored it
+          rr[l] = 1.0f / ((k == 2) ? bb : aa[l] * d1[l - 1 < 0 ? 0 : l - 1] + bb);
+          d1[l] = d1c;
+        }
+      }
+      if (!FIRST && l == 0) d1[0] = d1c;
+      sv[l] = s;
+      if (k == 1) w_bot = w_c;
+      if (k == nk) w_top1 = w_p;
+      // ---- u, v and their averages
+      if (on) {
+        sto(a.uY, c, un0);
+        sto(a.vY, c, vn0);
+        if (a.fold) {
+          sto(a.rru, c, avg_uv(a, rruc, uXc, un0));
+          sto(a.rrv, c, avg_uv(a, rrvc, vXc, vn0));
+        }
+      }
+      A_m = A;
+      B_m = B;
+      s_m = s;
+      pp_m = pp_c;
+      pa_m = pa_c;
+      pa_c = pa_p;
+      th_m = thc;
+      w_c = w_p;
+    }
+    h0[wv][lane] = s_m;
+  }
+  __syncthreads();
+  if (k0 <= nk && k0 > 1) {
+    const float A_m = sA[k0 - 2][lane], B_m = sB[k0 - 2][lane], pp_m = sP[k0 - 2][lane], s_m = h0[wv - 1][lane];
+    aa[0] = -asq * (+mm0 * A_m);
+    const float cc = -asq * (-mm0 * B0);
+    const float bb = 1.0f - asq * (+mm0 * (-A0 + B_m));
+    const float fwk = dts * wt0 + beta * (-mm0 * (p0 - pp_m));
+    dd[0] = w0 + fwk + alph * (-mm0 * (sv[0] - s_m));
+    if (FIRST) {
+      rr[0] = bb;
+      d1[0] = cc;
+    } else {
+      rr[0] = 1.0f / ((k0 == 2) ? bb : aa[0] * d1m + bb);
+    }
+  }
+  __syncthreads();
+  // forward sweep, wavefront after wavefront; h0 hands over d2, h1 d1
+  for (int q = 0; q < sg.nw; q++) {
+    if (wv == q && k0 <= nk) {
+      float d1p = (FIRST && q > 0) ? h1[q - 1][lane] : 0.0f, d2p = (q > 0) ? h0[q - 1][lane] : 0.0f;
+#pragma unroll
+      for (int l = 0; l < L; l++) {
+        const int k = k0 + l;
+        if (k > nk) break;
+        if (k == 1) continue;
+        if (FIRST) {
+          const float bb = rr[l], cc = d1[l];
+          const float r = 1.0f / ((k == 2) ? bb : aa[l] * d1p + bb);
+          d1p = -cc * r;
+          d2p = (k == 2) ? dd[l] * r : (dd[l] - aa[l] * d2p) * r;
+          d1[l] = d1p;
+        } else {
+          d2p = (k == 2) ? dd[l] * rr[l] : (dd[l] - aa[l] * d2p) * rr[l];
+        }
+        dd[l] = d2p;
+      }
+      h0[q][lane] = d2p;
+      if (FIRST) h1[q][lane] = d1p;
+    }
+    __syncthreads();
+  }
+  // The old w and its running average for step 3, in the registers of the
+  // forward sweep's terms (the last-level cache still holds the w that step
+  // 1 read); d1 of a later substep likewise
+  if (k0 <= nk) {
+    if (a.fold) {
+      const float *src = a.init ? a.wa : a.rrw;
+#pragma unroll
+      for (int l = 0; l < L; l++)
+        if (k0 + l <= nk) {
+          aa[l] = ldo(src, c0 + l * pxyB);
+          rr[l] = a.pair ? ldo(a.wR, c0 + l * pxyB) : 0.0f;
+        }
+    }
+  }
+  // backward sweep; dd becomes w, h1 hands over the lowest w of a wavefront
+  for (int q = sg.nw - 1; q >= 0; q--) {
+    if (wv == q && k0 <= nk) {
+      float w_above = (k0 + L <= nk) ? h1[q + 1][lane] : w_top1;
+#pragma unroll
+      for (int l = L - 1; l >= 0; l--) {
+        const int k = k0 + l;
+        if (k > nk) continue;
+        float w;
+        if (k == nk) w = dd[l];
+        else if (k >= 2) w = d1[l] * w_above + dd[l];
+        else w = w_bot;
+        dd[l] = w;
+        w_above = w;
+      }
+      h1[q][lane] = w_above;
+    }
+    __syncthreads();
+  }
+  // pi' update with divergence damping (src/sound.F:739-765), w average
+  if (k0 > nk || !on) return;
+  unsigned c = c0;
+  const float w_next = (k0 + L <= nk) ? h1[wv + 1][lane] : w_top1;
+#pragma unroll
+  for (int l = 0; l < L; l++, c += pxyB) {
+    const int k = k0 + l;
+    if (k > nk) break;
+    const float wk = dd[l];
+    const float w_above = (k == nk) ? w_top1 : (l + 1 < L) ? dd[l + 1 < L ? l + 1 : l] : w_next;
+    const float p_old = sP[k - 1][lane];
+    float pn = sv[l] + alph * (wk * sA[k - 1][lane] + w_above * sB[k - 1][lane]);
+    if (fabsf(pn) < smeps) pn = 0.0f;
+    const float d = a.kdiv * (pn - p_old);
+    if (a.fold) {
+      float r = a.init ? aa[l] * beta : aa[l];
+      if (a.pair) r = r + rr[l];
+      sto(a.rrw, c, a.last ? (r + wk * alph) * a.tavg : r + wk);
+    }
+    if (k >= 2 || a.wR != a.w3d) sto(a.w3d, c, wk);
+    sto(a.pp3d, c, pn);
+    if (a.ppx) sto(a.ppx, c, d);
+    sto(a.ppdY, c, pn + d);
+    if (!a.last) put_p_halo(P, a.ppdY, i, j, k, pn + d);
+    if (FIRST && k >= 2 && k < nk) sto(a.dum1, c, d1[l]);
+  }
+}
+
+// The slab variants: levels per wavefront and levels a workgroup holds.
+constexpr int SLAB_L[] = {0, 4, 8, 12, 12}, SLAB_CAP[] = {0, 64, 64, 96, 192};
+
+template <int V, bool FIRST>
+static void slab_go(cm1g_model *m, dim3 grd, dim3 blk, const KP &P, const SubArgs &a, const SlabGrid &sg) {
+  constexpr int L = SLAB_L[V], CAP = SLAB_CAP[V], NT = 64 * (CAP / L);
+  launch<NT, 4>(m, grd, blk, [=] __device__(int bx, int, int) { sound_slab<L, CAP, FIRST>(P, a, sg, bx); });
+}
+static void slab_launch(cm1g_model *m, int v, dim3 grd, dim3 blk, const KP &P, const SubArgs &a,
+                        const SlabGrid &sg) {
+  if (v == 1) a.first ? slab_go<1, true>(m, grd, blk, P, a, sg) : slab_go<1, false>(m, grd, blk, P, a, sg);
+  else if (v == 2) a.first ? slab_go<2, true>(m, grd, blk, P, a, sg) : slab_go<2, false>(m, grd, blk, P, a, sg);
+  else if (v == 3) a.first ? slab_go<3, true>(m, grd, blk, P, a, sg) : slab_go<3, false>(m, grd, blk, P, a, sg);
+  else a.first ? slab_go<4, true>(m, grd, blk, P, a, sg) : slab_go<4, false>(m, grd, blk, P, a, sg);
+}
+
+// Which kernel runs the substep (0: sound_sub, one thread per column, for
+// columns too deep for a workgroup's LDS and fields of 4 GiB and more).  Up
+// to 64 levels 8 per wavefront, unless the grid is too small to fill the
+// chip: under 1024 tiles (four workgroups per CU) 4 per wavefront put more
+// wavefronts on a column.
+static int slab_variant(const cm1g_model *m) {
+  const int nk = m->plan_nk > m->P.nk ? m->plan_nk : m->P.nk;
+  const long tiles = m->plan_tiles > 0 ? m->plan_tiles : (long)((m->P.ni + 63) / 64) * m->P.nj;
+  if (nk > 192 || m->ntot >= ((size_t)1 << 30)) return 0;
+  if (nk <= 64) return tiles < 1024 ? 1 : 2;
+  return nk <= 96 ? 3 : 4;
 }
 
 void sound_run(cm1g_model *m, int nrk, bool fold1) {
@@ -406,12 +768,23 @@ void sound_run(cm1g_model *m, int nrk, bool fold1) {
   // copy of the scratch pair back into u3d/v3d)
   const bool fold = (nrk >= 2) || fold1;
   a.wa = wa;
+  const int slab = slab_variant(m);
   const ColGrid cg = col_grid(ni, nj, m->tile_rows);
-  const dim3 blk = col_threads(cg), grd = col_blocks(cg);
+  SlabGrid sg;
+  sg.nj = nj;
+  sg.gx = (ni + 63) / 64;
+  sg.nt = sg.gx * nj;
+  sg.per = (sg.nt + NXCD - 1) / NXCD;
+  const int plan_nk = m->plan_nk > nk ? m->plan_nk : nk;
+  const int lev = slab == 0 ? 1 : SLAB_L[slab];
+  sg.nw = (plan_nk + lev - 1) / lev;
+  const dim3 blk = slab ? dim3(64 * sg.nw) : col_threads(cg);
+  dim3 grd = slab ? dim3(sg.per * NXCD) : col_blocks(cg);
   {
     const int nthr = (int)blk.x, npts = (ni + nj + 1) * nk;
     a.nring = (npts + nthr - 1) / nthr;
   }
+  grd.x += a.nring;
   // the per-level solver coefficients of this stage's dts, with the
   // reference's expressions (src/sound.F:117-180)
   {
@@ -454,13 +827,21 @@ void sound_run(cm1g_model *m, int nrk, bool fold1) {
     a.ppdY = ppdb[(n - 1) & 1];
     a.wR = (n == 1 && fold) ? wa : w3d;
     a.ppR = (n == 1 && fold) ? ppi : pp3d;
+    a.wRp = (n == 2 && fold) ? wa : w3d;
     a.first = (n == 1);
     a.last = (n == nloop);
+    a.fold = ((nloop - n) & 1) == 0;
+    a.pair = (n > 1);
+    a.init = (n <= 2);
+    // the stage's damping term goes straight to ppx, unless this substep
+    // also reads ppx at neighbouring columns (a single-substep stage)
+    a.ppx = (nrk == 3 && a.last) ? (a.first ? m->tz : ppx) : nullptr;
     ktimer_mark(m, CM1G_KT_SOUND_SUBSTEP);
-    launch<256>(m, dim3(grd.x + a.nring), blk,
-                [=] __device__(int bx, int, int) { sound_sub(P, a, cg, bx); });
+    if (slab == 0)
+      launch<256>(m, grd, blk, [=] __device__(int bx, int, int) { sound_sub(P, a, cg, bx); });
+    else
+      slab_launch(m, slab, grd, blk, P, a, sg);
     ktimer_mark(m, CM1G_KT_SOUND_SUBSTEP);
-    if (n < nloop) bc_fill(m, BC_P, a.ppdY);
     uprev = udst;
     vprev = vdst;
   }
@@ -473,11 +854,13 @@ void sound_run(cm1g_model *m, int nrk, bool fold1) {
       v3d[c] = vs[c];
     });
   }
-  if (nrk == 3)
+  if (nrk == 3 && nloop == 1) {
+    const float *d = m->tz;
     for3(m, 1, ni, 1, nj, 1, nk, [=] __device__(int i, int j, int k) {
       int c = IXD(P, i, j, k);
-      ppx[c] = dum1[c];
+      ppx[c] = d[c];
     });
+  }
 }
 
 // Explicit acoustic substeps, psolver=2 (sounde, src/sounde.F:10-1026;

@@ -26,6 +26,8 @@ def short(name):
     if f:
         return f"{f.group(1)}<{f.group(2).split('::')[-1]} λ{f.group(3)}>"
     t = re.match(r"(\w+)<([^>]*)>\(", body)
+    if t and t.group(1) == "slab_go":
+        return "sound_sub"
     if t and t.group(1) in ("advs_launch", "advm_launch"):
         return {"advs_launch": "advs_col", "advm_launch": "advm_col"}[t.group(1)] + f"<{t.group(2)}>"
     h = re.match(r"([\w:]+)(?:\(.*?\))?::\{lambda\(int, int(?:, int)?\)#(\d+)\}", body)

@@ -1,0 +1,36 @@
+"""The acoustic substep's kernels at the edges of their tiles (64 columns, 4,
+8 or 12 levels per wavefront, 64, 96 or 192 levels per workgroup) and of the
+averages' pairing of substeps, against the oracle bit for bit."""
+import numpy as np
+import pytest
+
+from common import PROG, case, interior, make_gpu, make_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ni,nj,nk,nsound,bc", [
+    (8, 8, 6, 2, 2),        # the smallest grid; single-substep stages
+    (65, 9, 64, 4, 2),      # one column past a tile, every level of the 4-level form
+    (63, 8, 61, 6, 1),      # a last wavefront with one level
+    (64, 1025, 17, 6, 2),   # 8 levels per wavefront
+    (130, 520, 64, 6, 1),   # the same, full, three tiles per row
+    (12, 10, 65, 6, 2),     # 12 levels per wavefront, the last one short
+    (70, 8, 96, 8, 1),      # full
+    (9, 8, 97, 6, 2),       # sixteen wavefronts
+    (8, 9, 192, 4, 1),      # full
+    (8, 8, 193, 6, 2),      # one thread per column
+])
+def test_substep_edges_match_oracle(require_gpu, ni, nj, nk, nsound, bc):
+    dz = 15000.0 / nk
+    cfgd, cols, fields = case(ni=ni, nj=nj, nk=nk, nsound=nsound, bc=bc, dz=dz, dt=0.4 * nsound, amp=2.0)
+    g = make_gpu(cfgd, cols, fields)
+    o = make_oracle(cfgd, cols, fields)
+    for n in (1, 2):  # the first step and one that starts from exchanged buffers
+        g.step(n)
+        o.step(n)
+        for name, stag in PROG + [("ppx", None)]:
+            a = g.interior(name, stag)
+            b = interior(o.f(name), nk, nj, ni, stag)
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (n, name)
+    g.close()
