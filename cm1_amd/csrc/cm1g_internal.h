@@ -137,6 +137,10 @@ struct cm1g_model {
   // pinned host staging of cm1g_put_array / cm1g_get_array
   float *pin;
   size_t pin_cap;
+  // pinned chunks that box_move's kernels read and write from the device,
+  // and the event of each chunk's last kernel (allocated on first use)
+  float *xfer[2];
+  hipEvent_t xfer_ev[2];
 };
 
 // zeroed device allocation of n floats

@@ -1,0 +1,22 @@
+"""put / get of a field through the pinned chunks: boxes below, at and past
+the chunk size (2**20 floats), whole boxes equal."""
+import numpy as np
+import pytest
+
+from cm1_amd import model
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ni,nj,nk", [(8, 8, 6), (57, 121, 125), (249, 121, 29), (250, 121, 29), (401, 230, 70)])
+def test_put_get_round_trip(require_gpu, ni, nj, nk):
+    m = model.Model(model.make_config(ni=ni, nj=nj, nk=nk))
+    rng = np.random.default_rng(ni)
+    a = rng.standard_normal((m.pz, m.py, ni + 7)).astype(np.float32)
+    b = rng.standard_normal((m.pz, m.py, ni + 7)).astype(np.float32)
+    for _ in range(2):
+        m.put("dum1", a)
+        m.put("dum2", b)
+        assert np.array_equal(m.get("dum1"), a)
+        assert np.array_equal(m.get("dum2"), b)
+    m.close()
