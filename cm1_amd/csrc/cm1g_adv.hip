@@ -53,8 +53,8 @@ __device__ __forceinline__ float pdef_dum(const KP &P, int dir, const float *vel
   // writes it (src/pdef.F:44-45, :256-257, :482-483)
   const float sc = s[c];
   float sdiv;
-  if (dir == 0) sdiv = sc * (hi - lo) * P.rdx * P.uh[i + 2];
-  else if (dir == 1) sdiv = sc * (hi - lo) * P.rdy * P.vh[j + 2];
+  if (dir == 0) sdiv = sc * (hi - lo) * P.rdx;
+  else if (dir == 1) sdiv = sc * (hi - lo) * P.rdy;
   else sdiv = sc * (hi - lo) * P.rdz * P.mh[k];
   float d = P.rho0[k] * s0[c] + dt * (adv[c] + sdiv);
   if (dir == 0) {
@@ -162,7 +162,7 @@ __device__ __forceinline__ void pdef_xy(const KP &P, const PdefArgs &a, int bx, 
     if (flag) {
       float lo, hi;
       pdef_faces(P, 0, a.rru, a.scale, c, k, lo, hi);
-      out = (d[2] + mass - r0s0) * rdt - a.s[c] * (hi - lo) * P.rdx * P.uh[i + 2];
+      out = (d[2] + mass - r0s0) * rdt - a.s[c] * (hi - lo) * P.rdx;
     }
     a.ax_out[c] = out;
   }
@@ -174,7 +174,7 @@ __device__ __forceinline__ void pdef_xy(const KP &P, const PdefArgs &a, int bx, 
     if (flag) {
       float lo, hi;
       pdef_faces(P, 1, a.rrv, a.scale, c, k, lo, hi);
-      out = (dys[ty + 2][tx] + mass - r0s0) * rdt - a.s[c] * (hi - lo) * P.rdy * P.vh[j + 2];
+      out = (dys[ty + 2][tx] + mass - r0s0) * rdt - a.s[c] * (hi - lo) * P.rdy;
     }
     a.ay_out[c] = out;
   }
@@ -183,17 +183,17 @@ __device__ __forceinline__ void pdef_xy(const KP &P, const PdefArgs &a, int bx, 
 // z direction (pdefz) marched up each column with a window of dum, then the
 // tendency with the corrected advx, advy, advz and the s0 + dt*sten update
 __device__ __forceinline__ void pdef_z(const KP &P, const PdefArgs &a, const ColGrid &cg, int bx) {
-  int i, j;
-  if (!col_tile_b(cg, bx, i, j)) return;
+  int i, j, ks, ke;
   const int ni = P.ni, nj = P.nj, nk = P.nk;
+  if (!col_tile_seg(cg, bx, nk, i, j, ks, ke)) return;
   if (i > ni || j > nj) return;
   const float smeps = P.K.smeps, rdt = 1.0f / a.dt;
   auto dz = [&](int kk) -> float {  // dum of pdefz; zero outside 1..nk
     if (kk < 1 || kk > nk) return 0.0f;
     return pdef_dum(P, 2, a.rrw, a.scale, a.advz, a.s0, a.s, a.dt, i, j, kk);
   };
-  float dm2 = 0.0f, dm1 = 0.0f, d0 = dz(1), dp1 = dz(2), dp2 = dz(3);
-  for (int k = 1; k <= nk; k++) {
+  float dm2 = dz(ks - 2), dm1 = dz(ks - 1), d0 = dz(ks), dp1 = dz(ks + 1), dp2 = dz(ks + 2);
+  for (int k = ks; k <= ke; k++) {
     const int c = IXD(P, i, j, k);
     bool flag;
     const float mass = pdef_gather(dm2, dm1, d0, dp1, dp2, k - 1 >= 1, k + 1 <= nk, smeps, flag);
@@ -246,31 +246,35 @@ struct AdvLevel {
   float wnew;                          // s(k+4), entering the vertical window
 };
 
+// o: the column's byte offset in a level.  The start of level k of an array,
+// and of its neighbouring rows, is formed in scalar registers, so a level's
+// loads need no address arithmetic in vector registers.
 template <bool WENO, bool TH>
-__device__ __forceinline__ void advs_load(const KP &P, const AdvsArgs &a, int i, int j, int k,
+__device__ __forceinline__ void advs_load(const KP &P, const AdvsArgs &a, unsigned o, int k,
                                           AdvLevel &L) {
-  const int px = P.px, pxy = P.pxy, nk = P.nk;
-  const int c = IXD(P, i, j, k);
-  const float *s = a.s;
-  L.xm3 = s[c - 3]; L.xm2 = s[c - 2]; L.xm1 = s[c - 1];
-  L.xp1 = s[c + 1]; L.xp2 = s[c + 2]; L.xp3 = s[c + 3];
-  L.ym3 = s[c - 3 * px]; L.ym2 = s[c - 2 * px]; L.ym1 = s[c - px];
-  L.yp1 = s[c + px]; L.yp2 = s[c + 2 * px]; L.yp3 = s[c + 3 * px];
-  L.ru0 = a.rru[c]; L.ru1 = a.rru[c + 1];
-  L.rv0 = a.rrv[c]; L.rv1 = a.rrv[c + px];
-  L.rw1 = (k < nk) ? a.rrw[c + pxy] : 0.0f;
+  const int nk = P.nk;
+  const int px = P.px;
+  const size_t kb = (size_t)k * P.pxy;
+  const float *s = a.s + kb;
+  L.xm3 = ldo(s - 3, o); L.xm2 = ldo(s - 2, o); L.xm1 = ldo(s - 1, o);
+  L.xp1 = ldo(s + 1, o); L.xp2 = ldo(s + 2, o); L.xp3 = ldo(s + 3, o);
+  L.ym3 = ldo(s - 3 * px, o); L.ym2 = ldo(s - 2 * px, o); L.ym1 = ldo(s - px, o);
+  L.yp1 = ldo(s + px, o); L.yp2 = ldo(s + 2 * px, o); L.yp3 = ldo(s + 3 * px, o);
+  L.ru0 = ldo(a.rru + kb, o); L.ru1 = ldo(a.rru + kb + 1, o);
+  L.rv0 = ldo(a.rrv + kb, o); L.rv1 = ldo(a.rrv + kb + px, o);
+  L.rw1 = (k < nk) ? ldo(a.rrw + kb + P.pxy, o) : 0.0f;
   if (a.scale) {
     const float r0 = P.rho0[k];
     L.ru0 = L.ru0 * r0; L.ru1 = L.ru1 * r0;
     L.rv0 = L.rv0 * r0; L.rv1 = L.rv1 * r0;
     if (k < nk) L.rw1 = L.rw1 * P.rf0[k + 1];
   }
-  L.wnew = (k + 4 <= nk) ? s[c + 4 * pxy] : 0.0f;
-  L.dv = a.divx[c];
-  L.st0 = a.sten0[c];
-  L.sv0 = a.s0[c];
-  L.t11v = TH ? a.t11[c] : 0.0f;
-  L.thtv = TH ? a.thterm[c] : 0.0f;
+  L.wnew = (k + 4 <= nk) ? ldo(s + 4 * (size_t)P.pxy, o) : 0.0f;
+  L.dv = ldo(a.divx + kb, o);
+  L.st0 = ldo(a.sten0 + kb, o);
+  L.sv0 = ldo(a.s0 + kb, o);
+  L.t11v = TH ? ldo(a.t11 + kb, o) : 0.0f;
+  L.thtv = TH ? ldo(a.thterm + kb, o) : 0.0f;
 }
 
 // One column (i,j) of advs (src/adv.F:14-658 with hadv_flx5/vadv_flx5, or
@@ -284,29 +288,40 @@ __device__ __forceinline__ void advs_load(const KP &P, const AdvsArgs &a, int i,
 // (theta's t11*thterm term), MODE1 (advx/advy/advz for the pdef pass).
 template <bool WENO, bool SADD, bool TH, bool MODE1>
 __device__ __forceinline__ void advs_col(const KP &P, const AdvsArgs &a, const ColGrid &cg, int bx) {
-  int i, j;
-  if (!col_tile_b(cg, bx, i, j)) return;
+  int i, j, ks, ke;
   const int ni = P.ni, nj = P.nj, nk = P.nk;
+  if (!col_tile_seg(cg, bx, nk, i, j, ks, ke)) return;
   if (i > ni || j > nj) return;
   const bool doitw = (P.wbc == 2 && P.ibw == 1), doite = (P.ebc == 2 && P.ibe == 1);
   const bool doits = (P.sbc == 2 && P.ibs == 1), doitn = (P.nbc == 2 && P.ibn == 1);
-  const float *s = a.s;
   constexpr bool sadd = SADD;
   const float th0r = P.K.th0r;
+  const unsigned o = 4u * (unsigned)IX2D(P, i, j);
   auto val = [&](int kk) -> float {  // column value at level kk (1..nk)
     if (kk < 1 || kk > nk) return 0.0f;
-    const float v = s[IXD(P, i, j, kk)];
+    const float v = ldo(a.s + (size_t)kk * P.pxy, o);
     return sadd ? (P.th0[kk] - th0r) + v : v;
   };
   // window: wv[0..5] = S(k-2 .. k+3)
-  float wv0 = val(-1), wv1 = val(0), wv2 = val(1), wv3 = val(2), wv4 = val(3), wv5 = val(4);
-  float fz_lo = 0.0f;
+  float wv0 = val(ks - 2), wv1 = val(ks - 1), wv2 = val(ks), wv3 = val(ks + 1), wv4 = val(ks + 2), wv5 = val(ks + 3);
   AdvLevel nx;
-  advs_load<WENO, TH>(P, a, i, j, 1, nx);
-  for (int k = 1; k <= nk; k++) {
+  advs_load<WENO, TH>(P, a, o, ks, nx);
+  float fz_lo = 0.0f;
+  if (ks > 1) {
+    // the flux through a segment's lowest face
+    float rw = ldo(a.rrw + (size_t)ks * P.pxy, o);
+    if (a.scale) rw = rw * P.rf0[ks];
+    const float wm = val(ks - 3);
+    auto S = [=](int kk) -> float {
+      const int q = kk - ks;  // -3..2
+      return q == -3 ? wm : q == -2 ? wv0 : q == -1 ? wv1 : q == 0 ? wv2 : q == 1 ? wv3 : wv4;
+    };
+    fz_lo = WENO ? vfluxw_of(P, 1, rw, S, ks, a.pdefweno, a.weps) : vflux5_of(P, 1, rw, S, ks);
+  }
+  for (int k = ks; k <= ke; k++) {
     const AdvLevel L = nx;
-    if (k < nk) advs_load<WENO, TH>(P, a, i, j, k + 1, nx);
-    const int c = IXD(P, i, j, k);
+    if (k < ke) advs_load<WENO, TH>(P, a, o, k + 1, nx);
+    const size_t kb = (size_t)k * P.pxy;
     const float tem = sadd ? (P.th0[k] - th0r) : 0.0f;
     auto H = [=](float v) -> float { return sadd ? tem + v : v; };
     const float sc = wv2;
@@ -328,12 +343,13 @@ __device__ __forceinline__ void advs_col(const KP &P, const AdvsArgs &a, const C
     const float fy0_raw = fy0;
     if (doits && j == 1 && rv0 >= 0.0f) fy0 = fy1;
     if (doitn && j == nj && rv1 <= 0.0f) fy1 = fy0_raw;
-    float ax = -(fx1 - fx0) * P.rdx * P.uh[i + 2];
-    float ay = -(fy1 - fy0) * P.rdy * P.vh[j + 2];
-    if (doitw && i == 1 && ru0 >= 0.0f) ax = ax - sc * (ru1 - ru0) * P.rdx * P.uh[1 + 2];
-    if (doite && i == ni && ru1 <= 0.0f) ax = ax - sc * (ru1 - ru0) * P.rdx * P.uh[ni + 2];
-    if (doits && j == 1 && rv0 >= 0.0f) ay = ay - sc * (rv1 - rv0) * P.rdy * P.vh[1 + 2];
-    if (doitn && j == nj && rv1 <= 0.0f) ay = ay - sc * (rv1 - rv0) * P.rdy * P.vh[nj + 2];
+    // (uh, vh are 1)
+    float ax = -(fx1 - fx0) * P.rdx;
+    float ay = -(fy1 - fy0) * P.rdy;
+    if (doitw && i == 1 && ru0 >= 0.0f) ax = ax - sc * (ru1 - ru0) * P.rdx;
+    if (doite && i == ni && ru1 <= 0.0f) ax = ax - sc * (ru1 - ru0) * P.rdx;
+    if (doits && j == 1 && rv0 >= 0.0f) ay = ay - sc * (rv1 - rv0) * P.rdy;
+    if (doitn && j == nj && rv1 <= 0.0f) ay = ay - sc * (rv1 - rv0) * P.rdy;
     // vertical face k+1 from S(k-2..k+3)
     float fz_hi = 0.0f;
     if (k + 1 <= nk) {
@@ -350,18 +366,18 @@ __device__ __forceinline__ void advs_col(const KP &P, const AdvsArgs &a, const C
     else if (k == nk) az = +fz_lo * P.rdz * P.mh[nk];
     else az = -(fz_hi - fz_lo) * P.rdz * P.mh[k];
     if (MODE1) {
-      a.advx[c] = ax;
-      a.advy[c] = ay;
-      a.advz[c] = az;
+      sto(a.advx + kb, o, ax);
+      sto(a.advy + kb, o, ay);
+      sto(a.advz + kb, o, az);
     } else {
       float st = L.st0;
       if (TH) st = st - L.t11v * L.thtv;
       st = st + ((ax + ay) + az + sc * L.dv) * P.rr0[k];
-      if (a.out_sten) a.out_sten[c] = st;
+      if (a.out_sten) sto(a.out_sten + kb, o, st);
       if (a.out_new) {
         float v = L.sv0 + a.dt * st;
         if (a.smeps_flush && fabsf(v) < P.K.smeps) v = 0.0f;
-        a.out_new[c] = v;
+        sto(a.out_new + kb, o, v);
       }
     }
     fz_lo = fz_hi;
@@ -384,14 +400,8 @@ __device__ __forceinline__ void advs_col(const KP &P, const AdvsArgs &a, const C
 // (src/solve2.F:1416-1426, :1518-1528).
 template <bool WENO, bool SADD, bool TH, bool MODE1>
 static void advs_launch(cm1g_model *m, const KP &P, const AdvsArgs &a, const ColGrid &cg) {
-  // 8 waves per SIMD (64 registers) for the fifth-order scalar passes: the
-  // 4096 workgroups of a 1024 x 1024 grid then run in exactly two rounds (7
-  // waves per SIMD leave a third round 29% full).  Measured per launch: q
-  // 849 against 943 us, the pdef pass 793 against 866 us (both without
-  // spilling), theta 1158 against 1185 us (20 bytes per lane spilled)
-  constexpr int W = (CM1G_COL_WAVES >= 1 && !WENO && (!TH || CM1G_COL_WAVES >= 2)) ? 8 : 0;
-  launch<256, W>(m, col_blocks(cg), col_threads(cg),
-                 [=] __device__(int bx, int, int) { advs_col<WENO, SADD, TH, MODE1>(P, a, cg, bx); });
+  launch<256>(m, col_blocks(cg), col_threads(cg),
+              [=] __device__(int bx, int, int) { advs_col<WENO, SADD, TH, MODE1>(P, a, cg, bx); });
 }
 
 void advs_run(cm1g_model *m, int nrk, const float *s_in, float sadd, const float *s0,
@@ -435,7 +445,8 @@ void advs_run(cm1g_model *m, int nrk, const float *s_in, float sadd, const float
     // the pdef pass: advx/advy/advz only (the t11 term is added by pdef_z)
     return weno ? advs_launch<true, false, false, true> : advs_launch<false, false, false, true>;
   };
-  const ColGrid cg = col_grid(ni, nj, m->tile_rows);
+  ColGrid cg = col_grid(ni, nj, m->tile_rows);
+  col_split(m, cg, nk);
   // an in-place update (out_new aliasing the advected field) writes a
   // partner array, since neighbouring columns still read the old values;
   // the field and its partner then exchange buffers
@@ -475,7 +486,11 @@ void advs_run(cm1g_model *m, int nrk, const float *s_in, float sadd, const float
     pa.smeps_flush = smeps_flush;
     launch<256>(m, dim3((ni + 63) / 64, (nj + 3) / 4, nk), dim3(64, 4, 1),
                 [=] __device__(int bx, int by, int bz) { pdef_xy(P, pa, bx, by, bz); });
-    launch<256>(m, col_blocks(cg), col_threads(cg), [=] __device__(int bx, int, int) { pdef_z(P, pa, cg, bx); });
+    // (a segment's start costs pdef_z five evaluations of dum: large grids
+    // stay uncut, 848 against 901 us at 1024 x 1024 x 96)
+    ColGrid cz = col_grid(ni, nj, m->tile_rows);
+    col_split(m, cz, nk, false);
+    launch<256>(m, col_blocks(cz), col_threads(cz), [=] __device__(int bx, int, int) { pdef_z(P, pa, cz, bx); });
   }
   if (inplace) {
     // the partner now holds the new field: exchange the two buffers

@@ -19,6 +19,7 @@ struct AdvmArgs {
   float *ten;                        // uten / vten / wten
   double weps;
   int buoy;                          // w: add the buoyancy term (src/solve2.F:899-907)
+  int copy;                          // copy ten_in to ten where the component is not advected
   int i1, i2, j1, j2;                // point range of the staggered grid
 };
 
@@ -35,70 +36,80 @@ struct AdvmLevel {
   float wnew;                          // a(k+4), entering the vertical window
 };
 
+// o: the column's byte offset in a level; the start of level k of an array,
+// and of its neighbouring rows, is formed in scalar registers
 template <int STAG, bool OWN>
-__device__ __forceinline__ void advm_load(const KP &P, const AdvmArgs &g, int i, int j, int k,
+__device__ __forceinline__ void advm_load(const KP &P, const AdvmArgs &g, unsigned o, int k,
                                           AdvmLevel &L) {
-  const int px = P.px, pxy = P.pxy, nk = P.nk;
-  const int c = IXD(P, i, j, k);
-  const float *a = g.a;
-  L.xm3 = a[c - 3]; L.xm2 = a[c - 2]; L.xm1 = a[c - 1];
-  L.xp1 = a[c + 1]; L.xp2 = a[c + 2]; L.xp3 = a[c + 3];
-  L.ym3 = a[c - 3 * px]; L.ym2 = a[c - 2 * px]; L.ym1 = a[c - px];
-  L.yp1 = a[c + px]; L.yp2 = a[c + 2 * px]; L.yp3 = a[c + 3 * px];
-  L.ten = g.ten_in[c];
+  const int nk = P.nk;
+  const int px = P.px;
+  const size_t kb = (size_t)k * P.pxy, pxy = (size_t)P.pxy;
+  const float *a = g.a + kb, *ru = g.rru + kb, *rv = g.rrv + kb, *rw = g.rrw + kb, *dx = g.divx + kb;
+  L.xm3 = ldo(a - 3, o); L.xm2 = ldo(a - 2, o); L.xm1 = ldo(a - 1, o);
+  L.xp1 = ldo(a + 1, o); L.xp2 = ldo(a + 2, o); L.xp3 = ldo(a + 3, o);
+  L.ym3 = ldo(a - 3 * px, o); L.ym2 = ldo(a - 2 * px, o); L.ym1 = ldo(a - px, o);
+  L.yp1 = ldo(a + px, o); L.yp2 = ldo(a + 2 * px, o); L.yp3 = ldo(a + 3 * px, o);
+  L.ten = ldo(g.ten_in + kb, o);
   if (STAG == 2) {
     // rru(i-1), rru(i), rru(i+1); rrv(i,j), rrv(i-1,j), rrv(i,j+1), rrv(i-1,j+1)
     if (!OWN) {
-      L.r0 = g.rru[c - 1]; L.r1 = g.rru[c]; L.r2 = g.rru[c + 1];
+      L.r0 = ldo(ru - 1, o); L.r1 = ldo(ru, o); L.r2 = ldo(ru + 1, o);
     }
-    L.r3 = g.rrv[c]; L.q0 = g.rrv[c - 1]; L.q1 = g.rrv[c + px];
-    L.b8 = g.rrv[c + px - 1];
+    L.r3 = ldo(rv, o); L.q0 = ldo(rv - 1, o); L.q1 = ldo(rv + px, o);
+    L.b8 = ldo(rv + px - 1, o);
     // vertical face k+1: rrw(i,k+1), rrw(i-1,k+1)
-    L.wz0 = (k < nk) ? g.rrw[c + pxy] : 0.0f;
-    L.wz1 = (k < nk) ? g.rrw[c + pxy - 1] : 0.0f;
-    L.dv0 = g.divx[c]; L.dv1 = g.divx[c - 1];
-    L.wnew = (k + 4 <= nk) ? a[c + 4 * pxy] : 0.0f;
+    L.wz0 = (k < nk) ? ldo(rw + pxy, o) : 0.0f;
+    L.wz1 = (k < nk) ? ldo(rw + pxy - 1, o) : 0.0f;
+    L.dv0 = ldo(dx, o); L.dv1 = ldo(dx - 1, o);
+    L.wnew = (k + 4 <= nk) ? ldo(a + 4 * pxy, o) : 0.0f;
   } else if (STAG == 3) {
     // rrv(j-1), rrv(j), rrv(j+1); rru(i,j), rru(i,j-1), rru(i+1,j), rru(i+1,j-1)
     if (!OWN) {
-      L.r0 = g.rrv[c - px]; L.r1 = g.rrv[c]; L.r2 = g.rrv[c + px];
+      L.r0 = ldo(rv - px, o); L.r1 = ldo(rv, o); L.r2 = ldo(rv + px, o);
     }
-    L.r3 = g.rru[c]; L.q0 = g.rru[c - px]; L.q1 = g.rru[c + 1];
-    L.b8 = g.rru[c + 1 - px];
-    L.wz0 = (k < nk) ? g.rrw[c + pxy] : 0.0f;
-    L.wz1 = (k < nk) ? g.rrw[c + pxy - px] : 0.0f;
-    L.dv0 = g.divx[c]; L.dv1 = g.divx[c - px];
-    L.wnew = (k + 4 <= nk) ? a[c + 4 * pxy] : 0.0f;
+    L.r3 = ldo(ru, o); L.q0 = ldo(ru - px, o); L.q1 = ldo(ru + 1, o);
+    L.b8 = ldo(ru - px + 1, o);
+    L.wz0 = (k < nk) ? ldo(rw + pxy, o) : 0.0f;
+    L.wz1 = (k < nk) ? ldo(rw + pxy - px, o) : 0.0f;
+    L.dv0 = ldo(dx, o); L.dv1 = ldo(dx - px, o);
+    L.wnew = (k + 4 <= nk) ? ldo(a + 4 * pxy, o) : 0.0f;
   } else {
     // rru(i), rru(i+1), rrv(j), rrv(j+1) at level k
-    L.r0 = g.rru[c]; L.r1 = g.rru[c + 1]; L.r2 = g.rrv[c]; L.r3 = g.rrv[c + px];
+    L.r0 = ldo(ru, o); L.r1 = ldo(ru + 1, o); L.r2 = ldo(rv, o); L.r3 = ldo(rv + px, o);
     L.q0 = L.q1 = 0.0f;
     // vertical face k (between w(k) and w(k+1)): rrw(k), rrw(k+1)
     if (!OWN) {
-      L.wz0 = g.rrw[c];
-      L.wz1 = g.rrw[c + pxy];
+      L.wz0 = ldo(rw, o);
+      L.wz1 = ldo(rw + pxy, o);
     }
-    L.dv0 = g.divx[c]; L.dv1 = 0.0f;
-    L.b8 = g.buoy ? g.dum8[c] : 0.0f;
-    L.wnew = (k + 4 <= nk + 1) ? a[c + 4 * pxy] : 0.0f;
+    L.dv0 = ldo(dx, o); L.dv1 = 0.0f;
+    L.b8 = g.buoy ? ldo(g.dum8 + kb, o) : 0.0f;
+    L.wnew = (k + 4 <= nk + 1) ? ldo(a + 4 * pxy, o) : 0.0f;
   }
 }
 
 template <int STAG, bool WENO, bool OWN>
 __device__ __forceinline__ void advm_col(const KP &P, const AdvmArgs &g, const ColGrid &cg, int bx) {
-  int i, j;
-  if (!col_tile_b(cg, bx, i, j)) return;
-  if (i < g.i1 || i > g.i2 || j < g.j1 || j > g.j2) return;
+  int i, j, ks, ke;
   const int ni = P.ni, nj = P.nj, nk = P.nk;
+  if (!col_tile_seg(cg, bx, nk, i, j, ks, ke)) return;
+  const unsigned o = 4u * (unsigned)IX2D(P, i, j);
+  const size_t pxy = (size_t)P.pxy;
+  if (i < g.i1 || i > g.i2 || j < g.j1 || j > g.j2) {
+    if (g.copy && i <= ni + 1 && j <= nj + 1)
+      for (int k = ks; k <= ke; k++) sto(g.ten + (size_t)k * pxy, o, ldo(g.ten_in + (size_t)k * pxy, o));
+    return;
+  }
+  if (STAG == 4 && g.copy && ks == 1) sto(g.ten + pxy, o, ldo(g.ten_in + pxy, o));
   const bool doitw = (P.wbc == 2 && P.ibw == 1), doite = (P.ebc == 2 && P.ibe == 1);
   const bool doits = (P.sbc == 2 && P.ibs == 1), doitn = (P.nbc == 2 && P.ibn == 1);
-  const float *a = g.a;
   const double weps = g.weps;
   auto val = [&](int kk) -> float {  // column value at level kk (stencil range only)
     if (kk < 0 || kk > nk + 1) return 0.0f;
-    return a[IXD(P, i, j, kk)];
+    return ldo(g.a + (size_t)kk * pxy, o);
   };
-  const int k0 = (STAG == 4) ? 2 : 1;
+  // (w is advanced from level 2 on)
+  const int k0 = (STAG == 4 && ks < 2) ? 2 : ks;
   // vertical window: u, v use S(kf-3..kf+2) for face kf = k+1 (w0..w5 =
   // a(k-2..k+3)); w uses S(k-2..k+3) for face k (w0..w5 = a(k-2..k+3))
   float w0 = val(k0 - 2), w1 = val(k0 - 1), w2 = val(k0), w3 = val(k0 + 1), w4 = val(k0 + 2),
@@ -106,28 +117,39 @@ __device__ __forceinline__ void advm_col(const KP &P, const AdvmArgs &g, const C
   float fz_lo = 0.0f;
   // w: the level k-1 horizontal mass fluxes, divx, dum8 and face k-1 flux
   float pr0 = 0.0f, pr1 = 0.0f, pr2 = 0.0f, pr3 = 0.0f, pdv = 0.0f, pb8 = 0.0f;
-  if (STAG == 4) {
-    const int c1 = IXD(P, i, j, 1);
-    pr0 = g.rru[c1]; pr1 = g.rru[c1 + 1]; pr2 = g.rrv[c1]; pr3 = g.rrv[c1 + P.px];
-    pdv = g.divx[c1];
-    pb8 = g.buoy ? g.dum8[c1] : 0.0f;
-    // face 1
-    auto S1 = [=](int kk) -> float {  // S(kk) = a(kk): the window holds a(0..5)
-      const int o = kk - 2;
-      return o == -2 ? w0 : o == -1 ? w1 : o == 0 ? w2 : o == 1 ? w3 : o == 2 ? w4 : w5;
-    };
-    const float rw1 = OWN ? 0.0f : g.rrw[c1];
-    // the window holds a(0..5) here: w(2) = w2
-    const float rw2 = OWN ? ((nk >= 2) ? P.rf0[2] * w2 : 0.0f) : g.rrw[c1 + P.pxy];
-    const float wb = 0.5f * (rw1 + rw2);
-    fz_lo = WENO ? vfluxw_of(P, 4, wb, S1, 1, 0, weps) : vflux5_of(P, 4, wb, S1, 1);
-  }
   AdvmLevel nx;
-  advm_load<STAG, OWN>(P, g, i, j, k0, nx);
-  for (int k = k0; k <= nk; k++) {
+  advm_load<STAG, OWN>(P, g, o, k0, nx);
+  if (STAG == 4) {
+    const int km = k0 - 1;
+    const size_t mb = (size_t)km * pxy;
+    pr0 = ldo(g.rru + mb, o); pr1 = ldo(g.rru + mb + 1, o); pr2 = ldo(g.rrv + mb, o);
+    pr3 = ldo(g.rrv + mb + P.px, o);
+    pdv = ldo(g.divx + mb, o);
+    pb8 = g.buoy ? ldo(g.dum8 + mb, o) : 0.0f;
+    // face k0 - 1, from a(k0-3..k0+2)
+    const float wm = val(k0 - 3);
+    auto S1 = [=](int kk) -> float {
+      const int q = kk - km;
+      return q == -2 ? wm : q == -1 ? w0 : q == 0 ? w1 : q == 1 ? w2 : q == 2 ? w3 : w4;
+    };
+    const float rw1 = OWN ? ((km == 1) ? 0.0f : P.rf0[km] * w1) : ldo(g.rrw + mb, o);
+    const float rw2 = OWN ? P.rf0[k0] * w2 : ldo(g.rrw + mb + pxy, o);
+    const float wb = 0.5f * (rw1 + rw2);
+    fz_lo = WENO ? vfluxw_of(P, 4, wb, S1, km, 0, weps) : vflux5_of(P, 4, wb, S1, km);
+  } else if (ks > 1) {
+    // u, v: the flux through a segment's lowest face, from a(ks-3..ks+2)
+    const float wm = val(ks - 3);
+    auto S = [=](int kk) -> float {
+      const int q = kk - ks;
+      return q == -3 ? wm : q == -2 ? w0 : q == -1 ? w1 : q == 0 ? w2 : q == 1 ? w3 : w4;
+    };
+    const float *rw = g.rrw + (size_t)ks * pxy;
+    const float wb = 0.5f * (ldo(rw, o) + ldo(STAG == 2 ? rw - 1 : rw - P.px, o));
+    fz_lo = WENO ? vfluxw_of(P, STAG, wb, S, ks, 0, weps) : vflux5_of(P, STAG, wb, S, ks);
+  }
+  for (int k = k0; k <= ke; k++) {
     AdvmLevel L = nx;
-    if (k < nk) advm_load<STAG, OWN>(P, g, i, j, k + 1, nx);
-    const int c = IXD(P, i, j, k);
+    if (k < ke) advm_load<STAG, OWN>(P, g, o, k + 1, nx);
     if (OWN) {
       if (STAG == 2) {
         const float r = P.rho0[k];
@@ -147,7 +169,7 @@ __device__ __forceinline__ void advm_col(const KP &P, const AdvmArgs &g, const C
       const float ub1 = 0.5f * (L.r1 + L.r2), ub0 = 0.5f * (L.r0 + L.r1);
       const float fx1 = hface5<WENO>(ub1, L.xm2, L.xm1, sc, L.xp1, L.xp2, L.xp3, 0, weps);
       const float fx0 = hface5<WENO>(ub0, L.xm3, L.xm2, L.xm1, sc, L.xp1, L.xp2, 0, weps);
-      ax = -(fx1 - fx0) * P.rdx * P.uf[i + 2];
+      ax = -(fx1 - fx0) * P.rdx;
       // rrv(i,j) = r3, rrv(i-1,j) = q0, rrv(i,j+1) = q1, rrv(i-1,j+1) = b8
       const float vb0 = 0.5f * (L.r3 + L.q0), vb1 = 0.5f * (L.q1 + L.b8);
       float fy0 = hface5<WENO>(vb0, L.ym3, L.ym2, L.ym1, sc, L.yp1, L.yp2, 0, weps);
@@ -157,9 +179,9 @@ __device__ __forceinline__ void advm_col(const KP &P, const AdvmArgs &g, const C
       const bool fn = doitn && j == nj && (L.q1 + L.b8) <= 0.0f;
       if (fs) fy0 = fy1;
       if (fn) fy1 = fy0_raw;
-      ay = -(fy1 - fy0) * P.rdy * P.vh[j + 2];
-      if (fs) ay = ay - sc * 0.5f * ((L.b8 - L.q0) + (L.q1 - L.r3)) * P.rdy * P.vh[1 + 2];
-      if (fn) ay = ay - sc * 0.5f * ((L.b8 - L.q0) + (L.q1 - L.r3)) * P.rdy * P.vh[nj + 2];
+      ay = -(fy1 - fy0) * P.rdy;
+      if (fs) ay = ay - sc * 0.5f * ((L.b8 - L.q0) + (L.q1 - L.r3)) * P.rdy;
+      if (fn) ay = ay - sc * 0.5f * ((L.b8 - L.q0) + (L.q1 - L.r3)) * P.rdy;
       float fz_hi = 0.0f;
       if (k < nk) {
         const int kf = k + 1;
@@ -186,13 +208,13 @@ __device__ __forceinline__ void advm_col(const KP &P, const AdvmArgs &g, const C
       const bool fe = doite && i == ni && (L.q1 + L.b8) <= 0.0f;
       if (fw) fx0 = fx1;
       if (fe) fx1 = fx0_raw;
-      ax = -(fx1 - fx0) * P.rdx * P.uh[i + 2];
-      if (fw) ax = ax - sc * 0.5f * ((L.b8 - L.q0) + (L.q1 - L.r3)) * P.rdx * P.uh[1 + 2];
-      if (fe) ax = ax - sc * 0.5f * ((L.b8 - L.q0) + (L.q1 - L.r3)) * P.rdx * P.uh[ni + 2];
+      ax = -(fx1 - fx0) * P.rdx;
+      if (fw) ax = ax - sc * 0.5f * ((L.b8 - L.q0) + (L.q1 - L.r3)) * P.rdx;
+      if (fe) ax = ax - sc * 0.5f * ((L.b8 - L.q0) + (L.q1 - L.r3)) * P.rdx;
       const float vb1 = 0.5f * (L.r1 + L.r2), vb0 = 0.5f * (L.r0 + L.r1);
       const float fy1 = hface5<WENO>(vb1, L.ym2, L.ym1, sc, L.yp1, L.yp2, L.yp3, 0, weps);
       const float fy0 = hface5<WENO>(vb0, L.ym3, L.ym2, L.ym1, sc, L.yp1, L.yp2, 0, weps);
-      ay = -(fy1 - fy0) * P.rdy * P.vf[j + 2];
+      ay = -(fy1 - fy0) * P.rdy;
       float fz_hi = 0.0f;
       if (k < nk) {
         const int kf = k + 1;
@@ -220,9 +242,9 @@ __device__ __forceinline__ void advm_col(const KP &P, const AdvmArgs &g, const C
       const bool fe = doite && i == ni && ub1 <= 0.0f;
       if (fw) fx0 = fx1;
       if (fe) fx1 = fx0_raw;
-      ax = -(fx1 - fx0) * P.rdx * P.uh[i + 2];
-      if (fw) ax = ax - sc * (P.c1[k] * (pr1 - pr0) + P.c2[k] * (L.r1 - L.r0)) * P.rdx * P.uh[1 + 2];
-      if (fe) ax = ax - sc * (P.c1[k] * (pr1 - pr0) + P.c2[k] * (L.r1 - L.r0)) * P.rdx * P.uh[ni + 2];
+      ax = -(fx1 - fx0) * P.rdx;
+      if (fw) ax = ax - sc * (P.c1[k] * (pr1 - pr0) + P.c2[k] * (L.r1 - L.r0)) * P.rdx;
+      if (fe) ax = ax - sc * (P.c1[k] * (pr1 - pr0) + P.c2[k] * (L.r1 - L.r0)) * P.rdx;
       const float vb0 = cc2 * L.r2 + cc1 * pr2, vb1 = cc2 * L.r3 + cc1 * pr3;
       float fy0 = hface5<WENO>(vb0, L.ym3, L.ym2, L.ym1, sc, L.yp1, L.yp2, 0, weps);
       float fy1 = hface5<WENO>(vb1, L.ym2, L.ym1, sc, L.yp1, L.yp2, L.yp3, 0, weps);
@@ -231,9 +253,9 @@ __device__ __forceinline__ void advm_col(const KP &P, const AdvmArgs &g, const C
       const bool fn = doitn && j == nj && vb1 <= 0.0f;
       if (fs) fy0 = fy1;
       if (fn) fy1 = fy0_raw;
-      ay = -(fy1 - fy0) * P.rdy * P.vh[j + 2];
-      if (fs) ay = ay - sc * (P.c1[k] * (pr3 - pr2) + P.c2[k] * (L.r3 - L.r2)) * P.rdy * P.vh[1 + 2];
-      if (fn) ay = ay - sc * (P.c1[k] * (pr3 - pr2) + P.c2[k] * (L.r3 - L.r2)) * P.rdy * P.vh[nj + 2];
+      ay = -(fy1 - fy0) * P.rdy;
+      if (fs) ay = ay - sc * (P.c1[k] * (pr3 - pr2) + P.c2[k] * (L.r3 - L.r2)) * P.rdy;
+      if (fn) ay = ay - sc * (P.c1[k] * (pr3 - pr2) + P.c2[k] * (L.r3 - L.r2)) * P.rdy;
       // vertical face k from a(k-2..k+3)
       auto S = [=](int kk) -> float {
         const int o = kk - k;
@@ -247,36 +269,13 @@ __device__ __forceinline__ void advm_col(const KP &P, const AdvmArgs &g, const C
       if (g.buoy) t = t + (P.c1[k] * pb8 + P.c2[k] * L.b8);
       pr0 = L.r0; pr1 = L.r1; pr2 = L.r2; pr3 = L.r3; pdv = L.dv0; pb8 = L.b8;
     }
-    g.ten[c] = t;
+    sto(g.ten + (size_t)k * pxy, o, t);
     w0 = w1;
     w1 = w2;
     w2 = w3;
     w3 = w4;
     w4 = w5;
     w5 = L.wnew;
-  }
-}
-
-// With from_ten1 the tendencies start from uten1/vten1/wten1 (the copy of
-// src/solve2.F:459-471): the advection kernels read them, and this kernel
-// copies the points they do not write (the faces i=ni+1 / j=nj+1, the
-// open-boundary faces outside the advected range, and w at k=1).
-__device__ __forceinline__ void ten_edges(const KP &P, const float *u1, const float *v1, const float *w1,
-                                          float *u, float *v, float *w, int ui1, int ui2, int vj1,
-                                          int vj2, int bx, int by) {
-  const int i = 1 + bx * (int)blockDim.x + (int)threadIdx.x;
-  const int j = 1 + by * (int)blockDim.y + (int)threadIdx.y;
-  const int ni = P.ni, nj = P.nj, nk = P.nk;
-  if (i > ni + 1 || j > nj + 1) return;
-  const bool ucol = (j == nj + 1) || i < ui1 || i > ui2;
-  const bool vcol = (i == ni + 1) || j < vj1 || j > vj2;
-  const bool wcol = (i == ni + 1) || (j == nj + 1);
-  for (int k = 1; k <= nk; k++) {
-    const int c = IXD(P, i, j, k);
-    if (ucol) u[c] = u1[c];
-    if (vcol) v[c] = v1[c];
-    if (wcol || k == 1) w[c] = w1[c];
-    if (!(ucol || vcol || wcol)) break;
   }
 }
 
@@ -304,15 +303,11 @@ void advm_run(cm1g_model *m, int nrk, int mask, int buoy, int from_ten1, int own
   g.buoy = buoy;
   const int ui1 = P.ibw == 1 ? 2 : 1, ui2 = P.ibe == 1 ? ni : ni + 1;
   const int vj1 = P.ibs == 1 ? 2 : 1, vj2 = P.ibn == 1 ? nj : nj + 1;
-  if (from_ten1) {
-    // the launch covers all three components, so every mask bit must be set
-    const float *u1 = m->f[CM1G_UTEN1], *v1 = m->f[CM1G_VTEN1], *w1 = m->f[CM1G_WTEN1];
-    float *u = m->f[CM1G_UTEN], *v = m->f[CM1G_VTEN], *w = m->f[CM1G_WTEN];
-    launch<256>(m, dim3((ni + 1 + 63) / 64, (nj + 1 + 3) / 4, 1), dim3(64, 4, 1),
-                [=] __device__(int bx, int by, int) {
-                  ten_edges(P, u1, v1, w1, u, v, w, ui1, ui2, vj1, vj2, bx, by);
-                });
-  }
+  // from uten1/vten1/wten1 (the copy of src/solve2.F:459-471) the kernels
+  // also copy the points they do not advect (the faces i=ni+1 / j=nj+1, the
+  // open-boundary faces, w at k=1), so their tiles cover those columns
+  g.copy = from_ten1;
+  const int ci = from_ten1 ? 1 : 0, cj = from_ten1 ? 1 : 0;
   if (mask & 1) {
     g.a = src3 ? src3[0] : m->f[CM1G_U3D];
     g.ten = m->f[CM1G_UTEN];
@@ -321,7 +316,8 @@ void advm_run(cm1g_model *m, int nrk, int mask, int buoy, int from_ten1, int own
     g.i2 = ui2;
     g.j1 = 1;
     g.j2 = nj;
-    const ColGrid cg = col_grid(ni + 1, nj, m->tile_rows);
+    ColGrid cg = col_grid(ni + 1, nj + cj, m->tile_rows);
+    col_split(m, cg, P.nk);
     auto *kern = own ? (weno ? advm_launch<2, true, true> : advm_launch<2, false, true>)
                      : (weno ? advm_launch<2, true, false> : advm_launch<2, false, false>);
     kern(m, P, g, cg);
@@ -334,7 +330,8 @@ void advm_run(cm1g_model *m, int nrk, int mask, int buoy, int from_ten1, int own
     g.i2 = ni;
     g.j1 = vj1;
     g.j2 = vj2;
-    const ColGrid cg = col_grid(ni, nj + 1, m->tile_rows);
+    ColGrid cg = col_grid(ni + ci, nj + 1, m->tile_rows);
+    col_split(m, cg, P.nk);
     auto *kern = own ? (weno ? advm_launch<3, true, true> : advm_launch<3, false, true>)
                      : (weno ? advm_launch<3, true, false> : advm_launch<3, false, false>);
     kern(m, P, g, cg);
@@ -347,7 +344,8 @@ void advm_run(cm1g_model *m, int nrk, int mask, int buoy, int from_ten1, int own
     g.i2 = ni;
     g.j1 = 1;
     g.j2 = nj;
-    const ColGrid cg = col_grid(ni, nj, m->tile_rows);
+    ColGrid cg = col_grid(ni + ci, nj + cj, m->tile_rows);
+    col_split(m, cg, P.nk);
     auto *kern = own ? (weno ? advm_launch<4, true, true> : advm_launch<4, false, true>)
                      : (weno ? advm_launch<4, true, false> : advm_launch<4, false, false>);
     kern(m, P, g, cg);
@@ -366,6 +364,7 @@ void advw_tke(cm1g_model *m, int nrk, int advweno, const float *rru, const float
   g.dum8 = m->f[CM1G_DUM8];
   g.weps = (double)(100.0f * P.K.epsilon);
   g.buoy = 0;
+  g.copy = 0;
   g.a = a;
   g.ten_in = ten_in;
   g.ten = ten;
@@ -373,7 +372,8 @@ void advw_tke(cm1g_model *m, int nrk, int advweno, const float *rru, const float
   g.i2 = P.ni;
   g.j1 = 1;
   g.j2 = P.nj;
-  const ColGrid cg = col_grid(P.ni, P.nj, m->tile_rows);
+  ColGrid cg = col_grid(P.ni, P.nj, m->tile_rows);
+    col_split(m, cg, P.nk);
   auto *kern = weno ? advm_launch<4, true, false> : advm_launch<4, false, false>;
   kern(m, P, g, cg);
 }

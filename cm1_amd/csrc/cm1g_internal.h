@@ -273,13 +273,6 @@ void launch_many(hipStream_t s, const void *fs, const BatchSlot *slots, int nmem
     hipLaunchKernelGGL((k_many<NT, F>), dim3(nblocks), block, 0, s, (const F *)fs, slots, nmem);
 }
 
-// Scalar advection column kernels compiled for 8 waves per SIMD: 0 none
-// (the compiler's choice), 1 the fifth-order passes of q and the pdef pass,
-// 2 also theta's.
-#ifndef CM1G_COL_WAVES
-#define CM1G_COL_WAVES 2
-#endif
-
 // W > 0: the kernel is compiled for at least W waves per SIMD
 template <int NT, int W = 0, class F>
 inline void launch(cm1g_model *m, dim3 g, dim3 b, const F &f) {
@@ -348,6 +341,7 @@ constexpr int NXCD = 8;
 struct ColGrid {
   int gx, gy, ty, nb, per;  // tiles in i and j, tile rows, tiles, tiles per XCD
   int i0, j0;               // first column of tile 0 (i0 on a line start)
+  int nseg, slen;           // segments a column is split into, levels of each (col_split)
 };
 // columns i = 1..ni, j = 1..nj
 inline ColGrid col_grid(int ni, int nj, int ty = 4) {
@@ -359,6 +353,8 @@ inline ColGrid col_grid(int ni, int nj, int ty = 4) {
   g.per = (g.nb + NXCD - 1) / NXCD;
   g.i0 = 1;
   g.j0 = 1;
+  g.nseg = 1;
+  g.slen = 1 << 30;
   return g;
 }
 // columns covering [ilo,ihi] x [jlo,jhi], tiles aligned as for3 aligns them
@@ -369,6 +365,30 @@ inline ColGrid col_grid_box(int ilo, int ihi, int jlo, int jhi, int ty = 4) {
   g.i0 = i0;
   g.j0 = jlo;
   return g;
+}
+// Split the levels k = 1..nk of a marching kernel whose levels depend on
+// their neighbours only (advection, mass fluxes) into segments, each marched
+// by a wavefront of its own that first forms what the level below its first
+// one would have left it (about two levels' work).  A column's levels take
+// their loads' latency one after the other (1 to 2 us a level), so a grid
+// with few columns is cut until 16384 wavefronts run (16 per SIMD), with no
+// segment under 4 levels.  Measured per step, uncut -> cut: 64 x 64 x 40 2.57
+// -> 1.10 ms, 301 x 227 x 63 4.9 -> 4.0 ms; 4096 or 8192 wavefronts 3 to 10%
+// slower at 301 x 227 x 63 and 512 x 512 x 128, at least 8 levels 10% slower
+// at 64 x 64 x 40, 3 levels within 3%.  With `even`, larger grids are cut
+// too, into segments of 24 levels: shorter workgroups leave less of the chip
+// idle at a launch's end, and no cap on registers is needed for the rounds
+// to come out even (1024 x 1024 x 96: advs 849 -> 779 us, theta 1150 -> 1019
+// us, advw 909 -> 750 us; segments of 12 levels the same).
+inline void col_split(const cm1g_model *m, ColGrid &g, int nk, bool even = true) {
+  const long rows = m->plan_tiles > 0 ? m->plan_tiles : (long)g.gx * g.gy * g.ty;
+  int n = (int)((16384 + rows - 1) / rows);
+  if (n > nk / 4) n = nk / 4;
+  if (even && n < nk / 24) n = nk / 24;
+  if (n < 1) n = 1;
+  g.slen = (nk + n - 1) / n;
+  g.nseg = (nk + g.slen - 1) / g.slen;
+  g.per = (g.nb * g.nseg + NXCD - 1) / NXCD;
 }
 inline dim3 col_blocks(const ColGrid &g) { return dim3(g.per * NXCD, 1, 1); }
 inline dim3 col_threads(const ColGrid &g) { return dim3(64 * g.ty, 1, 1); }
@@ -381,6 +401,24 @@ __device__ __forceinline__ bool col_tile_b(const ColGrid &g, int b, int &i, int 
   j = g.j0 + (t / g.gx) * g.ty + (int)(threadIdx.x >> 6);
   return true;
 }
+
+// the same for a split column: the segment's levels are ks..ke of 1..nk
+__device__ __forceinline__ bool col_tile_seg(const ColGrid &g, int b, int nk, int &i, int &j, int &ks, int &ke) {
+  const int t = (b % NXCD) * g.per + b / NXCD;
+  if (t >= g.nb * g.nseg) return false;
+  const int seg = t / g.nb, q = t - seg * g.nb;
+  i = g.i0 + (q % g.gx) * 64 + (int)(threadIdx.x & 63);
+  j = g.j0 + (q / g.gx) * g.ty + (int)(threadIdx.x >> 6);
+  ks = 1 + seg * g.slen;
+  ke = ks + g.slen - 1 < nk ? ks + g.slen - 1 : nk;
+  return true;
+}
+
+// A load (store) at a byte offset from an array's (or a level's) base: the
+// base stays in scalar registers, the offset is one 32-bit register that
+// serves every array.
+__device__ __forceinline__ float ldo(const float *p, unsigned o) { return *(const float *)((const char *)p + o); }
+__device__ __forceinline__ void sto(float *p, unsigned o, float v) { *(float *)((char *)p + o) = v; }
 
 // ---------------------------------------------------------- reductions
 // Reduction over a 256-thread workgroup in the pairing order of a halving

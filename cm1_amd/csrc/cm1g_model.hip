@@ -793,7 +793,7 @@ __device__ __forceinline__ void mass_level_sums(const KP &P, const float *rho, c
   for (int j = 1 + b; j <= P.nj; j += MASS_NB)
     for (int i = 1 + (int)threadIdx.x; i <= P.ni; i += blockDim.x) {
       int c = IXD(P, i, j, k);
-      a3 += (double)(rho[c] * P.ruh[i + 2] * P.rvh[j + 2] * P.rmh[k]);
+      a3 += (double)(rho[c] * P.rmh[k]);
       a4 += (double)(P.pi0[k] + pp3d[c]);
     }
   a3 = block_reduce256(a3, r3, OpAdd());
@@ -960,43 +960,44 @@ extern "C" int cm1g_getset(cm1g_model *m, int fresh_start) {
 __device__ __forceinline__ void massflux_div(const KP &P, const float *u3d, const float *v3d, const float *w3d,
                                              float *rru, float *rrv, float *rrw, float *divx,
                                              const ColGrid &cg, int bx) {
-  int i, j;
-  if (!col_tile_b(cg, bx, i, j)) return;
+  int i, j, ks, ke;
   const int ni = P.ni, nj = P.nj, nk = P.nk;
+  if (!col_tile_seg(cg, bx, nk, i, j, ks, ke)) return;
   if (i < 0 || i > ni + 2 || j > nj + 2) return;
   const bool du = (j <= nj + 1), dv = (i <= ni + 1), dd = du && dv;
-  const int px = P.px, pxy = P.pxy;
-  int c = IXD(P, i, j, 1);
-  float u0 = u3d[c], u1 = dd ? u3d[c + 1] : 0.0f, v0 = v3d[c], v1 = dd ? v3d[c + px] : 0.0f;
-  float wk = 0.0f, wk1 = (dd && nk >= 2) ? w3d[c + pxy] : 0.0f;
-  for (int k = 1; k <= nk; k++, c += pxy) {
+  const unsigned o = 4u * (unsigned)IX2D(P, i, j);
+  const size_t pxy = (size_t)P.pxy;
+  size_t kb = (size_t)ks * pxy;
+  float u0 = ldo(u3d + kb, o), u1 = dd ? ldo(u3d + kb + 1, o) : 0.0f;
+  float v0 = ldo(v3d + kb, o), v1 = dd ? ldo(v3d + kb + P.px, o) : 0.0f;
+  float wk = (dd && ks > 1) ? ldo(w3d + kb, o) : 0.0f, wk1 = (dd && ks + 1 <= nk) ? ldo(w3d + kb + pxy, o) : 0.0f;
+  for (int k = ks; k <= ke; k++, kb += pxy) {
     const float cu0 = u0, cu1 = u1, cv0 = v0, cv1 = v1, cw0 = wk, cw1 = wk1;
-    if (k < nk) {
-      const int cn = c + pxy;
-      u0 = u3d[cn];
-      v0 = v3d[cn];
+    if (k < ke) {
+      const size_t nb = kb + pxy;
+      u0 = ldo(u3d + nb, o);
+      v0 = ldo(v3d + nb, o);
       if (dd) {
-        u1 = u3d[cn + 1];
-        v1 = v3d[cn + px];
+        u1 = ldo(u3d + nb + 1, o);
+        v1 = ldo(v3d + nb + P.px, o);
         wk = cw1;
-        wk1 = (k + 1 < nk) ? w3d[cn + pxy] : 0.0f;
+        wk1 = (k + 1 < nk) ? ldo(w3d + nb + pxy, o) : 0.0f;
       }
     }
     const float r0 = P.rho0[k];
     const float ru0 = r0 * cu0, rv0 = r0 * cv0;
-    if (du) rru[c] = ru0;
-    if (dv) rrv[c] = rv0;
+    if (du) sto(rru + kb, o, ru0);
+    if (dv) sto(rrv + kb, o, rv0);
     if (dd) {
       const float rw0 = (k == 1) ? 0.0f : P.rf0[k] * cw0;
       const float rw1 = (k == nk) ? 0.0f : P.rf0[k + 1] * cw1;
-      rrw[c] = rw0;
-      if (k == nk) rrw[c + pxy] = 0.0f;
+      sto(rrw + kb, o, rw0);
+      if (k == nk) sto(rrw + kb + pxy, o, 0.0f);
       if (i <= ni + 1 && j <= nj + 1) {
         const float ru1 = r0 * cu1, rv1 = r0 * cv1;
-        float d = ((ru1 - ru0) * P.rdx * P.uh[i + 2] + (rv1 - rv0) * P.rdy * P.vh[j + 2]) +
-                  (rw1 - rw0) * P.rdz * P.mh[k];
+        float d = ((ru1 - ru0) * P.rdx + (rv1 - rv0) * P.rdy) + (rw1 - rw0) * P.rdz * P.mh[k];
         if (fabsf(d) < P.K.smeps) d = 0.0f;
-        divx[c] = d;
+        sto(divx + kb, o, d);
       }
     }
   }
@@ -1183,7 +1184,8 @@ extern "C" int cm1g_solve2(cm1g_model *m) {
     bc_fill(m, BC_P, t11);
     // rru, rrv, rrw (src/solve2.F:490-545) and divx (:587-625) in one pass
     {
-      const ColGrid cg = col_grid_box(0, ni + 2, 0, nj + 2, m->tile_rows);
+      ColGrid cg = col_grid_box(0, ni + 2, 0, nj + 2, m->tile_rows);
+      col_split(m, cg, nk);
       launch<256>(m, col_blocks(cg), col_threads(cg), [=] __device__(int bx, int, int) {
         massflux_div(P, u_r, v_r, w_r, rru, rrv, rrw, divx, cg, bx);
       });

@@ -67,14 +67,14 @@ __device__ __forceinline__ float sub_u(const KP &P, const SubArgs &a, int i, int
   float u = a.uX[c];
   if (j >= 1 && j <= P.nj) {
     if (a.opw && i == 1)
-      u = u + a.dts * (-a.radbcw[(j + 2) + k * P.py] * (a.uX[IXD(P, 2, j, k)] - u) * P.rdx * P.uh[1 + 2] +
+      u = u + a.dts * (-a.radbcw[(j + 2) + k * P.py] * (a.uX[IXD(P, 2, j, k)] - u) * P.rdx +
                        a.uten[c]);
     if (a.ope && i == P.ni + 1)
-      u = u + a.dts * (-a.radbce[(j + 2) + k * P.py] * (u - a.uX[IXD(P, P.ni, j, k)]) * P.rdx * P.uh[P.ni + 2] +
+      u = u + a.dts * (-a.radbce[(j + 2) + k * P.py] * (u - a.uX[IXD(P, P.ni, j, k)]) * P.rdx +
                        a.uten[c]);
   }
   const float dtu = a.dts * a.dtu0[IX2D(P, i, j)];
-  return u + dtu * (a.uten[c] - a.tem1 * (a.ppdX[c] - a.ppdX[c - 1]) * P.uf[i + 2] * (a.thv[c] + a.thv[c - 1]));
+  return u + dtu * (a.uten[c] - a.tem1 * (a.ppdX[c] - a.ppdX[c - 1]) * (a.thv[c] + a.thv[c - 1]));
 }
 
 // new v at (i,j,k) (ssopenbcs/n, src/bc.F:2538-2684; src/sound.F:327-345)
@@ -83,15 +83,15 @@ __device__ __forceinline__ float sub_v(const KP &P, const SubArgs &a, int i, int
   float v = a.vX[c];
   if (i >= 1 && i <= P.ni) {
     if (a.ops && j == 1)
-      v = v + a.dts * (-a.radbcs[(i + 2) + k * P.px] * (a.vX[IXD(P, i, 2, k)] - v) * P.rdy * P.vh[1 + 2] +
+      v = v + a.dts * (-a.radbcs[(i + 2) + k * P.px] * (a.vX[IXD(P, i, 2, k)] - v) * P.rdy +
                        a.vten[c]);
     if (a.opn && j == P.nj + 1)
-      v = v + a.dts * (-a.radbcn[(i + 2) + k * P.px] * (v - a.vX[IXD(P, i, P.nj, k)]) * P.rdy * P.vh[P.nj + 2] +
+      v = v + a.dts * (-a.radbcn[(i + 2) + k * P.px] * (v - a.vX[IXD(P, i, P.nj, k)]) * P.rdy +
                        a.vten[c]);
   }
   const float dtv = a.dts * a.dtv0[IX2D(P, i, j)];
   const int cs = c - P.px;
-  return v + dtv * (a.vten[c] - a.tem2 * (a.ppdX[c] - a.ppdX[cs]) * P.vf[j + 2] * (a.thv[c] + a.thv[cs]));
+  return v + dtv * (a.vten[c] - a.tem2 * (a.ppdX[c] - a.ppdX[cs]) * (a.thv[c] + a.thv[cs]));
 }
 
 // the running average r (rru, rrv) with the previous substep's value x0 and
@@ -254,10 +254,10 @@ __device__ __forceinline__ void sound_sub(const KP &P, const SubArgs &a, const C
     const float rw = L.rw, re = L.re, rs = L.rs, rn = L.rn;
     // ---- u, v (ssopenbc* then src/sound.F:307-345)
     float uo0 = uXc, uo1 = uXe, vo0 = vXc, vo1 = vXn;
-    if (bw) uo0 = uo0 + dts * (-rw * (uXe - uo0) * rdx * P.uh[1 + 2] + utc);
-    if (be) uo1 = uo1 + dts * (-re * (uo1 - uXc) * rdx * P.uh[ni + 2] + ute);
-    if (bs) vo0 = vo0 + dts * (-rs * (vXn - vo0) * rdy * P.vh[1 + 2] + vtc);
-    if (bn) vo1 = vo1 + dts * (-rn * (vo1 - vXc) * rdy * P.vh[nj + 2] + vtn);
+    if (bw) uo0 = uo0 + dts * (-rw * (uXe - uo0) * rdx + utc);
+    if (be) uo1 = uo1 + dts * (-re * (uo1 - uXc) * rdx + ute);
+    if (bs) vo0 = vo0 + dts * (-rs * (vXn - vo0) * rdy + vtc);
+    if (bn) vo1 = vo1 + dts * (-rn * (vo1 - vXc) * rdy + vtn);
     const float un0 = uo0 + dtu_c * (utc - tem1 * (pdc - pdw) * uf_c * (thc + thw));
     const float un1 = uo1 + dtu_e * (ute - tem1 * (pde - pdc) * uf_e * (the + thc));
     const float vn0 = vo0 + dtv_c * (vtc - tem2 * (pdc - pds) * vf_c * (thc + ths));
@@ -409,12 +409,8 @@ __device__ __forceinline__ void sound_sub(const KP &P, const SubArgs &a, const C
 //
 // The horizontal metrics uh, uf, vh, vf of sound_sub are all 1 (cm1g_create
 // sets no other), and a product with 1 changes no value: left out here.
-// Loads and stores at a byte offset: fields are below 4 GiB (slab_variant
-// checks it), so one 32-bit offset per point serves every array, with the
-// array's base in scalar registers.
-__device__ __forceinline__ float ldo(const float *p, unsigned o) { return *(const float *)((const char *)p + o); }
-__device__ __forceinline__ void sto(float *p, unsigned o, float v) { *(float *)((char *)p + o) = v; }
-
+// Points are addressed by 32-bit byte offsets (ldo, sto): fields are below
+// 4 GiB (slab_variant checks it).
 struct SlabGrid {
   int nt, gx, per, nj, nw;  // tiles (64 columns x 1 row), tiles along i, tiles per XCD, rows, wavefronts
 };
@@ -924,19 +920,19 @@ void sounde_run(cm1g_model *m, int nrk) {
       for2(m, 1, nj, 1, nk, [=] __device__(int j, int k) {
         if (opw)
           u3d[IXD(P, 1, j, k)] = u3d[IXD(P, 1, j, k)] + dts * (-radbcw[(j + 2) + k * P.py] *
-              (u3d[IXD(P, 2, j, k)] - u3d[IXD(P, 1, j, k)]) * rdx * P.uh[1 + 2] + uten[IXD(P, 1, j, k)]);
+              (u3d[IXD(P, 2, j, k)] - u3d[IXD(P, 1, j, k)]) * rdx + uten[IXD(P, 1, j, k)]);
         if (ope)
           u3d[IXD(P, ni + 1, j, k)] = u3d[IXD(P, ni + 1, j, k)] + dts * (-radbce[(j + 2) + k * P.py] *
-              (u3d[IXD(P, ni + 1, j, k)] - u3d[IXD(P, ni, j, k)]) * rdx * P.uh[ni + 2] + uten[IXD(P, ni + 1, j, k)]);
+              (u3d[IXD(P, ni + 1, j, k)] - u3d[IXD(P, ni, j, k)]) * rdx + uten[IXD(P, ni + 1, j, k)]);
       });
     if (ops || opn)
       for2(m, 1, ni, 1, nk, [=] __device__(int i, int k) {
         if (ops)
           v3d[IXD(P, i, 1, k)] = v3d[IXD(P, i, 1, k)] + dts * (-radbcs[(i + 2) + k * P.px] *
-              (v3d[IXD(P, i, 2, k)] - v3d[IXD(P, i, 1, k)]) * rdy * P.vh[1 + 2] + vten[IXD(P, i, 1, k)]);
+              (v3d[IXD(P, i, 2, k)] - v3d[IXD(P, i, 1, k)]) * rdy + vten[IXD(P, i, 1, k)]);
         if (opn)
           v3d[IXD(P, i, nj + 1, k)] = v3d[IXD(P, i, nj + 1, k)] + dts * (-radbcn[(i + 2) + k * P.px] *
-              (v3d[IXD(P, i, nj + 1, k)] - v3d[IXD(P, i, nj, k)]) * rdy * P.vh[nj + 2] + vten[IXD(P, i, nj + 1, k)]);
+              (v3d[IXD(P, i, nj + 1, k)] - v3d[IXD(P, i, nj, k)]) * rdy + vten[IXD(P, i, nj + 1, k)]);
       });
     // u, v, w forward and the velocity averages
     {
@@ -944,9 +940,9 @@ void sounde_run(cm1g_model *m, int nrk) {
       for3(m, 1, ni + 1, 1, nj + 1, 1, nk, [=] __device__(int i, int j, int k) {
         const int c = IXD(P, i, j, k);
         const float dtu = dts * dtu0[IX2D(P, i, j)], dtv = dts * dtv0[IX2D(P, i, j)];
-        const float u = u3d[c] + dtu * (uten[c] - tem1 * P.uf[i + 2] * (ppd[c] - ppd[c - 1]) *
+        const float u = u3d[c] + dtu * (uten[c] - tem1 * (ppd[c] - ppd[c - 1]) *
                                                       (thv[c] + thv[c - 1]));
-        const float v = v3d[c] + dtv * (vten[c] - tem2 * P.vf[j + 2] * (ppd[c] - ppd[c - P.px]) *
+        const float v = v3d[c] + dtv * (vten[c] - tem2 * (ppd[c] - ppd[c - P.px]) *
                                                       (thv[c] + thv[c - P.px]));
         float w = w3d[c];
         if (k >= 2 && i <= ni && j <= nj) {
@@ -988,11 +984,11 @@ void sounde_run(cm1g_model *m, int nrk) {
         const float u0 = u3d[c], u1 = u3d[c + 1], v0 = v3d[c], v1 = v3d[c + P.px];
         const float w0 = w3d[c], w1 = w3d[c + P.pxy];
         const float pa = piadv[c];
-        float div = ((u1 - u0) * rdx * P.uh[i + 2] + (v1 - v0) * rdy * P.vh[j + 2]) + (w1 - w0) * rdz * mh;
+        float div = ((u1 - u0) * rdx + (v1 - v0) * rdy) + (w1 - w0) * rdz * mh;
         if (fabsf(div) < smeps) div = 0.0f;
         const float delp = dts * (ppten[c] - ppterm[c] * div) +
-                           (-(u0 * (pa - piadv[c - 1]) + u1 * (piadv[c + 1] - pa)) * temx * P.uh[i + 2] -
-                            (v0 * (pa - piadv[c - P.px]) + v1 * (piadv[c + P.px] - pa)) * temy * P.vh[j + 2]) +
+                           (-(u0 * (pa - piadv[c - 1]) + u1 * (piadv[c + 1] - pa)) * temx -
+                            (v0 * (pa - piadv[c - P.px]) + v1 * (piadv[c + P.px] - pa)) * temy) +
                            (w0 * pk1 + w1 * pk2);
         float p = pp3d[c] + delp;
         if (fabsf(p) < smeps) p = 0.0f;
@@ -1024,8 +1020,8 @@ void getdiv_both(cm1g_model *m, int want_t11, int want_divx, float *div) {
   for3(m, 1, ni, 1, nj, 1, nk, [=] __device__(int i, int j, int k) {
     int c = IXD(P, i, j, k);
     if (want_t11) {
-      float d = ((rru[IXD(P, i + 1, j, k)] - rru[c]) * P.rdx * P.uh[i + 2] +
-                 (rrv[IXD(P, i, j + 1, k)] - rrv[c]) * P.rdy * P.vh[j + 2]) +
+      float d = ((rru[IXD(P, i + 1, j, k)] - rru[c]) * P.rdx +
+                 (rrv[IXD(P, i, j + 1, k)] - rrv[c]) * P.rdy) +
                 (rrw[IXD(P, i, j, k + 1)] - rrw[c]) * P.rdz * P.mh[k];
       if (fabsf(d) < smeps) d = 0.0f;
       t11[c] = d;
@@ -1035,7 +1031,7 @@ void getdiv_both(cm1g_model *m, int want_t11, int want_divx, float *div) {
     float rv1 = rrv[IXD(P, i, j + 1, k)] * P.rho0[k], rv0 = rrv[c] * P.rho0[k];
     float rw1 = (k == nk) ? 0.0f : rrw[IXD(P, i, j, k + 1)] * P.rf0[k + 1];
     float rw0 = (k == 1) ? 0.0f : rrw[c] * P.rf0[k];
-    float d = ((ru1 - ru0) * P.rdx * P.uh[i + 2] + (rv1 - rv0) * P.rdy * P.vh[j + 2]) +
+    float d = ((ru1 - ru0) * P.rdx + (rv1 - rv0) * P.rdy) +
               (rw1 - rw0) * P.rdz * P.mh[k];
     if (fabsf(d) < smeps) d = 0.0f;
     divx[c] = d;
@@ -1074,8 +1070,8 @@ __device__ __forceinline__ void cfl_levels(const KP &P, float dt, const float *u
   float cfl = 0.0f;
   for (int j = 1 + b; j <= P.nj; j += CFL_NB)
     for (int i = 1 + (int)threadIdx.x; i <= P.ni; i += blockDim.x) {
-      float a = (ua[IXD(P, i, j, k)] + ua[IXD(P, i + 1, j, k)]) * dtdx * P.uh[i + 2];
-      float bb = (va[IXD(P, i, j, k)] + va[IXD(P, i, j + 1, k)]) * dtdy * P.vh[j + 2];
+      float a = (ua[IXD(P, i, j, k)] + ua[IXD(P, i + 1, j, k)]) * dtdx;
+      float bb = (va[IXD(P, i, j, k)] + va[IXD(P, i, j + 1, k)]) * dtdy;
       float c = (wa[IXD(P, i, j, k)] + wa[IXD(P, i, j, k + 1)]) * dtdz * P.mh[k];
       float wsp = sqrtf((a * a + bb * bb) + c * c);
       cfl = fmaxf(cfl, wsp);
