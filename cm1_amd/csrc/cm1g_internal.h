@@ -420,6 +420,20 @@ __device__ __forceinline__ bool col_tile_seg(const ColGrid &g, int b, int nk, in
 __device__ __forceinline__ float ldo(const float *p, unsigned o) { return *(const float *)((const char *)p + o); }
 __device__ __forceinline__ void sto(float *p, unsigned o, float v) { *(float *)((char *)p + o) = v; }
 
+// The one-point halo fill of an interior value (BC_P, src/bc.F:372-520) by
+// the point that owns it: the copies of (i,j) outside the domain, corners
+// included (the reference fills west/east, then south/north over the filled
+// columns, so a corner holds the value of the interior point both map to).
+__device__ __forceinline__ void put_p_halo(const KP &P, float *p, int i, int j, int k, float v) {
+  const bool w = (i == 1), e = (i == P.ni), s = (j == 1), n = (j == P.nj);
+  if (!(w || e || s || n)) return;
+  const int xi = w ? (P.ebc == 1 ? P.ni + 1 : 0) : (P.wbc == 1 ? 0 : P.ni + 1);
+  const int xj = s ? (P.nbc == 1 ? P.nj + 1 : 0) : (P.sbc == 1 ? 0 : P.nj + 1);
+  if (w || e) p[IXD(P, xi, j, k)] = v;
+  if (s || n) p[IXD(P, i, xj, k)] = v;
+  if ((w || e) && (s || n)) p[IXD(P, xi, xj, k)] = v;
+}
+
 // ---------------------------------------------------------- reductions
 // Reduction over a 256-thread workgroup in the pairing order of a halving
 // tree, v(t) op v(t+128), then op v(t+64), then op v(t+32) ... v(t+1): the
@@ -452,6 +466,13 @@ struct OpMaxF {
 // bc fills (cm1g_bc.hip)
 void bc_fill(cm1g_model *m, int kind, float *a);
 void bc_fill_n(cm1g_model *m, int kind, float *const *arrs, int n);
+// any arrays, each of its own kind, in one launch (at most BC_MAX)
+constexpr int BC_MAX = 24;
+struct BcItem {
+  float *a;
+  int kind;
+};
+void bc_fill_list(cm1g_model *m, const BcItem *it, int n);
 void radbc4(cm1g_model *m, const float *ua, const float *u3d, const float *va,
             const float *v3d, float dt);
 // advection (cm1g_adv.hip)

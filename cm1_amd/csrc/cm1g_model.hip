@@ -814,17 +814,28 @@ __device__ inline void dd_add(double &hi, double &lo, double x) {
   lo += err;
 }
 
+// One workgroup: a thread per level adds its 32 partial sums, one thread
+// then accumulates the levels in order (one thread for all of it took 32 us
+// at 40 levels, 80 us at 96).
 __device__ __forceinline__ void mass_final(int nk, int mode, float rddcv, double ntot, const double *lev,
                                            double *dscal) {
-  double h3 = 0.0, l3 = 0.0, h4 = 0.0, l4 = 0.0;
-  for (int k = 1; k <= nk; k++) {
+  __shared__ double t3[512], t4[512];  // nk <= 510
+  for (int k = 1 + (int)threadIdx.x; k <= nk; k += 256) {
     double s3 = 0.0, s4 = 0.0;
+#pragma unroll 8
     for (int b = 0; b < MASS_NB; b++) {
       s3 += lev[2 * (k * MASS_NB + b)];
       s4 += lev[2 * (k * MASS_NB + b) + 1];
     }
-    dd_add(h3, l3, s3);
-    dd_add(h4, l4, s4);
+    t3[k] = s3;
+    t4[k] = s4;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  double h3 = 0.0, l3 = 0.0, h4 = 0.0, l4 = 0.0;
+  for (int k = 1; k <= nk; k++) {
+    dd_add(h3, l3, t3[k]);
+    dd_add(h4, l4, t4[k]);
   }
   double mass = h3 + l3, p2 = h4 + l4;
   if (mode == 0) {
@@ -845,23 +856,52 @@ static void mass_levels(cm1g_model *m, const float *rho, int mode) {
   const double ntot = (double)((long long)P.ni * P.nj * P.nk);
   const int nk = P.nk;
   const float rddcv = P.K.rddcv;
-  launch<64>(m, dim3(1), dim3(1),
-             [=] __device__(int, int, int) { mass_final(nk, mode, rddcv, ntot, lev, dscal); });
+  launch<256>(m, dim3(1), dim3(256),
+              [=] __device__(int, int, int) { mass_final(nk, mode, rddcv, ntot, lev, dscal); });
 }
 
 // domain rain-accumulation budget (src/kessler.F:470-476): per-row sums in
 // i order, then rows in j order, as the reference does.
+// A workgroup takes 16 rows: its threads bring 16 x 128 values at a time into
+// LDS (whole lines of a row), one thread per row adds them in order.  A
+// thread per row reading its row alone took 118 us at 1024 x 1024.
+constexpr int TR_ROWS = 16, TR_COLS = 128;
 __device__ __forceinline__ void train_rows(int ni, int nj, const double *colbud, double *rows, int bx) {
-  const int j = bx * (int)blockDim.x + (int)threadIdx.x;
-  if (j >= nj) return;
+  __shared__ double tile[2][TR_ROWS][TR_COLS + 1];
+  const int t = (int)threadIdx.x, j0 = bx * TR_ROWS, nrow = min(TR_ROWS, nj - j0);
+  auto fetch = [&](int i0, int p) {
+    for (int e = t; e < TR_ROWS * TR_COLS; e += 256) {
+      const int r = e / TR_COLS, i = i0 + e % TR_COLS;
+      if (r < nrow && i < ni) tile[p][r][e % TR_COLS] = colbud[i + (j0 + r) * ni];
+    }
+  };
   double b = 0.0;
-  for (int i = 0; i < ni; i++) b = b + colbud[i + j * ni];
-  rows[j] = b;
+  fetch(0, 0);
+  __syncthreads();
+  for (int i0 = 0, p = 0; i0 < ni; i0 += TR_COLS, p ^= 1) {
+    if (i0 + TR_COLS < ni) fetch(i0 + TR_COLS, p ^ 1);
+    if (t < nrow) {
+      const int n = min(TR_COLS, ni - i0);
+      for (int q = 0; q < n; q++) b = b + tile[p][t][q];
+    }
+    __syncthreads();
+  }
+  if (t < nrow) rows[j0 + t] = b;
 }
+// the rows' products through LDS, 1024 at a time, added in order by one
+// thread (which read and multiplied them itself before: 65 us at 1024 rows)
 __device__ __forceinline__ void train_sum(int nj, double tem, const double *rows, double *dscal) {
+  __shared__ double x[1024];
   double tr = dscal[3];
-  for (int j = 0; j < nj; j++) tr = tr + rows[j] * tem;
-  dscal[3] = tr;
+  for (int j0 = 0; j0 < nj; j0 += 1024) {
+    const int n = min(1024, nj - j0);
+    for (int q = (int)threadIdx.x; q < n; q += 256) x[q] = rows[j0 + q] * tem;
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (int q = 0; q < n; q++) tr = tr + x[q];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) dscal[3] = tr;
 }
 // train += the fallout's column budgets of this call (the end of
 // src/kessler.F:fallout)
@@ -870,9 +910,9 @@ void train_accumulate(cm1g_model *m) {
   const double *colbud = m->dred;
   double *rows = m->dred + (size_t)ni * nj, *dscal = m->dscal;
   const double tem = (double)(m->c.dx * m->c.dy);
-  launch<64>(m, dim3((nj + 63) / 64), dim3(64),
-             [=] __device__(int bx, int, int) { train_rows(ni, nj, colbud, rows, bx); });
-  launch<64>(m, dim3(1), dim3(1), [=] __device__(int, int, int) { train_sum(nj, tem, rows, dscal); });
+  launch<256>(m, dim3((nj + TR_ROWS - 1) / TR_ROWS), dim3(256),
+              [=] __device__(int bx, int, int) { train_rows(ni, nj, colbud, rows, bx); });
+  launch<256>(m, dim3(1), dim3(256), [=] __device__(int, int, int) { train_sum(nj, tem, rows, dscal); });
 }
 
 // ------------------------------------------------------------------ getset
@@ -882,14 +922,15 @@ extern "C" int cm1g_getset(cm1g_model *m, int fresh_start) {
   const KP P = m->P;
   const int ni = P.ni, nj = P.nj, nk = P.nk;
   float **f = m->f;
-  bc_fill(m, BC_U, f[CM1G_UA]);
-  bc_fill(m, BC_V, f[CM1G_VA]);
-  bc_fill(m, BC_W1, f[CM1G_WA]);
-  bc_fill(m, BC_S, f[CM1G_PPI]);
-  bc_fill(m, BC_S, f[CM1G_THA]);
-  if (m->c.imoist == 1)
-    for (int n = 0; n < 3; n++) bc_fill(m, BC_S, f[CM1G_QA0 + n]);
-  for (int n = 0; n < m->c.npt; n++) bc_fill(m, BC_S, f[CM1G_PTA0 + n]);
+  {
+    BcItem it[BC_MAX] = {{f[CM1G_UA], BC_U}, {f[CM1G_VA], BC_V}, {f[CM1G_WA], BC_W1}, {f[CM1G_PPI], BC_S},
+                         {f[CM1G_THA], BC_S}};
+    int nb = 5;
+    if (m->c.imoist == 1)
+      for (int n = 0; n < 3; n++) it[nb++] = BcItem{f[CM1G_QA0 + n], BC_S};
+    for (int n = 0; n < m->c.npt; n++) it[nb++] = BcItem{f[CM1G_PTA0 + n], BC_S};
+    bc_fill_list(m, it, nb);
+  }
   const size_t bytes = m->ntot * sizeof(float);
   HIPCHK(hipMemcpyAsync(f[CM1G_U3D], f[CM1G_UA], bytes, hipMemcpyDeviceToDevice, m->stream));
   HIPCHK(hipMemcpyAsync(f[CM1G_V3D], f[CM1G_VA], bytes, hipMemcpyDeviceToDevice, m->stream));
@@ -1162,7 +1203,7 @@ extern "C" int cm1g_solve2(cm1g_model *m) {
       int c = IXD(P, i, j, k);
       sadv[c] = P.pi0[k] + pp_r[c];
       if (i < 1 || i > ni || j < 1 || j > nj) return;
-      float th = th_r[c];
+      float th = th_r[c], thv;
       if (moist) {
         float ql = qc_r[c];
         ql = ql + qr_r[c];
@@ -1170,18 +1211,19 @@ extern "C" int cm1g_solve2(cm1g_model *m) {
         float qli = fmaxf(0.0f, ql + 0.0f);
         float cpli = K.cpl * fmaxf(0.0f, ql) + K.cpi * fmaxf(0.0f, 0.0f);
         dum8[c] = K.g * (th * P.rth0[k] + K.repsm1 * (qvv - P.qv0[k]) - (qli - P.qc0[k] - P.qi0[k]));
-        t11[c] = (P.th0[k] + th) * (1.0f + K.reps * qvv) / (1.0f + qvv + qli);
+        thv = (P.th0[k] + th) * (1.0f + K.reps * qvv) / (1.0f + qvv + qli);
         float cpm = K.cp + K.cpv * qvv + cpli;
         float cvm = 1.0f / (K.cv + K.cvv * qvv + cpli);
         thterm[c] = (P.th0[k] + th) * (K.rd + K.rv * qvv - K.rovcp * cpm) * cvm;
         t22[c] = (P.pi0[k] + pp_r[c]) * K.rovcp * cpm * cvm;
       } else {
         dum8[c] = K.g * th * P.rth0[k];
-        t11[c] = P.th0[k] + th;
+        thv = P.th0[k] + th;
         t22[c] = (P.pi0[k] + pp_r[c]) * K.rddcv;
       }
+      t11[c] = thv;
+      put_p_halo(P, t11, i, j, k, thv);
     });
-    bc_fill(m, BC_P, t11);
     // rru, rrv, rrw (src/solve2.F:490-545) and divx (:587-625) in one pass
     {
       ColGrid cg = col_grid_box(0, ni + 2, 0, nj + 2, m->tile_rows);
@@ -1251,23 +1293,31 @@ extern "C" int cm1g_solve2(cm1g_model *m) {
       });
       if (m->c.apmasscon == 1) mass_levels(m, rho, 1);
     }
-    bc_fill(m, BC_U, u3d);
-    bc_fill(m, BC_V, v3d);
-    bc_fill(m, BC_W1, w3d);
-    if (nrk < 3) {
-      float *arr[5] = {rho, pp3d, nullptr, nullptr, nullptr};
-      bc_fill_n(m, BC_P, arr, 2);
-      float *sarr[4] = {th3d, f[CM1G_Q3D0], f[CM1G_Q3D1], f[CM1G_Q3D2]};
-      bc_fill_n(m, BC_S, sarr, moist ? 4 : 1);
-    }
     // passive tracers (src/solve2.F:1902-1970)
     for (int n = 0; n < m->c.npt; n++) {
       advs_run(m, nrk, from_a ? f[CM1G_PTA0 + n] : f[CM1G_PT3D0 + n], 0.0f, f[CM1G_PTA0 + n],
                f[CM1G_PTTEN0 + n], nullptr, nullptr, f[CM1G_PT3D0 + n],
                (nrk == 3 && m->c.pdtra == 1) ? 1 : 0, 1, dttmp, (double)(1.0f * P.K.epsilon), 0);
-      if (nrk <= 2) bc_fill(m, BC_S, f[CM1G_PT3D0 + n]);
     }
     if (from_a) m->swapped = 0;
+    // the halos of everything the stage advanced, in one launch
+    {
+      BcItem it[BC_MAX];
+      int n = 0;
+      it[n++] = BcItem{u3d, BC_U};
+      it[n++] = BcItem{v3d, BC_V};
+      it[n++] = BcItem{w3d, BC_W1};
+      if (m->turb.cm1setup == 1) it[n++] = BcItem{f[CM1G_TKE3D], BC_W1};
+      if (nrk < 3) {
+        it[n++] = BcItem{rho, BC_P};
+        it[n++] = BcItem{pp3d, BC_P};
+        it[n++] = BcItem{f[CM1G_TH3D], BC_S};
+        if (moist)
+          for (int q = 0; q < 3; q++) it[n++] = BcItem{f[CM1G_Q3D0 + q], BC_S};
+        for (int t = 0; t < m->c.npt; t++) it[n++] = BcItem{f[CM1G_PT3D0 + t], BC_S};
+      }
+      bc_fill_list(m, it, n);
+    }
     // finish the dry-mass adjustment (src/solve2.F:1973-2030)
     if (nrk == 3 && m->c.apmasscon == 1) {
       const double *dscal = m->dscal;
@@ -1287,10 +1337,9 @@ extern "C" int cm1g_solve2(cm1g_model *m) {
       });
     }
   }
-  for (int n = 0; n < m->c.npt; n++) {
+  for (int n = 0; n < m->c.npt; n++)
     if (m->c.pdtra == 1) pdefq_run(m, 0.0f, rho, f[CM1G_PT3D0 + n]);
-    bc_fill(m, BC_S, f[CM1G_PT3D0 + n]);
-  }
+  if (m->c.npt > 0) bc_fill_n(m, BC_S, &f[CM1G_PT3D0], m->c.npt);
   m->synced = 0;
   return check_launch();
 }
@@ -1321,13 +1370,12 @@ extern "C" int cm1g_solve3(cm1g_model *m) {
   const int moist = m->c.imoist;
   float *pp3d = f[CM1G_PP3D], *th3d = f[CM1G_TH3D], *ppx = f[CM1G_PPX], *rho = f[CM1G_RHO];
   float *rr = f[CM1G_RR], *rf = f[CM1G_RF];
-  bc_fill(m, BC_P, pp3d);
+  // rho's halo too: rf below reads it (ppx's follows with its update)
   {
-    float *sarr[4] = {th3d, f[CM1G_Q3D0], f[CM1G_Q3D1], f[CM1G_Q3D2]};
-    bc_fill_n(m, BC_S, sarr, moist ? 4 : 1);
+    BcItem it[6] = {{pp3d, BC_P}, {rho, BC_P}, {th3d, BC_S}, {f[CM1G_Q3D0], BC_S}, {f[CM1G_Q3D1], BC_S},
+                    {f[CM1G_Q3D2], BC_S}};
+    bc_fill_list(m, it, moist ? 6 : 3);
   }
-  // rho's halo first (rf below reads it); ppx's halo after the update
-  bc_fill(m, BC_P, rho);
   {
     // one pass over the step's final copies (src/solve3.F:246-705):
     // ppx = pp3d + ppx and the diabatic tendencies on the interior,
@@ -1375,7 +1423,9 @@ extern "C" int cm1g_solve3(cm1g_model *m) {
                                    P.cgt3 * rho[IXD(P, i, j, nk - 2)];
       }
       if (i < 1 || i > ni || j < 1 || j > nj) return;
-      ppx[c] = pp + ppx[c];
+      const float px = pp + ppx[c];
+      ppx[c] = px;
+      put_p_halo(P, ppx, i, j, k, px);
       if (diab) {
         qpten[c] = (pp - qpten[c]) * rdt;
         qtten[c] = (th - qtten[c]) * rdt;
@@ -1384,7 +1434,6 @@ extern "C" int cm1g_solve3(cm1g_model *m) {
       }
     });
   }
-  bc_fill(m, BC_P, ppx);
   if (m->ext_writers) {
     for (int n = 0; n < m->c.npt; n++) {
       float *pta = f[CM1G_PTA0 + n];

@@ -988,7 +988,7 @@ void tke_stage(cm1g_model *m, int nrk, float dttmp) {
     if (t < 1.0e-10f) t = 0.0f;
     tke3d[c] = t;
   });
-  bc_fill(m, BC_W1, tke3d);
+  // (solve2 fills tke3d's halo with the stage's other arrays)
 }
 
 void tke_copy(cm1g_model *m) {
