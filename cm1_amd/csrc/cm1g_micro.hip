@@ -265,6 +265,7 @@ static void surrogate_kessler_satadj(cm1g_model *m) {
   const float *zh = m->kf[CM1G_K_ZH];
   const float rztop = 1.0f / m->hk[CM1G_K_ZF][nk + 1];
   const float *prm = mlp_params(m->sur), *nm = mlp_norm(m->sur);
+  const MlpPack *pk = mlp_packed(m->sur);
   for2(m, 1, ni, 1, nj, [=] __device__(int i, int j) {
     colflag[(i - 1) + (j - 1) * ni] = 0;
     if (i == 1 && j == 1) {
@@ -351,7 +352,7 @@ static void surrogate_kessler_satadj(cm1g_model *m) {
   const int64_t groups = (n + 16 * MLP_G * MLP_WAVES - 1) / (16 * MLP_G * MLP_WAVES);
   const int nbx = (int)(groups < 1024 ? groups : 1024);
   launch<512>(m, dim3(nbx), dim3(512),
-              [=] __device__(int bx, int, int) { mlp_tiles(prm, n, nact, load, prep, out, bx, nbx); });
+              [=] __device__(int bx, int, int) { mlp_tiles(pk, prm, n, nact, load, prep, out, bx, nbx); });
   // apply the projected proposal as kessler applies its own result (the
   // theta, pi', p update after evaporation above 1e-7), or plain kessler in
   // flagged columns; then satadj

@@ -21,6 +21,9 @@ constexpr int NM_XLO = 2 * MLP_IN + 2 * MLP_OUT, NM_XHI = NM_XLO + MLP_IN;
 
 struct cm1g_mlp;
 const float *mlp_params(const cm1g_mlp *n);
+// the BF16 weights in fragment order (MlpPack), kept equal to the parameters
+// by everything that changes them (cm1g_mlp_create, _set_params, _adam)
+const struct MlpPack *mlp_packed(const cm1g_mlp *n);
 const float *mlp_norm(const cm1g_mlp *n);
 
 __device__ __forceinline__ unsigned short bf16_rne(float f) {
@@ -47,11 +50,25 @@ constexpr int MLP_G = 1;              // 16-sample groups per wavefront and roun
 constexpr int MLP_F1 = 8 * 1 * 256;   // layer 1: 8 output tiles x 1 k-step of 16 x 64 lanes x 4
 constexpr int MLP_FH = 8 * 4 * 512;   // hidden layers: 8 x 4 k-steps of 32 x 64 lanes x 8
 constexpr int MLP_F4 = 1 * 4 * 512;   // output layer: 1 (4 of 16 outputs used) x 4
-struct MlpLds {
+// The forward weights, then the backward ones (b2..b4: dX^T = W dY^T, the
+// same order with inputs and outputs exchanged).
+struct MlpFwd {
   bf16x4 w1[MLP_F1 / 4];
   bf16x8s w2[MLP_FH / 8];
   bf16x8s w3[MLP_FH / 8];
   bf16x8s w4[MLP_F4 / 8];
+};
+struct MlpBwd {
+  bf16x8s b2[MLP_FH / 8];
+  bf16x8s b3[MLP_FH / 8];
+  bf16x4 b4[MLP_F1 / 4];
+};
+struct MlpPack {
+  MlpFwd f;
+  MlpBwd b;
+};
+struct MlpLds {
+  MlpFwd f;
   float b[3 * MLP_H + 16];
 };
 
@@ -153,6 +170,26 @@ __device__ __forceinline__ void mlp_hidden(bf16x4 (&x)[MLP_G][8], const bf16x8s 
   mlp_silu_out(acc, x);
 }
 
+// packed weights to LDS in 16-byte pieces, 512 threads
+__device__ __forceinline__ void mlp_stage(void *lds, const void *src, int bytes, int tid) {
+  typedef int i4 __attribute__((ext_vector_type(4)));
+  const i4 *s = (const i4 *)src;
+  i4 *d = (i4 *)lds;
+#pragma unroll 4
+  for (int e = tid; e < bytes / 16; e += 512) d[e] = s[e];
+}
+// the biases, FP32: layers 1 to 3, then the 4 outputs padded to 16
+__device__ __forceinline__ void mlp_stage_bias(float *b, const float *__restrict__ prm, int tid) {
+  for (int e = tid; e < 3 * MLP_H + 16; e += 512) {
+    float v = 0.0f;
+    if (e < MLP_H) v = prm[OB1 + e];
+    else if (e < 2 * MLP_H) v = prm[OB2 + e - MLP_H];
+    else if (e < 3 * MLP_H) v = prm[OB3 + e - 2 * MLP_H];
+    else if (e < 3 * MLP_H + MLP_OUT) v = prm[OB4 + e - 3 * MLP_H];
+    b[e] = v;
+  }
+}
+
 // Run the network over samples 0..n-1.  load(s, r) fills r[MLP_KEEP] with
 // the raw values sample s needs (loads only), prep(s, r, x) turns them into
 // the 8 normalised inputs, out(s, y, r) takes the 4 normalised outputs.
@@ -166,7 +203,8 @@ constexpr int MLP_KEEP = 8;
 // n_dev, if not null, holds a count (in device memory, written by an
 // earlier launch) that caps n: the samples are then 0..min(n, *n_dev)-1.
 template <class LOAD, class PREP, class OUT>
-__device__ void mlp_tiles(const float *__restrict__ prm, int64_t n, const unsigned long long *n_dev,
+__device__ void mlp_tiles(const MlpPack *__restrict__ pk, const float *__restrict__ prm, int64_t n,
+                          const unsigned long long *n_dev,
                           const LOAD &load, const PREP &prep, const OUT &out, int bx, int nbx) {
   __shared__ MlpLds S;
   if (n_dev) {
@@ -174,29 +212,8 @@ __device__ void mlp_tiles(const float *__restrict__ prm, int64_t n, const unsign
     n = nd < n ? nd : n;
   }
   const int tid = (int)threadIdx.x, l = tid & 63, w = tid >> 6;
-  unsigned short *w1 = (unsigned short *)S.w1, *w2 = (unsigned short *)S.w2, *w3 = (unsigned short *)S.w3,
-                 *w4 = (unsigned short *)S.w4;
-  for (int e = tid; e < 16 * MLP_H; e += 512) {  // layer 1, inputs padded to 16
-    const int k = e / MLP_H, nn = e % MLP_H;
-    w1[mlp_wfrag(k, nn, 1)] = k < MLP_IN ? bf16_rne(prm[OW1 + k * MLP_H + nn]) : (unsigned short)0;
-  }
-  for (int e = tid; e < MLP_H * MLP_H; e += 512) {
-    const int k = e / MLP_H, nn = e % MLP_H;
-    w2[mlp_wfrag32(k, nn, 4)] = bf16_rne(prm[OW2 + e]);
-    w3[mlp_wfrag32(k, nn, 4)] = bf16_rne(prm[OW3 + e]);
-  }
-  for (int e = tid; e < MLP_H * 16; e += 512) {  // output layer, outputs padded to 16
-    const int k = e / 16, nn = e % 16;
-    w4[mlp_wfrag32(k, nn, 4)] = nn < MLP_OUT ? bf16_rne(prm[OW4 + k * MLP_OUT + nn]) : (unsigned short)0;
-  }
-  for (int e = tid; e < 3 * MLP_H + 16; e += 512) {
-    float v = 0.0f;
-    if (e < MLP_H) v = prm[OB1 + e];
-    else if (e < 2 * MLP_H) v = prm[OB2 + e - MLP_H];
-    else if (e < 3 * MLP_H) v = prm[OB3 + e - 2 * MLP_H];
-    else if (e < 3 * MLP_H + MLP_OUT) v = prm[OB4 + e - 3 * MLP_H];
-    S.b[e] = v;
-  }
+  mlp_stage(&S.f, &pk->f, (int)sizeof(MlpFwd), tid);
+  mlp_stage_bias(S.b, prm, tid);
   __syncthreads();
   constexpr int PER = 16 * MLP_G;  // samples per wavefront and round
   const int64_t stride = (int64_t)nbx * MLP_WAVES * PER;
@@ -226,9 +243,9 @@ __device__ void mlp_tiles(const float *__restrict__ prm, int64_t n, const unsign
     }
     float rn[MLP_G][MLP_KEEP];
     fetch(base + stride, rn);
-    mlp_first(x, S.w1, S.b, l);
-    mlp_hidden(x, S.w2, S.b + MLP_H, l);
-    mlp_hidden(x, S.w3, S.b + 2 * MLP_H, l);
+    mlp_first(x, S.f.w1, S.b, l);
+    mlp_hidden(x, S.f.w2, S.b + MLP_H, l);
+    mlp_hidden(x, S.f.w3, S.b + 2 * MLP_H, l);
     // output layer: one tile of 16 outputs (4 used); lane l < 16 ends up
     // with outputs 0..3 of its sample
     floatx4 acc[MLP_G];
@@ -236,7 +253,7 @@ __device__ void mlp_tiles(const float *__restrict__ prm, int64_t n, const unsign
     for (int g = 0; g < MLP_G; g++) acc[g] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int kb = 0; kb < 4; kb++) {
-      const bf16x8 wv = __builtin_bit_cast(bf16x8, S.w4[kb * 64 + l]);
+      const bf16x8 wv = __builtin_bit_cast(bf16x8, S.f.w4[kb * 64 + l]);
 #pragma unroll
       for (int g = 0; g < MLP_G; g++)
         acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, mlp_join(x[g][2 * kb], x[g][2 * kb + 1]), acc[g],

@@ -3,19 +3,15 @@
 // a learned surrogate for the local part of Kessler microphysics.  No
 // counterpart in the reference.
 //
-// Matrix products use v_mfma_f32_16x16x16_bf16: a wavefront multiplies a
-// 16x16 block of A by a 16x16 block of B into a 16x16 FP32 block, where
-//   lane l holds A(l%16, 4*(l/16) + t) and B(4*(l/16) + t, l%16), t = 0..3,
-//   and receives D(4*(l/16) + t, l%16).
-// Operands are rounded from FP32 to BF16 to nearest, ties to even.
-//
-// Training (forward with saved activations, backward, Adam) runs through one
-// tiled matrix-product kernel (k_gemm: 64x64 output tiles, K in steps of 16
-// staged through LDS, split over K for the weight gradients) and a few
-// element-wise kernels; the loss is the mean squared error of the
+// Operands are rounded from FP32 to BF16 to nearest, ties to even.  Training
+// (cm1g_mlp_loss_grad) is three kernels: k_train runs 16-sample groups
+// forward and backward in registers and writes the operands of the weight
+// gradients, k_wgrad contracts them over the samples, k_grad_final adds the
+// partial sums in a fixed order; the loss is the mean squared error of the
 // normalised outputs.  Inference runs fused (mlp_tiles in cm1g_mlp.h).
 #include "cm1g_mlp.h"
 
+#include <algorithm>
 #include <random>
 
 #define ARGCHK(cond, msg)          \
@@ -31,152 +27,410 @@ struct cm1g_mlp {
   float *dnorm = nullptr;                                          // normalisation (device)
   int64_t adam_t = 0;
   hipStream_t stream = nullptr;
-  // training workspace for `cap` rows
+  MlpPack *pk = nullptr;                                           // BF16 weights in fragment order
+  // training workspace for `cap` rows: the weight gradients' operands, and
+  // the partial sums of k_train's and k_wgrad's workgroups
   int64_t cap = 0;
-  float *z1 = nullptr, *h1 = nullptr, *z2 = nullptr, *h2 = nullptr, *z3 = nullptr, *h3 = nullptr;
-  float *y = nullptr, *dy = nullptr, *da = nullptr, *dz = nullptr, *part = nullptr, *red = nullptr;
+  unsigned short *frag = nullptr;
+  float *part = nullptr, *wpart = nullptr, *keep = nullptr, *red = nullptr;
 };
+const MlpPack *mlp_packed(const cm1g_mlp *n) { return n->pk; }
 
 const float *mlp_params(const cm1g_mlp *n) { return n->p; }
 const float *mlp_norm(const cm1g_mlp *n) { return n->dnorm; }
 
-// ------------------------------------------------------------ k_gemm
-// C(m,n) = sum_k A(m,k) B(k,n) over this split's K range, with
-// A(m,k) = A[m*sam + k*sak], B(k,n) = B[k*sbk + n*sbn]; split s writes
-// C + s*cs.  64x64 output tile per workgroup, four wavefronts of 32x32.
-#define GP 20  // LDS row pitch of the staged tiles (16 + 4, in BF16 elements)
-__global__ void __launch_bounds__(256) k_gemm(int M, int N, int K, int kchunk, const float *__restrict__ A,
-                                              long sam, long sak, const float *__restrict__ B, long sbk,
-                                              long sbn, float *__restrict__ C, long ldc, long cs) {
-  __shared__ unsigned short As[64 * GP];  // [m][k]
-  __shared__ unsigned short Bs[64 * GP];  // [n][k]
-  const int tid = (int)threadIdx.x, l = tid & 63, w = tid >> 6;
-  const int wm = w & 1, wn = w >> 1;
-  const int m0 = (int)blockIdx.x * 64, n0 = (int)blockIdx.y * 64, s = (int)blockIdx.z;
-  const int kb = s * kchunk, ke = min(K, kb + kchunk);
-  const bool akf = (sak == 1), bkf = (sbk == 1);
-  floatx4 acc[2][2];
-  for (int a = 0; a < 2; a++)
-    for (int b = 0; b < 2; b++) acc[a][b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int k0 = kb; k0 < ke; k0 += 16) {
-    for (int q = 0; q < 4; q++) {
-      const int e = tid + 256 * q;  // 0..1023 over the 64 x 16 tile
-      // the fast index follows the unit stride of each operand
-      const int ra = akf ? e / 16 : e % 64, ka = akf ? e % 16 : e / 64;
-      const int m = m0 + ra, kk = k0 + ka;
-      As[ra * GP + ka] = (m < M && kk < ke) ? bf16_rne(A[(long)m * sam + (long)kk * sak]) : (unsigned short)0;
-      const int cb = bkf ? e / 16 : e % 64, kb2 = bkf ? e % 16 : e / 64;
-      const int n = n0 + cb, kk2 = k0 + kb2;
-      Bs[cb * GP + kb2] = (n < N && kk2 < ke) ? bf16_rne(B[(long)kk2 * sbk + (long)n * sbn]) : (unsigned short)0;
-    }
-    __syncthreads();
-    bf16x4 af[2], bq[2];
-    for (int t = 0; t < 2; t++) {
-      const unsigned short *pa = &As[(32 * wm + 16 * t + (l & 15)) * GP + 4 * (l >> 4)];
-      const unsigned short *pb = &Bs[(32 * wn + 16 * t + (l & 15)) * GP + 4 * (l >> 4)];
-      for (int u = 0; u < 4; u++) {
-        af[t][u] = (short)pa[u];
-        bq[t][u] = (short)pb[u];
-      }
-    }
-    for (int a = 0; a < 2; a++)
-      for (int b = 0; b < 2; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(af[a], bq[b], acc[a][b], 0, 0, 0);
-    __syncthreads();
+// ------------------------------------------------------------ packing
+// the fragment positions of parameter i, BF16 (biases stay FP32 in the
+// parameters themselves)
+__device__ __forceinline__ void mlp_pack_one(MlpPack *pk, int i, float v) {
+  const unsigned short b = bf16_rne(v);
+  if (i < OB1) {
+    const int k = (i - OW1) / MLP_H, n = (i - OW1) % MLP_H;
+    ((unsigned short *)pk->f.w1)[mlp_wfrag(k, n, 1)] = b;
+  } else if (i >= OW2 && i < OB2) {
+    const int k = (i - OW2) / MLP_H, n = (i - OW2) % MLP_H;
+    ((unsigned short *)pk->f.w2)[mlp_wfrag32(k, n, 4)] = b;
+    ((unsigned short *)pk->b.b2)[mlp_wfrag32(n, k, 4)] = b;
+  } else if (i >= OW3 && i < OB3) {
+    const int k = (i - OW3) / MLP_H, n = (i - OW3) % MLP_H;
+    ((unsigned short *)pk->f.w3)[mlp_wfrag32(k, n, 4)] = b;
+    ((unsigned short *)pk->b.b3)[mlp_wfrag32(n, k, 4)] = b;
+  } else if (i >= OW4 && i < OB4) {
+    const int k = (i - OW4) / MLP_OUT, n = (i - OW4) % MLP_OUT;
+    ((unsigned short *)pk->f.w4)[mlp_wfrag32(k, n, 4)] = b;
+    ((unsigned short *)pk->b.b4)[mlp_wfrag(n, k, 1)] = b;
   }
-  for (int a = 0; a < 2; a++)
-    for (int b = 0; b < 2; b++)
-      for (int t = 0; t < 4; t++) {
-        const int m = m0 + 32 * wm + 16 * a + 4 * (l >> 4) + t, n = n0 + 32 * wn + 16 * b + (l & 15);
-        if (m < M && n < N) C[(long)s * cs + (long)m * ldc + n] = acc[a][b][t];
-      }
 }
-
-// C(m,n) = sum over splits of the partial products, in split order
-__global__ void __launch_bounds__(256) k_sum_splits(int M, int N, long ldc, int splits, long cs,
-                                                    const float *__restrict__ part, float *__restrict__ C) {
+// (the padding of the first and last layers stays the zero it was allocated
+// with)
+__global__ void __launch_bounds__(256) k_pack(const float *__restrict__ p, MlpPack *__restrict__ pk) {
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (i >= M * N) return;
-  float s = 0.0f;
-  for (int q = 0; q < splits; q++) s += part[(long)q * cs + i];
-  C[(long)(i / N) * ldc + (i % N)] = s;
+  if (i < MLP_NPARAM) mlp_pack_one(pk, i, p[i]);
 }
 
-static void gemm(hipStream_t st, int M, int N, int K, const float *A, long sam, long sak, const float *B,
-                 long sbk, long sbn, float *C, long ldc, float *part, int splits) {
-  if (splits <= 1 || K <= 1024) {
-    hipLaunchKernelGGL(k_gemm, dim3((M + 63) / 64, (N + 63) / 64, 1), dim3(256), 0, st, M, N, K, K, A, sam,
-                       sak, B, sbk, sbn, C, ldc, 0L);
-    return;
+// ------------------------------------------------------------ training
+// The weight gradients' operands of one 16-sample group: tiles of 16
+// features x 16 samples in BF16, lane l of a tile holding feature l%16,
+// samples 4(l/16)..+3 (what the matrix instructions take with the samples as
+// the summed index).
+constexpr int T_X = 0, T_H1 = 1, T_H2 = 9, T_H3 = 17, T_D1 = 25, T_D2 = 33, T_D3 = 41, T_DY = 49, T_N = 50;
+constexpr int T_ELEM = 256;
+constexpr int TP_N = 392;  // one workgroup's partial sums: 3 x 128 + 4 bias gradients, the loss
+constexpr int TP_LOSS = 3 * MLP_H + MLP_OUT;
+
+// (the caller's rows may start on any float)
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+
+struct TrainLds {
+  MlpPack w;
+  float b[3 * MLP_H + 16];
+  unsigned short tr[MLP_WAVES][64][16];  // a wavefront's transposes: 64 features x 16 samples
+};
+static_assert(sizeof(TrainLds) <= 160 * 1024, "k_train: LDS");
+
+// tiles nt0..nt0+n-1 (n <= 4) of a lane's values, sample l%16 and outputs
+// 16nt + 4(l/16) + t, to the layout above
+template <int N>
+__device__ __forceinline__ void put_tiles(unsigned short (*tr)[16], const bf16x4 *x, unsigned short *dst, int l) {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int q = 0; q < N; q++)
+#pragma unroll
+    for (int t = 0; t < 4; t++) tr[16 * q + 4 * (l >> 4) + t][l & 15] = (unsigned short)x[q][t];
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int q = 0; q < N; q++) {
+    const bf16x4 v = *(const bf16x4 *)&tr[16 * q + (l & 15)][4 * (l >> 4)];
+    *(bf16x4 *)(dst + q * T_ELEM + 4 * l) = v;
   }
-  int kchunk = (K + splits - 1) / splits;
-  kchunk = (kchunk + 15) / 16 * 16;
-  splits = (K + kchunk - 1) / kchunk;
-  const long cs = (long)M * N;
-  hipLaunchKernelGGL(k_gemm, dim3((M + 63) / 64, (N + 63) / 64, splits), dim3(256), 0, st, M, N, K, kchunk, A,
-                     sam, sak, B, sbk, sbn, part, (long)N, cs);
-  hipLaunchKernelGGL(k_sum_splits, dim3((M * N + 255) / 256), dim3(256), 0, st, M, N, ldc, splits, cs, part, C);
 }
 
-// ------------------------------------------------------------ element-wise
-// Z += bias (per column); H = SiLU(Z) if H is given
-__global__ void __launch_bounds__(256) k_bias_act(float *__restrict__ Z, int64_t rows, int width,
-                                                  const float *__restrict__ bias, float *__restrict__ H) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= rows * width) return;
-  const float z = Z[i] + bias[i % width];
-  Z[i] = z;
-  if (H) H[i] = silu_f(z);
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
 }
-
-// dZ = dH * SiLU'(Z)
-__global__ void __launch_bounds__(256) k_silu_back(const float *__restrict__ dH, const float *__restrict__ Z,
-                                                   int64_t count, float *__restrict__ dZ) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= count) return;
-  const float z = Z[i];
-  const float sg = 1.0f / (1.0f + expf(-z));
-  dZ[i] = dH[i] * (sg * (1.0f + z * (1.0f - sg)));
-}
-
-// dY = 2 (Y - T) / (rows * 4); per-block partial sums of (Y - T)^2
-__global__ void __launch_bounds__(256) k_mse(const float *__restrict__ Y, const float *__restrict__ T,
-                                             int64_t count, float *__restrict__ dY, float *__restrict__ part) {
-  __shared__ float r[256];
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  float e2 = 0.0f;
-  if (i < count) {
-    const float d = Y[i] - T[i];
-    dY[i] = 2.0f * d / (float)count;
-    e2 = d * d;
+// Sums over the 16 samples (lanes l%16) of a lane's 32 values: each step
+// hands half of the values to a partner lane and keeps the other half, so
+// lane s ends with values 2s', 2s'+1, s' = s; order fixed.
+__device__ __forceinline__ void sum16(const floatx4 (&z)[8], float &r0, float &r1, int l) {
+  const bool b3 = l & 8, b2 = l & 4, b1 = l & 2, b0 = l & 1;
+  float v[32];
+#pragma unroll
+  for (int q = 0; q < 32; q++) v[q] = z[q >> 2][q & 3];
+#pragma unroll
+  for (int q = 0; q < 16; q++) {
+    const float keep = b3 ? v[q + 16] : v[q], send = b3 ? v[q] : v[q + 16];
+    v[q] = keep + dpp<0x128>(send);  // row_ror:8
   }
-  e2 = block_reduce256(e2, r, OpAdd());
-  if (threadIdx.x == 0) part[blockIdx.x] = e2;
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    const float keep = b2 ? v[q + 8] : v[q], send = b2 ? v[q] : v[q + 8];
+    v[q] = keep + dpp<0x141>(send);  // row_half_mirror
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const float keep = b1 ? v[q + 4] : v[q], send = b1 ? v[q] : v[q + 4];
+    v[q] = keep + dpp<0x4E>(send);  // quad_perm [2,3,0,1]
+  }
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    const float keep = b0 ? v[q + 2] : v[q], send = b0 ? v[q] : v[q + 2];
+    v[q] = keep + dpp<0xB1>(send);  // quad_perm [1,0,3,2]
+  }
+  r0 += v[0];
+  r1 += v[1];
+  __builtin_amdgcn_sched_barrier(0);
 }
 
-// out[0] = sum(part[0..n)) / count, in a fixed order
-__global__ void __launch_bounds__(256) k_loss_final(const float *__restrict__ part, int n, int64_t count,
-                                                    float *__restrict__ out) {
-  __shared__ double r[256];
-  double s = 0.0;
-  for (int i = (int)threadIdx.x; i < n; i += 256) s += (double)part[i];
-  s = block_reduce256(s, r, OpAdd());
-  if (threadIdx.x == 0) out[0] = (float)(s / (double)count);
+// acc (pre-activations) -> x = SiLU in BF16, d = SiLU'.  The derivative uses
+// the sigmoid the activation was formed with.
+__device__ __forceinline__ void silu_both(const floatx4 (&acc)[1][8], bf16x4 (&x)[1][8], floatx4 (&d)[8]) {
+#pragma unroll
+  for (int nt = 0; nt < 8; nt++) {
+    floatx4 h;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const float z = acc[0][nt][t];
+      const float sg = __builtin_amdgcn_rcpf(1.0f + __expf(-z));
+      h[t] = z * sg;
+      d[nt][t] = sg * (1.0f + z * (1.0f - sg));
+    }
+    x[0][nt] = mlp_pack(h[0], h[1], h[2], h[3]);
+    if (nt & 1) __builtin_amdgcn_sched_barrier(0);
+  }
+}
+// acc += W x, 128 x 128 in four 32-deep steps (one step's weight fragments at
+// a time: two would not leave the registers to hold the derivatives)
+__device__ __forceinline__ void mlp_prod(floatx4 (&acc)[1][8], const bf16x4 (&x)[1][8], const bf16x8s *wf, int l) {
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int kb = 0; kb < 4; kb++) {
+    const bf16x8 xb = mlp_join(x[0][2 * kb], x[0][2 * kb + 1]);
+#pragma unroll
+    for (int nt = 0; nt < 8; nt++)
+      acc[0][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[(nt * 4 + kb) * 64 + l]), xb,
+                                                            acc[0][nt], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
 }
 
-// out[c] = sum over rows of D[r*width + c]: one workgroup per column
-__global__ void __launch_bounds__(256) k_colsum(const float *__restrict__ D, int64_t rows, int width,
-                                                float *__restrict__ out) {
-  __shared__ float r[256];
-  const int c = (int)blockIdx.x;
+// Forward and backward of 16-sample groups, one group per wavefront at a
+// time, activations, derivatives and gradients in registers throughout: each
+// layer is computed transposed (mlp_tiles has the argument), and so is its
+// backward product dX^T = W dY^T, whose second operand is again what the lane
+// holds.  The operands of the weight gradients (the layers' inputs and
+// pre-activation gradients, BF16) leave through a small LDS transpose, 25.6 KB
+// a group; bias gradients are summed from the FP32 gradients.  Bound by the
+// vector unit (exponential and reciprocal per hidden value) and by those
+// stores: 40 us for 65536 rows, k_wgrad 32, k_grad_final 7; the separate
+// products and element-wise passes they replace (FP32 activations through
+// memory, column sums by one workgroup each) took 1390 us.
+__global__ void __launch_bounds__(512) k_train(const MlpPack *__restrict__ pk, const float *__restrict__ prm,
+                                               const float *__restrict__ X, const float *__restrict__ T,
+                                               int64_t rows, int64_t ngroups, unsigned short *__restrict__ frag,
+                                               float *__restrict__ part, float *keep) {
+  __shared__ TrainLds S;
+  const int tid = (int)threadIdx.x, l0 = tid & 63, w = tid >> 6;
+  mlp_stage(&S.w, pk, (int)sizeof(MlpPack), tid);
+  mlp_stage_bias(S.b, prm, tid);
+  __syncthreads();
+  const int64_t count = rows * MLP_OUT;
+  float lsum = 0.0f, bs[3][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}, {0.0f, 0.0f}};
+  floatx4 b4 = {0.0f, 0.0f, 0.0f, 0.0f};
+  const floatx4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int64_t g = (int64_t)blockIdx.x * MLP_WAVES + w; g < ngroups; g += (int64_t)gridDim.x * MLP_WAVES) {
+    // opaque, so that the biases and weight fragments are read from LDS where
+    // they are used and not kept in registers over the loop
+    int l = l0;
+    asm volatile("" : "+v"(l));
+    const int64_t s = 16 * g + (l & 15);
+    unsigned short *fg = frag + g * (T_N * T_ELEM);
+    unsigned short(*tr)[16] = S.tr[w];
+    // the first layer's derivatives wait in memory (L2): three layers' would
+    // not fit the registers, and the compiler's own spills wait one by one
+    float *dk = keep + ((int64_t)blockIdx.x * MLP_WAVES + w) * (MLP_H * 16);
+    bf16x4 x[1][8];
+    floatx4 acc[1][8], d1[8], d2[8], d3[8];
+    {
+      // lanes 0-15 take inputs 0-3, lanes 16-31 inputs 4-7
+      floatx4 v = zero;
+      if (l < 32 && s < rows) v = *(const floatx4u *)(X + s * MLP_IN + 4 * (l >> 4));
+      x[0][0] = mlp_pack(v[0], v[1], v[2], v[3]);
+    }
+    floatx4 tv = zero;
+    if (l < 16 && s < rows) tv = *(const floatx4u *)(T + s * MLP_OUT);
+    put_tiles<1>(tr, &x[0][0], fg + T_X * T_ELEM, l);
+    mlp_bias_init(acc, S.b, l);
+#pragma unroll
+    for (int nt = 0; nt < 8; nt++)
+      acc[0][nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(S.w.f.w1[nt * 64 + l], x[0][0], acc[0][nt], 0, 0, 0);
+    silu_both(acc, x, d1);
+#pragma unroll
+    for (int nt = 0; nt < 8; nt++) *(floatx4 *)(dk + nt * 256 + 4 * l) = d1[nt];
+    put_tiles<4>(tr, &x[0][0], fg + T_H1 * T_ELEM, l);
+    put_tiles<4>(tr, &x[0][4], fg + (T_H1 + 4) * T_ELEM, l);
+    mlp_bias_init(acc, S.b + MLP_H, l);
+    mlp_prod(acc, x, S.w.f.w2, l);
+    silu_both(acc, x, d2);
+    put_tiles<4>(tr, &x[0][0], fg + T_H2 * T_ELEM, l);
+    put_tiles<4>(tr, &x[0][4], fg + (T_H2 + 4) * T_ELEM, l);
+    mlp_bias_init(acc, S.b + 2 * MLP_H, l);
+    mlp_prod(acc, x, S.w.f.w3, l);
+    silu_both(acc, x, d3);
+    put_tiles<4>(tr, &x[0][0], fg + T_H3 * T_ELEM, l);
+    put_tiles<4>(tr, &x[0][4], fg + (T_H3 + 4) * T_ELEM, l);
+    // outputs (lane l < 16: the 4 of its sample), loss, dY
+    floatx4 y = zero;
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++)
+      y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, S.w.f.w4[kb * 64 + l]),
+                                                  mlp_join(x[0][2 * kb], x[0][2 * kb + 1]), y, 0, 0, 0);
+    floatx4 dy = zero;
+    if (l < 16 && s < rows) {
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        const float e = (y[t] + S.b[3 * MLP_H + t]) - tv[t];
+        dy[t] = 2.0f * e / (float)count;
+        lsum += e * e;
+      }
+      b4 += dy;
+    }
+    bf16x4 dyp = mlp_pack(dy[0], dy[1], dy[2], dy[3]);
+    put_tiles<1>(tr, &dyp, fg + T_DY * T_ELEM, l);
+    // layer 3
+#pragma unroll
+    for (int nt = 0; nt < 8; nt++) {
+      const floatx4 a = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(S.w.b.b4[nt * 64 + l], dyp, zero, 0, 0, 0);
+      acc[0][nt] = a * d3[nt];
+      x[0][nt] = mlp_pack(acc[0][nt][0], acc[0][nt][1], acc[0][nt][2], acc[0][nt][3]);
+    }
+    sum16(acc[0], bs[2][0], bs[2][1], l);
+    put_tiles<4>(tr, &x[0][0], fg + T_D3 * T_ELEM, l);
+    put_tiles<4>(tr, &x[0][4], fg + (T_D3 + 4) * T_ELEM, l);
+    // layer 2
+#pragma unroll
+    for (int nt = 0; nt < 8; nt++) acc[0][nt] = zero;
+    mlp_prod(acc, x, S.w.b.b3, l);
+#pragma unroll
+    for (int nt = 0; nt < 8; nt++) {
+      acc[0][nt] = acc[0][nt] * d2[nt];
+      x[0][nt] = mlp_pack(acc[0][nt][0], acc[0][nt][1], acc[0][nt][2], acc[0][nt][3]);
+    }
+    sum16(acc[0], bs[1][0], bs[1][1], l);
+    put_tiles<4>(tr, &x[0][0], fg + T_D2 * T_ELEM, l);
+    put_tiles<4>(tr, &x[0][4], fg + (T_D2 + 4) * T_ELEM, l);
+    // layer 1
+#pragma unroll
+    for (int nt = 0; nt < 8; nt++) {
+      d1[nt] = *(const floatx4 *)(dk + nt * 256 + 4 * l);
+      acc[0][nt] = zero;
+    }
+    mlp_prod(acc, x, S.w.b.b2, l);
+#pragma unroll
+    for (int nt = 0; nt < 8; nt++) {
+      acc[0][nt] = acc[0][nt] * d1[nt];
+      x[0][nt] = mlp_pack(acc[0][nt][0], acc[0][nt][1], acc[0][nt][2], acc[0][nt][3]);
+    }
+    sum16(acc[0], bs[0][0], bs[0][1], l);
+    put_tiles<4>(tr, &x[0][0], fg + T_D1 * T_ELEM, l);
+    put_tiles<4>(tr, &x[0][4], fg + (T_D1 + 4) * T_ELEM, l);
+    if (g == ngroups - 1 && (ngroups & 1))  // k_wgrad takes groups in pairs
+      for (int q = 0; q < T_N; q++) *(bf16x4 *)(fg + (T_N + q) * T_ELEM + 4 * l) = bf16x4{0, 0, 0, 0};
+  }
+  // partial sums: the wavefronts', then the workgroup's
+  const int l = l0;
+  for (int o = 8; o > 0; o >>= 1) {
+    lsum += __shfl_down(lsum, o, 16);
+#pragma unroll
+    for (int t = 0; t < 4; t++) b4[t] += __shfl_down(b4[t], o, 16);
+  }
+  __syncthreads();
+  float *red = (float *)&S.tr[0][0][0];  // 8 x TP_N floats fit the transposes' space
+  static_assert(MLP_WAVES * TP_N * sizeof(float) <= sizeof(S.tr), "k_train: partial sums");
+  const int f = 2 * (l & 15);  // this lane's two values of sum16: 16nt + 4(l/16) + t
+#pragma unroll
+  for (int q = 0; q < 3; q++)
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      const int v = f + e;
+      red[w * TP_N + q * MLP_H + 16 * (v >> 2) + 4 * (l >> 4) + (v & 3)] = bs[q][e];
+    }
+  if (l == 0) {
+    for (int t = 0; t < 4; t++) red[w * TP_N + 3 * MLP_H + t] = b4[t];
+    red[w * TP_N + TP_LOSS] = lsum;
+  }
+  __syncthreads();
+  if (tid <= TP_LOSS) {
+    float s = 0.0f;
+    for (int q = 0; q < MLP_WAVES; q++) s += red[q * TP_N + tid];
+    part[(int64_t)blockIdx.x * TP_N + tid] = s;
+  }
+}
+
+// One weight gradient over a range of pairs of groups: dW(in, out) = sum over
+// samples of a(in) d(out), MA x NB tiles per wavefront, 32 samples a step (the
+// lane's four of either group; the same order of samples in both operands).
+template <int MA, int NB>
+__device__ __forceinline__ void wgrad(const unsigned short *__restrict__ frag, int64_t p0, int64_t p1, int ta, int tb,
+                                      float *out, int ld, int min_, int nout, int l) {
+  floatx4 acc[MA][NB];
+#pragma unroll
+  for (int a = 0; a < MA; a++)
+#pragma unroll
+    for (int b = 0; b < NB; b++) acc[a][b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  // the workspace holds whole pairs, the group after an odd last one zeroed.
+  // The next step's operands load while this one's instructions run.
+  bf16x8 av[MA], bv[NB], an[MA], bn[NB];
+  auto fetch = [&](int64_t p, bf16x8 (&a_)[MA], bf16x8 (&b_)[NB]) {
+    const unsigned short *g0 = frag + 2 * p * (T_N * T_ELEM) + 4 * l, *g1 = g0 + T_N * T_ELEM;
+#pragma unroll
+    for (int a = 0; a < MA; a++)
+      a_[a] = mlp_join(*(const bf16x4 *)(g0 + (ta + a) * T_ELEM), *(const bf16x4 *)(g1 + (ta + a) * T_ELEM));
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+      b_[b] = mlp_join(*(const bf16x4 *)(g0 + (tb + b) * T_ELEM), *(const bf16x4 *)(g1 + (tb + b) * T_ELEM));
+  };
+  if (p0 < p1) fetch(p0, av, bv);
+  for (int64_t p = p0; p < p1; p++) {
+    if (p + 1 < p1) fetch(p + 1, an, bn);
+#pragma unroll
+    for (int a = 0; a < MA; a++)
+#pragma unroll
+      for (int b = 0; b < NB; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[a], bv[b], acc[a][b], 0, 0, 0);
+#pragma unroll
+    for (int a = 0; a < MA; a++) av[a] = an[a];
+#pragma unroll
+    for (int b = 0; b < NB; b++) bv[b] = bn[b];
+  }
+#pragma unroll
+  for (int a = 0; a < MA; a++)
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        const int in = 16 * a + 4 * (l >> 4) + t, o = 16 * b + (l & 15);
+        if (in < min_ && o < nout) out[in * ld + o] = acc[a][b][t];
+      }
+}
+
+// The four weight gradients (blockIdx.y: W3, W2, W1, W4), each split over
+// gridDim.x ranges of samples; bound by reading the 25.6 KB of operands a
+// group (W2 and W3: a 64 x 64 quadrant per wavefront).
+__global__ void __launch_bounds__(256) k_wgrad(const unsigned short *__restrict__ frag, int64_t ngroups,
+                                               float *__restrict__ wpart) {
+  const int l = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
+  const int64_t np = (ngroups + 1) / 2, per = (np + gridDim.x - 1) / gridDim.x;
+  const int64_t p0 = (int64_t)blockIdx.x * per, p1 = p0 + per < np ? p0 + per : np;
+  float *out = wpart + (int64_t)blockIdx.x * MLP_NPARAM;
+  const int m4 = 4 * (w & 1), n4 = 4 * (w >> 1);
+  if (blockIdx.y == 0)
+    wgrad<4, 4>(frag, p0, p1, T_H2 + m4, T_D3 + n4, out + OW3 + 16 * (m4 * MLP_H + n4), MLP_H, MLP_H, MLP_H, l);
+  else if (blockIdx.y == 1)
+    wgrad<4, 4>(frag, p0, p1, T_H1 + m4, T_D2 + n4, out + OW2 + 16 * (m4 * MLP_H + n4), MLP_H, MLP_H, MLP_H, l);
+  else if (blockIdx.y == 2)
+    wgrad<1, 2>(frag, p0, p1, T_X, T_D1 + 2 * w, out + OW1 + 32 * w, MLP_H, MLP_IN, MLP_H, l);
+  else
+    wgrad<2, 1>(frag, p0, p1, T_H3 + 2 * w, T_DY, out + OW4 + 32 * w * MLP_OUT, MLP_OUT, MLP_H, MLP_OUT, l);
+}
+
+// The gradients and the loss: every parameter's partial sums in order (64
+// parameters a workgroup, its four wavefronts a quarter of the partials
+// each).  Workgroup 0 also adds the loss, in double.
+__global__ void __launch_bounds__(256) k_grad_final(const float *__restrict__ wpart, int splits,
+                                                    const float *__restrict__ part, int nwg, int64_t count,
+                                                    float *__restrict__ G, float *__restrict__ loss) {
+  __shared__ float r[4][64];
+  const int l = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
+  const int i = (int)blockIdx.x * 64 + l;
   float s = 0.0f;
-  for (int64_t q = threadIdx.x; q < rows; q += 256) s += D[q * width + c];
-  s = block_reduce256(s, r, OpAdd());
-  if (threadIdx.x == 0) out[c] = s;
+  if (i < MLP_NPARAM) {
+    // a bias's sums come from k_train, a weight's from k_wgrad
+    int col = -1;
+    if (i >= OB1 && i < OW2) col = i - OB1;
+    else if (i >= OB2 && i < OW3) col = MLP_H + i - OB2;
+    else if (i >= OB3 && i < OW4) col = 2 * MLP_H + i - OB3;
+    else if (i >= OB4) col = 3 * MLP_H + i - OB4;
+    const int n = col < 0 ? splits : nwg;
+    const float *src = col < 0 ? wpart + i : part + col;
+    const int64_t ld = col < 0 ? MLP_NPARAM : TP_N;
+    const int per = (n + 3) / 4, q1 = min(n, (w + 1) * per);
+#pragma unroll 8
+    for (int q = w * per; q < q1; q++) s += src[q * ld];
+  }
+  r[w][l] = s;
+  __syncthreads();
+  if (w == 0 && i < MLP_NPARAM) G[i] = ((r[0][l] + r[1][l]) + r[2][l]) + r[3][l];
+  if (blockIdx.x == 0) {
+    __shared__ double d[256];
+    const int q = (int)threadIdx.x;  // nwg <= 256
+    const double t = block_reduce256(q < nwg ? (double)part[(int64_t)q * TP_N + TP_LOSS] : 0.0, d, OpAdd());
+    if (q == 0) loss[0] = (float)(t / (double)count);
+  }
 }
 
 __global__ void __launch_bounds__(256) k_adam(float *__restrict__ p, const float *__restrict__ g,
                                               float *__restrict__ m1, float *__restrict__ m2, int n, float lr,
-                                              float bc1, float bc2) {
+                                              float bc1, float bc2, MlpPack *__restrict__ pk) {
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (i >= n) return;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1.0e-8f;
@@ -185,13 +439,16 @@ __global__ void __launch_bounds__(256) k_adam(float *__restrict__ p, const float
   const float b = b2 * m2[i] + (1.0f - b2) * gi * gi;
   m1[i] = a;
   m2[i] = b;
-  p[i] -= lr * (a / bc1) / (sqrtf(b / bc2) + eps);
+  const float v = p[i] - lr * (a / bc1) / (sqrtf(b / bc2) + eps);
+  p[i] = v;
+  mlp_pack_one(pk, i, v);
 }
 
 // fused inference over a row-major [n x 8] input, [n x 4] output
 template <class LOAD, class PREP, class OUT>
-__global__ void __launch_bounds__(512) k_mlp(const float *prm, int64_t n, LOAD load, PREP prep, OUT out) {
-  mlp_tiles(prm, n, nullptr, load, prep, out, (int)blockIdx.x, (int)gridDim.x);
+__global__ void __launch_bounds__(512) k_mlp(const MlpPack *pk, const float *prm, int64_t n, LOAD load, PREP prep,
+                                             OUT out) {
+  mlp_tiles(pk, prm, n, nullptr, load, prep, out, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // ------------------------------------------------------------ C ABI
@@ -206,12 +463,19 @@ extern "C" int cm1g_mlp_nparams(int64_t *n) {
 extern "C" int cm1g_mlp_destroy(cm1g_mlp *n) {
   if (!n) return 0;
   if (n->stream) hipStreamSynchronize(n->stream);
-  float *bufs[] = {n->p, n->g, n->m1, n->m2, n->dnorm, n->z1, n->h1, n->z2, n->h2, n->z3, n->h3,
-                   n->y, n->dy, n->da, n->dz, n->part, n->red};
-  for (float *b : bufs)
+  void *bufs[] = {n->p, n->g, n->m1, n->m2, n->dnorm, n->pk, n->frag, n->part, n->wpart, n->keep, n->red};
+  for (void *b : bufs)
     if (b) hipFree(b);
   if (n->stream) hipStreamDestroy(n->stream);
   delete n;
+  return 0;
+}
+
+// the packed weights of the parameters as they are on the device
+static int pack_params(cm1g_mlp *n) {
+  hipLaunchKernelGGL(k_pack, dim3(nb256(MLP_NPARAM)), dim3(256), 0, n->stream, n->p, n->pk);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(n->stream));
   return 0;
 }
 
@@ -224,6 +488,8 @@ extern "C" int cm1g_mlp_create(uint64_t seed, cm1g_mlp **out) {
   ok = ok && hipMalloc((void **)&n->m1, MLP_NPARAM * sizeof(float)) == hipSuccess;
   ok = ok && hipMalloc((void **)&n->m2, MLP_NPARAM * sizeof(float)) == hipSuccess;
   ok = ok && hipMalloc((void **)&n->dnorm, MLP_NNORM * sizeof(float)) == hipSuccess;
+  ok = ok && hipMalloc((void **)&n->pk, sizeof(MlpPack)) == hipSuccess;
+  ok = ok && hipMemset(n->pk, 0, sizeof(MlpPack)) == hipSuccess;
   if (!ok) {
     cm1g_mlp_destroy(n);
     cm1g_set_error("cm1g_mlp_create: allocation failed");
@@ -254,6 +520,7 @@ extern "C" int cm1g_mlp_create(uint64_t seed, cm1g_mlp **out) {
        hipMemcpy(n->m2, z.data(), MLP_NPARAM * sizeof(float), hipMemcpyHostToDevice) == hipSuccess &&
        hipMemcpy(n->g, z.data(), MLP_NPARAM * sizeof(float), hipMemcpyHostToDevice) == hipSuccess &&
        hipMemcpy(n->dnorm, nm.data(), MLP_NNORM * sizeof(float), hipMemcpyHostToDevice) == hipSuccess;
+  ok = ok && pack_params(n) == 0;
   if (!ok) {
     cm1g_mlp_destroy(n);
     cm1g_set_error("cm1g_mlp_create: upload failed");
@@ -274,7 +541,7 @@ extern "C" int cm1g_mlp_set_params(cm1g_mlp *n, const float *host) {
   ARGCHK(n && host, "cm1g_mlp_set_params: null argument");
   HIPCHK(hipStreamSynchronize(n->stream));
   HIPCHK(hipMemcpy(n->p, host, MLP_NPARAM * sizeof(float), hipMemcpyHostToDevice));
-  return 0;
+  return pack_params(n);
 }
 
 extern "C" int cm1g_mlp_set_norm(cm1g_mlp *n, const float *norm) {
@@ -304,74 +571,50 @@ extern "C" int cm1g_mlp_forward(cm1g_mlp *n, const float *x, int64_t rows, float
   const int64_t groups = (rows + 16 * MLP_G * MLP_WAVES - 1) / (16 * MLP_G * MLP_WAVES);
   const int nbx = (int)(groups < 1024 ? groups : 1024);
   hipLaunchKernelGGL((k_mlp<decltype(load), decltype(prep), decltype(out)>), dim3(nbx), dim3(512), 0, n->stream,
-                     n->p, rows, load, prep, out);
+                     n->pk, n->p, rows, load, prep, out);
   HIPCHK(hipGetLastError());
   return 0;
 }
 
+// k_train's workgroups (one per CU: the weights of both directions fill its
+// LDS) and k_wgrad's ranges of samples
+constexpr int TRAIN_WGS = 256, WGRAD_SPLITS = 64;
+
 static int ensure_workspace(cm1g_mlp *n, int64_t rows) {
+  struct {
+    float **p;
+    size_t n;
+  } fixed[] = {{&n->part, (size_t)TRAIN_WGS * TP_N},
+               {&n->wpart, (size_t)WGRAD_SPLITS * MLP_NPARAM},
+               {&n->keep, (size_t)TRAIN_WGS * MLP_WAVES * MLP_H * 16},
+               {&n->red, 1}};
+  for (auto &f : fixed)
+    if (!*f.p) HIPCHK(hipMalloc((void **)f.p, f.n * sizeof(float)));
   if (rows <= n->cap) return 0;
   HIPCHK(hipStreamSynchronize(n->stream));
-  float **bufs[] = {&n->z1, &n->h1, &n->z2, &n->h2, &n->z3, &n->h3, &n->da, &n->dz};
-  for (float **b : bufs) {
-    if (*b) hipFree(*b);
-    *b = nullptr;
-    HIPCHK(hipMalloc((void **)b, (size_t)rows * MLP_H * sizeof(float)));
-  }
-  for (float **b : {&n->y, &n->dy}) {
-    if (*b) hipFree(*b);
-    *b = nullptr;
-    HIPCHK(hipMalloc((void **)b, (size_t)rows * MLP_OUT * sizeof(float)));
-  }
-  if (n->part) hipFree(n->part);
-  if (n->red) hipFree(n->red);
-  n->part = n->red = nullptr;
-  HIPCHK(hipMalloc((void **)&n->part, (size_t)64 * MLP_H * MLP_H * sizeof(float)));
-  HIPCHK(hipMalloc((void **)&n->red, (size_t)(nb256(rows * MLP_OUT) + 1) * sizeof(float)));
+  if (n->frag) hipFree(n->frag);
+  n->frag = nullptr;
+  n->cap = 0;
+  const size_t groups = (size_t)((rows + 31) / 32) * 2;  // whole pairs
+  HIPCHK(hipMalloc((void **)&n->frag, groups * T_N * T_ELEM * sizeof(unsigned short)));
   n->cap = rows;
   return 0;
 }
 
-// forward with saved activations, MSE loss, backward into n->g
+// loss and gradients (into n->g) of one batch
 extern "C" int cm1g_mlp_loss_grad(cm1g_mlp *n, const float *x, const float *t, int64_t rows, float *loss,
                                   float *grad) {
   ARGCHK(n && x && t && rows >= 1 && rows <= (1 << 24), "cm1g_mlp_loss_grad: bad argument");
   int rc = ensure_workspace(n, rows);
   if (rc) return rc;
   hipStream_t st = n->stream;
-  const float *P = n->p;
-  float *G = n->g;
-  const int R = (int)rows, H = MLP_H;
-  const int splits = 64;
-  const unsigned eh = nb256(rows * H);
-  // forward
-  gemm(st, R, H, MLP_IN, x, MLP_IN, 1, P + OW1, H, 1, n->z1, H, n->part, 1);
-  hipLaunchKernelGGL(k_bias_act, dim3(eh), dim3(256), 0, st, n->z1, rows, H, P + OB1, n->h1);
-  gemm(st, R, H, H, n->h1, H, 1, P + OW2, H, 1, n->z2, H, n->part, 1);
-  hipLaunchKernelGGL(k_bias_act, dim3(eh), dim3(256), 0, st, n->z2, rows, H, P + OB2, n->h2);
-  gemm(st, R, H, H, n->h2, H, 1, P + OW3, H, 1, n->z3, H, n->part, 1);
-  hipLaunchKernelGGL(k_bias_act, dim3(eh), dim3(256), 0, st, n->z3, rows, H, P + OB3, n->h3);
-  gemm(st, R, MLP_OUT, H, n->h3, H, 1, P + OW4, MLP_OUT, 1, n->y, MLP_OUT, n->part, 1);
-  hipLaunchKernelGGL(k_bias_act, dim3(nb256(rows * MLP_OUT)), dim3(256), 0, st, n->y, rows, MLP_OUT, P + OB4,
-                     (float *)nullptr);
-  const unsigned nbl = nb256(rows * MLP_OUT);
-  hipLaunchKernelGGL(k_mse, dim3(nbl), dim3(256), 0, st, n->y, t, rows * MLP_OUT, n->dy, n->red + 1);
-  hipLaunchKernelGGL(k_loss_final, dim3(1), dim3(256), 0, st, n->red + 1, (int)nbl, rows * MLP_OUT, n->red);
-  // backward
-  gemm(st, H, MLP_OUT, R, n->h3, 1, H, n->dy, MLP_OUT, 1, G + OW4, MLP_OUT, n->part, splits);
-  hipLaunchKernelGGL(k_colsum, dim3(MLP_OUT), dim3(256), 0, st, n->dy, rows, MLP_OUT, G + OB4);
-  gemm(st, R, H, MLP_OUT, n->dy, MLP_OUT, 1, P + OW4, 1, MLP_OUT, n->da, H, n->part, 1);
-  hipLaunchKernelGGL(k_silu_back, dim3(eh), dim3(256), 0, st, n->da, n->z3, rows * H, n->dz);
-  gemm(st, H, H, R, n->h2, 1, H, n->dz, H, 1, G + OW3, H, n->part, splits);
-  hipLaunchKernelGGL(k_colsum, dim3(H), dim3(256), 0, st, n->dz, rows, H, G + OB3);
-  gemm(st, R, H, H, n->dz, H, 1, P + OW3, 1, H, n->da, H, n->part, 1);
-  hipLaunchKernelGGL(k_silu_back, dim3(eh), dim3(256), 0, st, n->da, n->z2, rows * H, n->dz);
-  gemm(st, H, H, R, n->h1, 1, H, n->dz, H, 1, G + OW2, H, n->part, splits);
-  hipLaunchKernelGGL(k_colsum, dim3(H), dim3(256), 0, st, n->dz, rows, H, G + OB2);
-  gemm(st, R, H, H, n->dz, H, 1, P + OW2, 1, H, n->da, H, n->part, 1);
-  hipLaunchKernelGGL(k_silu_back, dim3(eh), dim3(256), 0, st, n->da, n->z1, rows * H, n->dz);
-  gemm(st, MLP_IN, H, R, x, 1, MLP_IN, n->dz, H, 1, G + OW1, H, n->part, splits);
-  hipLaunchKernelGGL(k_colsum, dim3(H), dim3(256), 0, st, n->dz, rows, H, G + OB1);
+  const int64_t groups = (rows + 15) / 16, pairs = (groups + 1) / 2;
+  const int nwg = (int)std::min<int64_t>(TRAIN_WGS, (groups + MLP_WAVES - 1) / MLP_WAVES);
+  const int splits = (int)std::min<int64_t>(WGRAD_SPLITS, pairs);
+  hipLaunchKernelGGL(k_train, dim3(nwg), dim3(512), 0, st, n->pk, n->p, x, t, rows, groups, n->frag, n->part, n->keep);
+  hipLaunchKernelGGL(k_wgrad, dim3(splits, 4), dim3(256), 0, st, n->frag, groups, n->wpart);
+  hipLaunchKernelGGL(k_grad_final, dim3((MLP_NPARAM + 63) / 64), dim3(256), 0, st, n->wpart, splits, n->part, nwg,
+                     rows * MLP_OUT, n->g, n->red);
   HIPCHK(hipGetLastError());
   if (loss) {
     HIPCHK(hipMemcpyAsync(loss, n->red, sizeof(float), hipMemcpyDeviceToHost, st));
@@ -379,7 +622,7 @@ extern "C" int cm1g_mlp_loss_grad(cm1g_mlp *n, const float *x, const float *t, i
   }
   if (grad) {
     HIPCHK(hipStreamSynchronize(st));
-    HIPCHK(hipMemcpy(grad, G, MLP_NPARAM * sizeof(float), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(grad, n->g, MLP_NPARAM * sizeof(float), hipMemcpyDeviceToHost));
   }
   return 0;
 }
@@ -389,7 +632,7 @@ extern "C" int cm1g_mlp_adam(cm1g_mlp *n, float lr) {
   n->adam_t++;
   const float bc1 = 1.0f - std::pow(0.9f, (float)n->adam_t), bc2 = 1.0f - std::pow(0.999f, (float)n->adam_t);
   hipLaunchKernelGGL(k_adam, dim3(nb256(MLP_NPARAM)), dim3(256), 0, n->stream, n->p, n->g, n->m1, n->m2,
-                     MLP_NPARAM, lr, bc1, bc2);
+                     MLP_NPARAM, lr, bc1, bc2, n->pk);
   HIPCHK(hipGetLastError());
   return 0;
 }
