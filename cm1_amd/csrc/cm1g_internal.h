@@ -417,8 +417,10 @@ __device__ __forceinline__ bool col_tile_seg(const ColGrid &g, int b, int nk, in
 // A load (store) at a byte offset from an array's (or a level's) base: the
 // base stays in scalar registers, the offset is one 32-bit register that
 // serves every array.
-__device__ __forceinline__ float ldo(const float *p, unsigned o) { return *(const float *)((const char *)p + o); }
-__device__ __forceinline__ void sto(float *p, unsigned o, float v) { *(float *)((char *)p + o) = v; }
+template <class O>
+__device__ __forceinline__ float ldo(const float *p, O o) { return *(const float *)((const char *)p + o); }
+template <class O>
+__device__ __forceinline__ void sto(float *p, O o, float v) { *(float *)((char *)p + o) = v; }
 
 // The one-point halo fill of an interior value (BC_P, src/bc.F:372-520) by
 // the point that owns it: the copies of (i,j) outside the domain, corners
@@ -486,7 +488,7 @@ void advs_run(cm1g_model *m, int nrk, const float *s_in, float sadd, const float
               int pdef, int pdefweno, float dt, double weps, int smeps_flush);
 // acoustic (cm1g_sound.hip)
 void sound_run(cm1g_model *m, int nrk, bool fold1 = false);
-void sounde_run(cm1g_model *m, int nrk);
+void sounde_run(cm1g_model *m, int nrk, bool fold1 = false);
 void getdiv_both(cm1g_model *m, int want_t11, int want_divx = 1, float *div = nullptr);
 void scale_mass_fluxes(cm1g_model *m);
 void cfl_run(cm1g_model *m, float dt, const float *u, const float *v, const float *w);

@@ -1238,7 +1238,7 @@ extern "C" int cm1g_solve2(cm1g_model *m) {
       const float *src3[3] = {u_r, v_r, w_r};
       adv_uvw(m, nrk, 7, 1, 1, 1, from_a ? src3 : nullptr);
     }
-    if (m->c.psolver == 2) sounde_run(m, nrk);
+    if (m->c.psolver == 2) sounde_run(m, nrk, nrk == 1 && (m->synced || m->swapped));
     else sound_run(m, nrk, nrk == 1 && m->synced);
     if (nrk == 3) cfl_run(m, dt, u3d, v3d, w3d);
     if (m->c.irbc == 4 && (P.ibw || P.ibe || P.ibs || P.ibn))

@@ -34,7 +34,7 @@ struct SubArgs {
   float tem1, tem2, temx, temy;   // cp*rdx/2, cp*rdy/2, dts*rdx/2, dts*rdy/2
   int last, opw, ope, ops, opn;
   const float *uX, *vX;           // u, v at the start of the substep
-  float *uY, *vY;                 // u, v after the substep
+  float *uY, *vY, *wY;            // u, v after the substep (wY: explicit substeps)
   const float *ppdX;              // pi' + divergence damping from the previous substep
   float *ppdY;                    // ... written by this substep
   const float *uten, *vten, *wten, *thv, *piadv, *ppterm, *ppten, *dtu0, *dtv0;
@@ -56,7 +56,8 @@ struct SubArgs {
   // order of the substeps.  fold: this substep updates the averages; pair:
   // with the previous substep's values too; init: they start here.
   int fold, pair, init;
-  const float *wRp;               // the wR of the previous substep
+  const float *wring, *wringp;    // w on the averaging ring, this substep's and the previous one's
+  int expl;                       // explicit substeps: w enters its average like u and v
   float *ppx;                     // last substep of the last stage: the damping term
 };
 
@@ -112,9 +113,13 @@ __device__ __forceinline__ void put_v(const SubArgs &a, int c, float v) {
 // w on the ring, where the step does not change it
 __device__ __forceinline__ void put_w_ring(const SubArgs &a, int c) {
   if (!a.fold) return;
+  const float w = a.wring[c];
+  if (a.expl) {
+    a.rrw[c] = avg_uv(a, a.init ? 0.0f : a.rrw[c], w, w);
+    return;
+  }
   float r = a.init ? a.wa[c] * a.beta : a.rrw[c];
-  if (a.pair) r = r + a.wRp[c];
-  const float w = a.wR[c];
+  if (a.pair) r = r + a.wringp[c];
   a.rrw[c] = a.last ? (r + w * a.alph) * a.tavg : r + w;
 }
 
@@ -687,33 +692,20 @@ static int slab_variant(const cm1g_model *m) {
   return nk <= 96 ? 3 : 4;
 }
 
-void sound_run(cm1g_model *m, int nrk, bool fold1) {
-  const KP P = m->P;
-  const int ni = P.ni, nj = P.nj, nk = P.nk;
-  const float dt = m->c.dt, alph = m->c.alph, kdiv = m->c.kdiv;
-  int nloop;
-  float dts;
-  sound_nloop(nrk, m->c.nsound, dt, &nloop, &dts);
-  const float beta = 1.0f - alph;
-  float *dum1 = m->f[CM1G_DUM1];
-  float *ppd = m->f[CM1G_DUM7];
-  float *u3d = m->f[CM1G_U3D], *v3d = m->f[CM1G_V3D], *w3d = m->f[CM1G_W3D];
-  const float *ua = m->f[CM1G_UA], *va = m->f[CM1G_VA], *wa = m->f[CM1G_WA];
-  float *rru = m->f[CM1G_RRU], *rrv = m->f[CM1G_RRV], *rrw = m->f[CM1G_RRW];
-  const float *ppi = m->f[CM1G_PPI];
-  float *pp3d = m->f[CM1G_PP3D], *ppx = m->f[CM1G_PPX];
-
-  SubArgs a;
-  a.dts = dts;
-  a.alph = alph;
-  a.beta = beta;
-  a.asq = alph * alph;
-  a.kdiv = kdiv;
-  a.tavg = 1.0f / (float)nloop;
+// the arguments that do not change over a stage, and its substep count
+static void sub_args(cm1g_model *m, int nrk, SubArgs &a, int *nloop) {
+  const KP &P = m->P;
+  memset(&a, 0, sizeof(a));
+  sound_nloop(nrk, m->c.nsound, m->c.dt, nloop, &a.dts);
+  a.alph = m->c.alph;
+  a.beta = 1.0f - a.alph;
+  a.asq = a.alph * a.alph;
+  a.kdiv = m->c.kdiv;
+  a.tavg = 1.0f / (float)*nloop;
   a.tem1 = P.rdx * P.K.cp * 0.5f;
   a.tem2 = P.rdy * P.K.cp * 0.5f;
-  a.temx = dts * 0.5f * P.rdx;
-  a.temy = dts * 0.5f * P.rdy;
+  a.temx = a.dts * 0.5f * P.rdx;
+  a.temy = a.dts * 0.5f * P.rdy;
   a.opw = (P.wbc == 2 && P.ibw == 1);
   a.ope = (P.ebc == 2 && P.ibe == 1);
   a.ops = (P.sbc == 2 && P.ibs == 1);
@@ -731,14 +723,43 @@ void sound_run(cm1g_model *m, int nrk, bool fold1) {
   a.radbce = m->d2[CM1G_D_RADBCE];
   a.radbcs = m->d2[CM1G_D_RADBCS];
   a.radbcn = m->d2[CM1G_D_RADBCN];
-  a.w3d = w3d;
-  a.pp3d = pp3d;
+  a.w3d = m->f[CM1G_W3D];
+  a.pp3d = m->f[CM1G_PP3D];
   a.fpk = m->f[CM1G_DUM8];
-  a.dum1 = dum1;
+  a.dum1 = m->f[CM1G_DUM1];
   a.dum2 = m->f[CM1G_DUM2];
-  a.rru = rru;
-  a.rrv = rrv;
-  a.rrw = rrw;
+  a.rru = m->f[CM1G_RRU];
+  a.rrv = m->f[CM1G_RRV];
+  a.rrw = m->f[CM1G_RRW];
+  a.wa = m->f[CM1G_WA];
+}
+
+// a last stage of one substep: its damping term waited in scratch, since
+// other columns read ppx in the same launch
+static void ppx_single(cm1g_model *m, int nrk, int nloop) {
+  if (nrk != 3 || nloop != 1) return;
+  const KP P = m->P;
+  const float *d = m->tz;
+  float *ppx = m->f[CM1G_PPX];
+  for3(m, 1, P.ni, 1, P.nj, 1, P.nk, [=] __device__(int i, int j, int k) {
+    const int c = IXD(P, i, j, k);
+    ppx[c] = d[c];
+  });
+}
+
+void sound_run(cm1g_model *m, int nrk, bool fold1) {
+  const KP P = m->P;
+  const int ni = P.ni, nj = P.nj, nk = P.nk;
+  int nloop;
+  SubArgs a;
+  sub_args(m, nrk, a, &nloop);
+  const float dts = a.dts;
+  float *ppd = m->f[CM1G_DUM7];
+  float *u3d = m->f[CM1G_U3D], *v3d = m->f[CM1G_V3D], *w3d = m->f[CM1G_W3D];
+  const float *ua = m->f[CM1G_UA], *va = m->f[CM1G_VA], *wa = m->f[CM1G_WA];
+  const float *ppi = m->f[CM1G_PPI];
+  float *pp3d = m->f[CM1G_PP3D], *ppx = m->f[CM1G_PPX];
+
   // The copies the reference makes before the substeps (u3d=ua, ..., ppd=ppx,
   // src/sound.F:191-250) are folded into the first substep, which reads ua,
   // va, wa, ppi, ppx directly (after the first RK stage) and starts the
@@ -749,7 +770,6 @@ void sound_run(cm1g_model *m, int nrk, bool fold1) {
   // them when the caller says so, fold1: the folded form then needs no
   // copy of the scratch pair back into u3d/v3d)
   const bool fold = (nrk >= 2) || fold1;
-  a.wa = wa;
   const int slab = slab_variant(m);
   const ColGrid cg = col_grid(ni, nj, m->tile_rows);
   SlabGrid sg;
@@ -809,7 +829,8 @@ void sound_run(cm1g_model *m, int nrk, bool fold1) {
     a.ppdY = ppdb[(n - 1) & 1];
     a.wR = (n == 1 && fold) ? wa : w3d;
     a.ppR = (n == 1 && fold) ? ppi : pp3d;
-    a.wRp = (n == 2 && fold) ? wa : w3d;
+    a.wring = a.wR;
+    a.wringp = (n == 2 && fold) ? wa : w3d;
     a.first = (n == 1);
     a.last = (n == nloop);
     a.fold = ((nloop - n) & 1) == 0;
@@ -836,161 +857,225 @@ void sound_run(cm1g_model *m, int nrk, bool fold1) {
       v3d[c] = vs[c];
     });
   }
-  if (nrk == 3 && nloop == 1) {
-    const float *d = m->tz;
-    for3(m, 1, ni, 1, nj, 1, nk, [=] __device__(int i, int j, int k) {
-      int c = IXD(P, i, j, k);
-      ppx[c] = d[c];
-    });
+  ppx_single(m, nrk, nloop);
+}
+
+// ------------------------------------------------- explicit substeps
+// Operands of one level of a sounde_col column (raw loads; w and wten at
+// k + 1, which is where the level above starts).
+struct EXLoads {
+  float uXc, uXe, utc, ute, vXc, vXn, vtc, vtn;
+  float pdw, pde, pds, pdn, pdp;
+  float thw, the, ths, thn, thp;
+  float paw, pae, pas, pan, pap;
+  float ppterm, ppten, pp, w_p, wt_p;
+  float rru, rrv, rrw;
+};
+
+// c: the point's byte offset (O: 32 bits, or 64 for fields of 4 GiB and more)
+template <class O>
+__device__ __forceinline__ void ex_load(const KP &P, const SubArgs &a, O c, int k, EXLoads &L) {
+  const O pxB = (O)4 * P.px, pxyB = (O)4 * P.pxy, cN = c + pxB, cS = c - pxB, cU = c + pxyB;
+  L.uXc = ldo(a.uX, c); L.uXe = ldo(a.uX + 1, c);
+  L.utc = ldo(a.uten, c); L.ute = ldo(a.uten + 1, c);
+  L.vXc = ldo(a.vX, c); L.vXn = ldo(a.vX, cN);
+  L.vtc = ldo(a.vten, c); L.vtn = ldo(a.vten, cN);
+  L.pdw = ldo(a.ppdX - 1, c); L.pde = ldo(a.ppdX + 1, c); L.pds = ldo(a.ppdX, cS); L.pdn = ldo(a.ppdX, cN);
+  L.thw = ldo(a.thv - 1, c); L.the = ldo(a.thv + 1, c); L.ths = ldo(a.thv, cS); L.thn = ldo(a.thv, cN);
+  L.paw = ldo(a.piadv - 1, c); L.pae = ldo(a.piadv + 1, c); L.pas = ldo(a.piadv, cS); L.pan = ldo(a.piadv, cN);
+  L.ppterm = ldo(a.ppterm, c); L.ppten = ldo(a.ppten, c); L.pp = ldo(a.ppR, c);
+  if (k < P.nk) {
+    L.pdp = ldo(a.ppdX, cU); L.thp = ldo(a.thv, cU); L.pap = ldo(a.piadv, cU);
+    L.w_p = ldo(a.wR, cU); L.wt_p = ldo(a.wten, cU);
+  } else {
+    L.pdp = L.thp = L.pap = L.wt_p = 0.0f;
+    L.w_p = ldo(a.w3d, cU);  // the lid
+  }
+  L.rru = L.rrv = L.rrw = 0.0f;
+  if (a.fold && !a.init) {
+    L.rru = ldo(a.rru, c); L.rrv = ldo(a.rrv, c); L.rrw = ldo(a.rrw, c);
+  }
+}
+
+// One explicit acoustic substep of a column (src/sounde.F:333-352, 548-563,
+// 770-795): u, v, w from the previous substep's ppd, and the pressure from the
+// new velocities, whose values at i+1, j+1 and k+1 are formed here too (the
+// one at k+1 is then the level above's own).  u, v, w and ppd alternate
+// between two arrays, so neighbours read the old values; the averages take in
+// two substeps at a time, as in sound.  Per level row k of coef: p3, p4, p1,
+// p2 of the pi0 advection (src/sounde.F:117-136, 160-170), temw, c1, c2, mh.
+//
+// Memory bound: 12 arrays read and 5 written a substep, and the averages
+// every other one, against 18 and 8 for a velocity pass and a pressure pass.
+// Measured on 512 x 512 x 128: 0.70 ms a substep at 4.7 TB/s, what a large copy
+// reaches here, against 0.74 ms in two passes, and 0.9 ms a stage of copies that
+// set the substep's fields up no longer run.
+template <class O>
+__device__ __forceinline__ void sounde_col(const KP &P, const SubArgs &a, const ColGrid &cg, int bx) {
+  const int nmain = cg.per * NXCD;
+  if (bx >= nmain) {
+    const int npts = P.ni + P.nj + 1;
+    const int t = (bx - nmain) * (int)blockDim.x + (int)threadIdx.x;
+    if (t < npts * P.nk) sound_ring_point(P, a, t % npts, 1 + t / npts);
+    return;
+  }
+  int i, j, ks, ke;
+  const int ni = P.ni, nj = P.nj, nk = P.nk;
+  if (!col_tile_seg(cg, bx, nk, i, j, ks, ke)) return;
+  if (i > ni || j > nj) return;
+  const bool bw = a.opw && i == 1, be = a.ope && i == ni, bs = a.ops && j == 1, bn = a.opn && j == nj;
+  const bool edge = __builtin_amdgcn_ballot_w64(bw || be || bs || bn) != 0ULL;
+  const float dts = a.dts, rdx = P.rdx, rdy = P.rdy, rdz = P.rdz, smeps = P.K.smeps;
+  const float tem1 = a.tem1, tem2 = a.tem2, temx = a.temx, temy = a.temy;
+  // dts times the masks dtu0, dtv0 (zero on the faces of a non-periodic side)
+  const float dtu_c = (P.ibw && i == 1) ? 0.0f : dts, dtu_e = (P.ibe && i == ni) ? 0.0f : dts;
+  const float dtv_c = (P.ibs && j == 1) ? 0.0f : dts, dtv_n = (P.ibn && j == nj) ? 0.0f : dts;
+  const O pxyB = (O)4 * P.pxy;
+  O c = (O)4 * IX2D(P, i, j) + (O)ks * pxyB;
+  // values of this level carried from the one below
+  float pd_c = ldo(a.ppdX, c), th_c = ldo(a.thv, c), pa_c = ldo(a.piadv, c), pa_m = 0.0f;
+  float wo_c = ldo(a.wR, c), wn_c = wo_c;  // old and new w(k); w(1) does not change
+  EXLoads nx;
+  ex_load<O>(P, a, c, ks, nx);
+  if (ks > 1) {
+    const float *cf = a.coef + 8 * ks;
+    pa_m = ldo(a.piadv, c - pxyB);
+    wn_c = wo_c + dts * (ldo(a.wten, c) - cf[4] * (pd_c - ldo(a.ppdX, c - pxyB)) *
+                                                 (cf[6] * th_c + cf[5] * ldo(a.thv, c - pxyB)));
+  }
+  for (int k = ks; k <= ke; k++, c += pxyB) {
+    const EXLoads L = nx;
+    if (k < ke) ex_load<O>(P, a, c + pxyB, k + 1, nx);
+    float uo0 = L.uXc, uo1 = L.uXe, vo0 = L.vXc, vo1 = L.vXn;
+    if (edge) {
+      if (bw) uo0 = uo0 + dts * (-a.radbcw[(j + 2) + k * P.py] * (L.uXe - uo0) * rdx + L.utc);
+      if (be) uo1 = uo1 + dts * (-a.radbce[(j + 2) + k * P.py] * (uo1 - L.uXc) * rdx + L.ute);
+      if (bs) vo0 = vo0 + dts * (-a.radbcs[(i + 2) + k * P.px] * (L.vXn - vo0) * rdy + L.vtc);
+      if (bn) vo1 = vo1 + dts * (-a.radbcn[(i + 2) + k * P.px] * (vo1 - L.vXc) * rdy + L.vtn);
+    }
+    const float u0 = uo0 + dtu_c * (L.utc - tem1 * (pd_c - L.pdw) * (th_c + L.thw));
+    const float u1 = uo1 + dtu_e * (L.ute - tem1 * (L.pde - pd_c) * (L.the + th_c));
+    const float v0 = vo0 + dtv_c * (L.vtc - tem2 * (pd_c - L.pds) * (th_c + L.ths));
+    const float v1 = vo1 + dtv_n * (L.vtn - tem2 * (L.pdn - pd_c) * (L.thn + th_c));
+    const float *cf = a.coef + 8 * k;
+    float w1 = L.w_p, pk1 = 0.0f, pk2 = 0.0f;
+    if (k < nk) {
+      w1 = w1 + dts * (L.wt_p - cf[8 + 4] * (L.pdp - pd_c) * (cf[8 + 6] * L.thp + cf[8 + 5] * th_c));
+      pk2 = cf[3] * L.pap + cf[2] * pa_c;
+    }
+    if (k > 1) pk1 = cf[0] * pa_m + cf[1] * pa_c;
+    const float w0 = wn_c;
+    float div = ((u1 - u0) * rdx + (v1 - v0) * rdy) + (w1 - w0) * rdz * cf[7];
+    if (fabsf(div) < smeps) div = 0.0f;
+    const float delp = dts * (L.ppten - L.ppterm * div) +
+                       (-(u0 * (pa_c - L.paw) + u1 * (L.pae - pa_c)) * temx -
+                        (v0 * (pa_c - L.pas) + v1 * (L.pan - pa_c)) * temy) +
+                       (w0 * pk1 + w1 * pk2);
+    float p = L.pp + delp;
+    if (fabsf(p) < smeps) p = 0.0f;
+    const float d = a.kdiv * delp;
+    sto(a.uY, c, u0);
+    sto(a.vY, c, v0);
+    sto(a.wY, c, w0);
+    sto(a.pp3d, c, p);
+    sto(a.ppdY, c, p + d);
+    if (!a.last) put_p_halo(P, a.ppdY, i, j, k, p + d);
+    if (a.ppx) sto(a.ppx, c, d);
+    if (a.fold) {
+      sto(a.rru, c, avg_uv(a, L.rru, L.uXc, u0));
+      sto(a.rrv, c, avg_uv(a, L.rrv, L.vXc, v0));
+      sto(a.rrw, c, avg_uv(a, L.rrw, wo_c, w0));
+    }
+    pd_c = L.pdp;
+    th_c = L.thp;
+    pa_m = pa_c;
+    pa_c = L.pap;
+    wo_c = L.w_p;
+    wn_c = w1;
   }
 }
 
 // Explicit acoustic substeps, psolver=2 (sounde, src/sounde.F:10-1026;
-// Cartesian, no terrain).  Per substep: the radiative open-boundary
-// velocities, then one kernel that advances u, v, w from the previous
-// substep's ppd (src/sounde.F:333-352, 548-563) and folds them into the
-// averages, then one kernel for the pressure (src/sounde.F:770-795) whose
-// pi0 vertical-advection coefficients pk1/pk2 (src/sounde.F:117-136,
-// 160-170) are evaluated on the fly.
-void sounde_run(cm1g_model *m, int nrk) {
+// Cartesian, no terrain).  The copies the reference makes before the substeps
+// (u3d=ua, ..., ppd=ppx, src/sounde.F:181-233) are folded into the first one
+// (fold: from the second stage on, or where the caller says that u3d..pp3d
+// equal ua..ppi).
+void sounde_run(cm1g_model *m, int nrk, bool fold1) {
   const KP P = m->P;
   const int ni = P.ni, nj = P.nj, nk = P.nk;
-  const float dt = m->c.dt, kdiv = m->c.kdiv;
   int nloop;
-  float dts;
-  sound_nloop(nrk, m->c.nsound, dt, &nloop, &dts);
-  float *dum1 = m->f[CM1G_DUM1], *ppd = m->f[CM1G_DUM7];
-  const float *piadv = m->f[CM1G_SADV], *thv = m->f[CM1G_T11], *ppterm = m->f[CM1G_T22];
-  float *u3d = m->f[CM1G_U3D], *v3d = m->f[CM1G_V3D], *w3d = m->f[CM1G_W3D];
-  const float *ua = m->f[CM1G_UA], *va = m->f[CM1G_VA], *wa = m->f[CM1G_WA];
-  const float *uten = m->f[CM1G_UTEN], *vten = m->f[CM1G_VTEN], *wten = m->f[CM1G_WTEN];
-  float *rru = m->f[CM1G_RRU], *rrv = m->f[CM1G_RRV], *rrw = m->f[CM1G_RRW];
-  const float *ppi = m->f[CM1G_PPI], *ppten = m->f[CM1G_PPTEN];
-  float *pp3d = m->f[CM1G_PP3D], *ppx = m->f[CM1G_PPX];
-  const float *radbcw = m->d2[CM1G_D_RADBCW], *radbce = m->d2[CM1G_D_RADBCE];
-  const float *radbcs = m->d2[CM1G_D_RADBCS], *radbcn = m->d2[CM1G_D_RADBCN];
-  const float *dtu0 = m->dtu0, *dtv0 = m->dtv0;
-  const float rdx = P.rdx, rdy = P.rdy, rdz = P.rdz, cp = P.K.cp, smeps = P.K.smeps;
-
-  // prep copies (src/sounde.F:181-233); the first stage skips u3d = ua ...
-  // because they are equal, except after an exchanging solve3, when the
-  // 3-D arrays still hold the previous step
-  if (nrk == 1 && !m->swapped) {
-    for3(m, 0, ni + 1, 0, nj + 1, 1, nk, [=] __device__(int i, int j, int k) {
-      int c = IXD(P, i, j, k);
-      ppd[c] = ppx[c];
-      rru[c] = 0.0f;
-      rrv[c] = 0.0f;
-      rrw[c] = 0.0f;
+  SubArgs a;
+  sub_args(m, nrk, a, &nloop);
+  a.expl = 1;
+  const bool fold = (nrk >= 2) || fold1;
+  {
+    float *cf = m->scoef;
+    const float dts = a.dts, rdz = P.rdz, cp = P.K.cp;
+    launch<64>(m, dim3((nk + 63) / 64), dim3(64), [=] __device__(int bx, int, int) {
+      const int k = 1 + bx * 64 + (int)threadIdx.x;
+      if (k > nk) return;
+      float *o = cf + 8 * k;
+      const float mh = P.mh[k], rr0 = P.rr0[k];
+      o[0] = dts * rdz * mh * rr0 * P.rf0[k] * P.c1[k];
+      o[1] = dts * rdz * mh * rr0 * P.rf0[k] * (P.c2[k] - 1.0f);
+      o[2] = dts * rdz * mh * rr0 * P.rf0[k + 1] * (1.0f - P.c1[k + 1]);
+      o[3] = -(dts * rdz * mh * rr0 * P.rf0[k + 1] * P.c2[k + 1]);
+      o[4] = rdz * cp * P.mf[k];
+      o[5] = P.c1[k];
+      o[6] = P.c2[k];
+      o[7] = mh;
     });
-  } else {
-    for3(m, 0, ni + 1, 0, nj + 1, 1, nk, [=] __device__(int i, int j, int k) {
-      int c = IXD(P, i, j, k);
-      u3d[c] = ua[c];
-      rru[c] = 0.0f;
-      v3d[c] = va[c];
-      rrv[c] = 0.0f;
-      w3d[c] = wa[c];
-      rrw[c] = 0.0f;
-      pp3d[c] = ppi[c];
-      ppd[c] = ppx[c];
-    });
+    a.coef = cf;
   }
-
-  const bool opw = (P.wbc == 2 && P.ibw == 1), ope = (P.ebc == 2 && P.ibe == 1);
-  const bool ops = (P.sbc == 2 && P.ibs == 1), opn = (P.nbc == 2 && P.ibn == 1);
-  const float tavg = 1.0f / (float)nloop;
+  ColGrid cg = col_grid(ni, nj, m->tile_rows);
+  col_split(m, cg, nk);
+  const dim3 blk = col_threads(cg);
+  dim3 grd = col_blocks(cg);
+  a.nring = ((ni + nj + 1) * nk + (int)blk.x - 1) / (int)blk.x;
+  grd.x += a.nring;
+  float *u3d = m->f[CM1G_U3D], *v3d = m->f[CM1G_V3D], *w3d = m->f[CM1G_W3D], *pp3d = m->f[CM1G_PP3D];
+  float *ppx = m->f[CM1G_PPX], *ppdb[2] = {m->f[CM1G_DUM7], m->tx};
+  const float *ua = m->f[CM1G_UA], *va = m->f[CM1G_VA], *wa = m->f[CM1G_WA], *ppi = m->f[CM1G_PPI];
+  float *us = m->scr1, *vs = m->scr2, *ws = m->ty;
+  const float *up = nullptr, *vp = nullptr, *wp = nullptr;
+  a.wring = fold ? wa : w3d;
   for (int n = 1; n <= nloop; n++) {
-    const bool last = (n == nloop);
-    if (opw || ope)
-      for2(m, 1, nj, 1, nk, [=] __device__(int j, int k) {
-        if (opw)
-          u3d[IXD(P, 1, j, k)] = u3d[IXD(P, 1, j, k)] + dts * (-radbcw[(j + 2) + k * P.py] *
-              (u3d[IXD(P, 2, j, k)] - u3d[IXD(P, 1, j, k)]) * rdx + uten[IXD(P, 1, j, k)]);
-        if (ope)
-          u3d[IXD(P, ni + 1, j, k)] = u3d[IXD(P, ni + 1, j, k)] + dts * (-radbce[(j + 2) + k * P.py] *
-              (u3d[IXD(P, ni + 1, j, k)] - u3d[IXD(P, ni, j, k)]) * rdx + uten[IXD(P, ni + 1, j, k)]);
-      });
-    if (ops || opn)
-      for2(m, 1, ni, 1, nk, [=] __device__(int i, int k) {
-        if (ops)
-          v3d[IXD(P, i, 1, k)] = v3d[IXD(P, i, 1, k)] + dts * (-radbcs[(i + 2) + k * P.px] *
-              (v3d[IXD(P, i, 2, k)] - v3d[IXD(P, i, 1, k)]) * rdy + vten[IXD(P, i, 1, k)]);
-        if (opn)
-          v3d[IXD(P, i, nj + 1, k)] = v3d[IXD(P, i, nj + 1, k)] + dts * (-radbcn[(i + 2) + k * P.px] *
-              (v3d[IXD(P, i, nj + 1, k)] - v3d[IXD(P, i, nj, k)]) * rdy + vten[IXD(P, i, nj + 1, k)]);
-      });
-    // u, v, w forward and the velocity averages
-    {
-      const float tem1 = rdx * cp * 0.5f, tem2 = rdy * cp * 0.5f;
-      for3(m, 1, ni + 1, 1, nj + 1, 1, nk, [=] __device__(int i, int j, int k) {
-        const int c = IXD(P, i, j, k);
-        const float dtu = dts * dtu0[IX2D(P, i, j)], dtv = dts * dtv0[IX2D(P, i, j)];
-        const float u = u3d[c] + dtu * (uten[c] - tem1 * (ppd[c] - ppd[c - 1]) *
-                                                      (thv[c] + thv[c - 1]));
-        const float v = v3d[c] + dtv * (vten[c] - tem2 * (ppd[c] - ppd[c - P.px]) *
-                                                      (thv[c] + thv[c - P.px]));
-        float w = w3d[c];
-        if (k >= 2 && i <= ni && j <= nj) {
-          const float temw = rdz * cp * P.mf[k];
-          w = w + dts * (wten[c] - temw * (ppd[c] - ppd[c - P.pxy]) *
-                                       (P.c2[k] * thv[c] + P.c1[k] * thv[c - P.pxy]));
-          w3d[c] = w;
-        }
-        u3d[c] = u;
-        v3d[c] = v;
-        if (last) {
-          rru[c] = (rru[c] + u) * tavg;
-          rrv[c] = (rrv[c] + v) * tavg;
-          rrw[c] = (rrw[c] + w) * tavg;
-        } else {
-          rru[c] = rru[c] + u;
-          rrv[c] = rrv[c] + v;
-          rrw[c] = rrw[c] + w;
-        }
-      });
-    }
-    // pressure
-    {
-      const float temx = dts * 0.5f * rdx, temy = dts * 0.5f * rdy;
-      for3(m, 1, ni, 1, nj, 1, nk, [=] __device__(int i, int j, int k) {
-        const int c = IXD(P, i, j, k);
-        const float mh = P.mh[k], rr0 = P.rr0[k];
-        float pk1 = 0.0f, pk2 = 0.0f;
-        if (k < nk) {
-          const float p1 = dts * rdz * mh * rr0 * P.rf0[k + 1] * (1.0f - P.c1[k + 1]);
-          const float p2 = -(dts * rdz * mh * rr0 * P.rf0[k + 1] * P.c2[k + 1]);
-          pk2 = p2 * piadv[c + P.pxy] + p1 * piadv[c];
-        }
-        if (k > 1) {
-          const float p3 = dts * rdz * mh * rr0 * P.rf0[k] * P.c1[k];
-          const float p4 = dts * rdz * mh * rr0 * P.rf0[k] * (P.c2[k] - 1.0f);
-          pk1 = p3 * piadv[c - P.pxy] + p4 * piadv[c];
-        }
-        const float u0 = u3d[c], u1 = u3d[c + 1], v0 = v3d[c], v1 = v3d[c + P.px];
-        const float w0 = w3d[c], w1 = w3d[c + P.pxy];
-        const float pa = piadv[c];
-        float div = ((u1 - u0) * rdx + (v1 - v0) * rdy) + (w1 - w0) * rdz * mh;
-        if (fabsf(div) < smeps) div = 0.0f;
-        const float delp = dts * (ppten[c] - ppterm[c] * div) +
-                           (-(u0 * (pa - piadv[c - 1]) + u1 * (piadv[c + 1] - pa)) * temx -
-                            (v0 * (pa - piadv[c - P.px]) + v1 * (piadv[c + P.px] - pa)) * temy) +
-                           (w0 * pk1 + w1 * pk2);
-        float p = pp3d[c] + delp;
-        if (fabsf(p) < smeps) p = 0.0f;
-        pp3d[c] = p;
-        const float d = kdiv * delp;
-        if (last) dum1[c] = d;
-        ppd[c] = p + d;
-        if (!last) put_p_halo(P, ppd, i, j, k, p + d);
-      });
-    }
+    // the last substep writes u3d; from the state arrays themselves the first
+    // one writes the scratch set
+    const bool scratch = fold ? ((nloop - n) & 1) != 0 : (n & 1) != 0;
+    a.uX = (n == 1) ? (fold ? ua : u3d) : up;
+    a.vX = (n == 1) ? (fold ? va : v3d) : vp;
+    a.wR = (n == 1) ? (fold ? wa : w3d) : wp;
+    a.uY = scratch ? us : u3d;
+    a.vY = scratch ? vs : v3d;
+    a.wY = scratch ? ws : w3d;
+    a.ppdX = (n == 1) ? ppx : ppdb[n & 1];
+    a.ppdY = ppdb[(n - 1) & 1];
+    a.ppR = (n == 1 && fold) ? ppi : pp3d;
+    a.first = (n == 1);
+    a.last = (n == nloop);
+    a.fold = ((nloop - n) & 1) == 0;
+    a.pair = (n > 1);
+    a.init = (n <= 2);
+    a.ppx = (nrk == 3 && a.last) ? (a.first ? m->tz : ppx) : nullptr;
+    if (m->ntot < ((size_t)1 << 30))
+      launch<256>(m, grd, blk, [=] __device__(int bx, int, int) { sounde_col<unsigned>(P, a, cg, bx); });
+    else
+      launch<256>(m, grd, blk, [=] __device__(int bx, int, int) { sounde_col<size_t>(P, a, cg, bx); });
+    up = a.uY;
+    vp = a.vY;
+    wp = a.wY;
   }
-  if (nrk == 3)
-    for3(m, 1, ni, 1, nj, 1, nk, [=] __device__(int i, int j, int k) {
-      int c = IXD(P, i, j, k);
-      ppx[c] = dum1[c];
+  if (!fold && (nloop & 1)) {
+    // the last substep wrote the scratch set: copy the updated range back
+    for3(m, 1, ni + 1, 1, nj + 1, 1, nk, [=] __device__(int i, int j, int k) {
+      const int c = IXD(P, i, j, k);
+      u3d[c] = us[c];
+      v3d[c] = vs[c];
+      if (i <= ni && j <= nj) w3d[c] = ws[c];
     });
+  }
+  ppx_single(m, nrk, nloop);
 }
 
 // getdiv (t11 from the time-averaged velocities) and getdivx (divx from the

@@ -34,3 +34,33 @@ def test_substep_edges_match_oracle(require_gpu, ni, nj, nk, nsound, bc):
             b = interior(o.f(name), nk, nj, ni, stag)
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (n, name)
     g.close()
+
+
+@pytest.mark.parametrize("ni,nj,nk,nsound,bc", [
+    (8, 8, 6, 2, 2),       # single-substep stages
+    (9, 8, 7, 5, 2),       # an odd count
+    (65, 9, 30, 7, 1),
+    (130, 12, 13, 10, 2),
+    (12, 10, 49, 12, 1),
+])
+@pytest.mark.parametrize("held", [False, True], ids=["exchanged", "addresses-held"])
+def test_explicit_substep_matches_oracle(require_gpu, ni, nj, nk, nsound, bc, held):
+    """psolver 2; also with the address of ua handed out, when every stage
+    starts from the 3-D arrays themselves."""
+    import ctypes as C
+    from cm1_amd import _native as N
+    cfgd, cols, fields = case(ni=ni, nj=nj, nk=nk, nsound=nsound, bc=bc, dz=15000.0 / nk, dt=0.25 * nsound, amp=2.0,
+                              psolver=2)
+    g = make_gpu(cfgd, cols, fields)
+    o = make_oracle(cfgd, cols, fields)
+    if held:
+        p = C.c_void_p()
+        N.check(g.L.cm1g_field_ptr(g.h, N.FID["ua"], C.byref(p)), "cm1g_field_ptr")
+    for n in (1, 2):
+        g.step(n)
+        o.step(n)
+        for name, stag in PROG + [("ppx", None)]:
+            a = g.interior(name, stag)
+            b = interior(o.f(name), nk, nj, ni, stag)
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (n, name)
+    g.close()
