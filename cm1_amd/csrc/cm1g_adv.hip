@@ -15,9 +15,14 @@
 // cell takes from or gives to its two neighbours (pdefx2/pdefy2/pdefz).
 // The reference scatters inside a sequential loop; here each cell gathers
 // the same terms in the same order (left neighbour, itself, right
-// neighbour), which reproduces the sequential sums bit for bit.  dum is not
-// stored: each cell evaluates it at the five points it needs, mapping halo
-// points to the interior point the fill copies.
+// neighbour), which reproduces the sequential sums bit for bit.
+//
+// Only a cell with a negative dum, and the cells next to it, are corrected.
+// So the advection kernel itself forms every cell's dum (it holds all the
+// operands), writes the uncorrected update and a bit per cell that says
+// whether a dum was negative; pdef_fix then reads the bits, and where one is
+// set nearby it evaluates dum at the points a cell needs, mapping halo points
+// to the interior point the fill copies, and writes the corrected update.
 
 // mass flux of direction dir at the lower face of (c, level k) and at the
 // upper one (c + stride): with scale, the getdivx scaling rho0(k) for u,v
@@ -70,8 +75,8 @@ __device__ __forceinline__ float pdef_dum(const KP &P, int dir, const float *vel
 // halo point of the horizontal fill (bcs, src/bc.F:180-364) -> the
 // interior point whose value it holds
 __device__ __forceinline__ int pdef_wrap(int m, int n, bool periodic) {
-  if (m < 1) return periodic ? m + n : 1;
-  if (m > n) return periodic ? m - n : n;
+  if (m < 1) return periodic ? max(m + n, 1) : 1;
+  if (m > n) return periodic ? min(m - n, n) : n;  // (past the halo: any point)
   return m;
 }
 
@@ -108,116 +113,130 @@ __device__ __forceinline__ float pdef_gather(float dm2, float dm1, float d0, flo
   return mass;
 }
 
-// x and y directions (pdefx1/x2, pdefy1/y2): corrected advx, advy
 struct PdefArgs {
-  const float *rru, *rrv, *rrw, *advx, *advy, *advz, *s0, *s;
-  float *ax_out, *ay_out;
-  const float *sten0, *t11, *thterm, *divx;
+  const float *rru, *rrv, *rrw, *advx, *advy, *advz, *s0, *s, *sten0, *divx;
+  const unsigned long long *marks;  // per level, row and 64 columns: advs_col
   float *out_sten, *out_new;
   float dt;
-  int smeps_flush, scale;
+  int smeps_flush, scale, gx, lev;
 };
 
-// One 64 x 4 block per tile of one level.  Each cell's dum in x and in y
-// is evaluated once and shared through LDS: a cell needs dum at i-2..i+2
-// and at j-2..j+2, so the block evaluates its own 64 x 4 points in each
-// direction plus the two-point halos (4 x 4 in x, 64 x 4 in y), at the
-// indices the halo fill maps them to.
-__device__ __forceinline__ void pdef_xy(const KP &P, const PdefArgs &a, int bx, int by, int bz) {
+constexpr int PDEF_L = 8;  // most levels a pdef_fix workgroup looks after
+
+// One workgroup per tile of 64 x 4 columns and a.lev levels: its threads
+// read the marks of the tile and of its neighbours, and the workgroup visits
+// the levels on which a cell of the tile can be corrected.  There each cell's
+// dum in x and in y is evaluated once and shared through LDS (the tile's own
+// points and two-point halos); dum in z stays in registers, as a window that
+// moves up while consecutive levels are visited.  A cell no correction
+// reaches keeps what the advection kernel wrote.
+//
+// Memory bound, in all 25 arrays a field before (advx, advy, advz written,
+// a pass over x and y, a pass over z), 11 and the visited tiles' now.
+// Measured, advection and correction of a field: 1024 x 1024 x 96 (qv, qc, qr)
+// 2.53 -> 1.48 ms, of which pdef_fix 0.25; 512 x 512 x 128 (WENO, tracers) 0.95
+// -> 0.55, pdef_fix 0.03; 64 x 64 x 40, where every tile is visited, 25 -> 19 us.
+__device__ __forceinline__ void pdef_fix(const KP &P, const PdefArgs &a, int bx, int by, int bz) {
   __shared__ float dxs[4][68];
   __shared__ float dys[8][64];
-  const int tx = (int)threadIdx.x, ty = (int)threadIdx.y;
+  __shared__ unsigned need;
+  const int tx = (int)threadIdx.x, ty = (int)threadIdx.y, t = ty * 64 + tx;
   const int i0 = 1 + bx * 64, j0 = 1 + by * 4;
   const int i = i0 + tx, j = j0 + ty;
-  const int k = 1 + bz;
-  const int ni = P.ni, nj = P.nj;
+  const int ni = P.ni, nj = P.nj, nk = P.nk;
+  const int lev = a.lev, k0 = 1 + bz * lev, k1 = min(k0 + lev - 1, nk);
   const bool perx = (P.wbc == 1), pery = (P.sbc == 1);
-  const bool in = (i <= ni && j <= nj);
+  if (t == 0) need = 0u;
+  __syncthreads();
   {
-    // x: own point of this row, and the row's halo points i0-2, i0-1, i0+64, i0+65
-    const int jj = pdef_wrap(j, nj, pery);
-    dxs[ty][tx + 2] = pdef_dum(P, 0, a.rru, a.scale, a.advx, a.s0, a.s, a.dt, pdef_wrap(i, ni, perx), jj, k);
-    if (tx < 4) {
-      const int o = (tx < 2) ? tx - 2 : 62 + tx;
-      dxs[ty][(tx < 2) ? tx : 64 + tx] =
-          pdef_dum(P, 0, a.rru, a.scale, a.advx, a.s0, a.s, a.dt, pdef_wrap(i0 + o, ni, perx), jj, k);
+    static_assert(6 * (PDEF_L + 2) + 8 * PDEF_L <= 256, "one word a thread");
+    const int own = 6 * (lev + 2);  // rows j0-1..j0+4, levels k0-1..k0+lev
+    const unsigned all = (1u << lev) - 1u;
+    unsigned m = 0u;
+    if (t < own) {
+      const int b = t / 6 - 1, r = t - 6 * (b + 1), k = k0 + b;
+      const int jj = pdef_wrap(j0 - 1 + r, nj, pery);
+      if (k >= 1 && k <= nk && a.marks[((size_t)(k - 1) * nj + (jj - 1)) * a.gx + bx])
+        m = (r == 0 || r == 5) ? (b >= 0 ? 1u << b : 0u) : (7u << (b + 1)) >> 2;
+    } else if (t < own + 8 * lev) {
+      // columns i0-1 and i0+64 of rows j0..j0+3
+      const int u = t - own, b = u >> 3, k = k0 + b;
+      const int ii = pdef_wrap((u & 1) ? i0 + 64 : i0 - 1, ni, perx);
+      const int jj = pdef_wrap(j0 + ((u >> 1) & 3), nj, pery);
+      if (k <= nk &&
+          ((a.marks[((size_t)(k - 1) * nj + (jj - 1)) * a.gx + ((ii - 1) >> 6)] >> ((ii - 1) & 63)) & 1ULL))
+        m = 1u << b;
     }
-    // y: own point of this column, and one halo row (j0-2, j0-1, j0+4, j0+5)
-    const int ii = (i <= ni) ? i : ni;
-    dys[ty + 2][tx] = pdef_dum(P, 1, a.rrv, a.scale, a.advy, a.s0, a.s, a.dt, ii, pdef_wrap(j, nj, pery), k);
-    const int hr = (ty < 2) ? ty : ty + 4;
-    dys[hr][tx] = pdef_dum(P, 1, a.rrv, a.scale, a.advy, a.s0, a.s, a.dt, ii,
-                           pdef_wrap(j0 - 2 + hr, nj, pery), k);
+    m &= all;
+    if (m) atomicOr(&need, m);
   }
   __syncthreads();
-  if (!in) return;
-  const int c = IXD(P, i, j, k);
-  const float smeps = P.K.smeps, rdt = 1.0f / a.dt;
-  const float r0s0 = P.rho0[k] * a.s0[c];
-  {
-    const float *d = &dxs[ty][tx];
-    bool flag;
-    const float mass = pdef_gather(d[0], d[1], d[2], d[3], d[4], i - 1 >= 0, i + 1 <= ni + 1, smeps, flag);
-    float out = a.advx[c];
-    if (flag) {
-      float lo, hi;
-      pdef_faces(P, 0, a.rru, a.scale, c, k, lo, hi);
-      out = (d[2] + mass - r0s0) * rdt - a.s[c] * (hi - lo) * P.rdx;
-    }
-    a.ax_out[c] = out;
-  }
-  {
-    bool flag;
-    const float mass = pdef_gather(dys[ty][tx], dys[ty + 1][tx], dys[ty + 2][tx], dys[ty + 3][tx],
-                                   dys[ty + 4][tx], j - 1 >= 0, j + 1 <= nj + 1, smeps, flag);
-    float out = a.advy[c];
-    if (flag) {
-      float lo, hi;
-      pdef_faces(P, 1, a.rrv, a.scale, c, k, lo, hi);
-      out = (dys[ty + 2][tx] + mass - r0s0) * rdt - a.s[c] * (hi - lo) * P.rdy;
-    }
-    a.ay_out[c] = out;
-  }
-}
-
-// z direction (pdefz) marched up each column with a window of dum, then the
-// tendency with the corrected advx, advy, advz and the s0 + dt*sten update
-__device__ __forceinline__ void pdef_z(const KP &P, const PdefArgs &a, const ColGrid &cg, int bx) {
-  int i, j, ks, ke;
-  const int ni = P.ni, nj = P.nj, nk = P.nk;
-  if (!col_tile_seg(cg, bx, nk, i, j, ks, ke)) return;
-  if (i > ni || j > nj) return;
+  const unsigned nd = __builtin_amdgcn_readfirstlane(need);
+  if (nd == 0u) return;
+  const bool in = (i <= ni && j <= nj);
+  const int ii = pdef_wrap(i, ni, perx), jj = pdef_wrap(j, nj, pery);
+  const int ic = min(i, ni), jc = min(j, nj);
+  const int o = (tx < 2) ? tx - 2 : 62 + tx, hr = (ty < 2) ? ty : ty + 4;
+  const int ih = pdef_wrap(i0 + o, ni, perx), jh = pdef_wrap(j0 - 2 + hr, nj, pery);
   const float smeps = P.K.smeps, rdt = 1.0f / a.dt;
   auto dz = [&](int kk) -> float {  // dum of pdefz; zero outside 1..nk
     if (kk < 1 || kk > nk) return 0.0f;
-    return pdef_dum(P, 2, a.rrw, a.scale, a.advz, a.s0, a.s, a.dt, i, j, kk);
+    return pdef_dum(P, 2, a.rrw, a.scale, a.advz, a.s0, a.s, a.dt, ic, jc, kk);
   };
-  float dm2 = dz(ks - 2), dm1 = dz(ks - 1), d0 = dz(ks), dp1 = dz(ks + 1), dp2 = dz(ks + 2);
-  for (int k = ks; k <= ke; k++) {
-    const int c = IXD(P, i, j, k);
-    bool flag;
-    const float mass = pdef_gather(dm2, dm1, d0, dp1, dp2, k - 1 >= 1, k + 1 <= nk, smeps, flag);
-    const float sc = a.s[c];
-    float az = a.advz[c];
-    if (flag) {
-      float lo, hi;
-      pdef_faces(P, 2, a.rrw, a.scale, c, k, lo, hi);
-      az = (d0 + mass - P.rho0[k] * a.s0[c]) * rdt - sc * (hi - lo) * P.rdz * P.mh[k];
+  float dm2 = 0.0f, dm1 = 0.0f, d0 = 0.0f, dp1 = 0.0f, dp2 = 0.0f;
+  for (int k = k0, last = -1; k <= k1; k++) {
+    if (!((nd >> (k - k0)) & 1u)) continue;
+    // (the previous level's cells have been read)
+    if (last >= 0) __syncthreads();
+    dxs[ty][tx + 2] = pdef_dum(P, 0, a.rru, a.scale, a.advx, a.s0, a.s, a.dt, ii, jc, k);
+    if (tx < 4)
+      dxs[ty][(tx < 2) ? tx : 64 + tx] = pdef_dum(P, 0, a.rru, a.scale, a.advx, a.s0, a.s, a.dt, ih, jc, k);
+    dys[ty + 2][tx] = pdef_dum(P, 1, a.rrv, a.scale, a.advy, a.s0, a.s, a.dt, ic, jj, k);
+    dys[hr][tx] = pdef_dum(P, 1, a.rrv, a.scale, a.advy, a.s0, a.s, a.dt, ic, jh, k);
+    if (last == k - 1) {
+      dm2 = dm1;
+      dm1 = d0;
+      d0 = dp1;
+      dp1 = dp2;
+    } else {
+      dm2 = dz(k - 2);
+      dm1 = dz(k - 1);
+      d0 = dz(k);
+      dp1 = dz(k + 1);
     }
-    float st = a.sten0[c];
-    if (a.t11) st = st - a.t11[c] * a.thterm[c];
-    st = st + ((a.ax_out[c] + a.ay_out[c]) + az + sc * a.divx[c]) * P.rr0[k];
-    if (a.out_sten) a.out_sten[c] = st;
-    if (a.out_new) {
-      float v = a.s0[c] + a.dt * st;
-      if (a.smeps_flush && fabsf(v) < P.K.smeps) v = 0.0f;
-      a.out_new[c] = v;
+    dp2 = dz(k + 2);
+    last = k;
+    __syncthreads();
+    bool fx, fy, fz;
+    const float *dx = &dxs[ty][tx];
+    const float mx = pdef_gather(dx[0], dx[1], dx[2], dx[3], dx[4], true, true, smeps, fx);
+    const float my = pdef_gather(dys[ty][tx], dys[ty + 1][tx], dys[ty + 2][tx], dys[ty + 3][tx], dys[ty + 4][tx],
+                                 true, true, smeps, fy);
+    const float mz = pdef_gather(dm2, dm1, d0, dp1, dp2, k - 1 >= 1, k + 1 <= nk, smeps, fz);
+    if (in && (fx || fy || fz)) {
+      const int c = IXD(P, i, j, k);
+      const float sc = a.s[c], s0 = a.s0[c], r0s0 = P.rho0[k] * s0;
+      float ax = a.advx[c], ay = a.advy[c], az = a.advz[c], lo, hi;
+      if (fx) {
+        pdef_faces(P, 0, a.rru, a.scale, c, k, lo, hi);
+        ax = (dx[2] + mx - r0s0) * rdt - sc * (hi - lo) * P.rdx;
+      }
+      if (fy) {
+        pdef_faces(P, 1, a.rrv, a.scale, c, k, lo, hi);
+        ay = (dys[ty + 2][tx] + my - r0s0) * rdt - sc * (hi - lo) * P.rdy;
+      }
+      if (fz) {
+        pdef_faces(P, 2, a.rrw, a.scale, c, k, lo, hi);
+        az = (d0 + mz - r0s0) * rdt - sc * (hi - lo) * P.rdz * P.mh[k];
+      }
+      const float st = a.sten0[c] + ((ax + ay) + az + sc * a.divx[c]) * P.rr0[k];
+      if (a.out_sten) a.out_sten[c] = st;
+      if (a.out_new) {
+        float v = s0 + a.dt * st;
+        if (a.smeps_flush && fabsf(v) < smeps) v = 0.0f;
+        a.out_new[c] = v;
+      }
     }
-    dm2 = dm1;
-    dm1 = d0;
-    d0 = dp1;
-    dp1 = dp2;
-    dp2 = dz(k + 3);
   }
 }
 
@@ -227,9 +246,10 @@ struct AdvsArgs {
   float sadd;                     // nonzero: advect (th0(k)-th0r) + s
   const float *s0, *sten0, *t11, *thterm, *rru, *rrv, *rrw, *divx;
   float *out_sten, *out_new;      // tendency and/or s0 + dt*tendency
-  float *advx, *advy, *advz;      // mode 1: the three advective tendencies
+  float *advx, *advy, *advz;      // positive-definite pass: the three advective tendencies,
+  unsigned long long *marks;      // and a bit per cell, set where a dum is negative
   float dt;
-  int smeps_flush, mode;          // mode 0: final tendency; 1: advx/advy/advz only
+  int smeps_flush, gx;            // gx: words of marks per row
   int pdef, pdefweno;             // WENO5 magnitude tests (horizontal / vertical)
   double weps;
   int scale;                      // rru/rrv/rrw are the averaged velocities: scale by
@@ -249,7 +269,7 @@ struct AdvLevel {
 // o: the column's byte offset in a level.  The start of level k of an array,
 // and of its neighbouring rows, is formed in scalar registers, so a level's
 // loads need no address arithmetic in vector registers.
-template <bool WENO, bool TH>
+template <bool PD, bool TH>
 __device__ __forceinline__ void advs_load(const KP &P, const AdvsArgs &a, unsigned o, int k,
                                           AdvLevel &L) {
   const int nk = P.nk;
@@ -262,7 +282,8 @@ __device__ __forceinline__ void advs_load(const KP &P, const AdvsArgs &a, unsign
   L.yp1 = ldo(s + px, o); L.yp2 = ldo(s + 2 * px, o); L.yp3 = ldo(s + 3 * px, o);
   L.ru0 = ldo(a.rru + kb, o); L.ru1 = ldo(a.rru + kb + 1, o);
   L.rv0 = ldo(a.rrv + kb, o); L.rv1 = ldo(a.rrv + kb + px, o);
-  L.rw1 = (k < nk) ? ldo(a.rrw + kb + P.pxy, o) : 0.0f;
+  // (unscaled, pdefz takes the top face as it is given)
+  L.rw1 = (k < nk || (PD && !a.scale)) ? ldo(a.rrw + kb + P.pxy, o) : 0.0f;
   if (a.scale) {
     const float r0 = P.rho0[k];
     L.ru0 = L.ru0 * r0; L.ru1 = L.ru1 * r0;
@@ -285,8 +306,9 @@ __device__ __forceinline__ void advs_load(const KP &P, const AdvsArgs &a, unsign
 // results are bitwise equal to separate flux / divergence passes.  The
 // operands of level k+1 are loaded before level k is evaluated and stored.
 // The uniform switches are compile-time: SADD (theta's offset form), TH
-// (theta's t11*thterm term), MODE1 (advx/advy/advz for the pdef pass).
-template <bool WENO, bool SADD, bool TH, bool MODE1>
+// (theta's t11*thterm term), PD (positive definite: advx/advy/advz and the
+// marks are written as well, for pdef_fix).
+template <bool WENO, bool SADD, bool TH, bool PD>
 __device__ __forceinline__ void advs_col(const KP &P, const AdvsArgs &a, const ColGrid &cg, int bx) {
   int i, j, ks, ke;
   const int ni = P.ni, nj = P.nj, nk = P.nk;
@@ -305,12 +327,14 @@ __device__ __forceinline__ void advs_col(const KP &P, const AdvsArgs &a, const C
   // window: wv[0..5] = S(k-2 .. k+3)
   float wv0 = val(ks - 2), wv1 = val(ks - 1), wv2 = val(ks), wv3 = val(ks + 1), wv4 = val(ks + 2), wv5 = val(ks + 3);
   AdvLevel nx;
-  advs_load<WENO, TH>(P, a, o, ks, nx);
-  float fz_lo = 0.0f;
+  advs_load<PD, TH>(P, a, o, ks, nx);
+  float fz_lo = 0.0f, rw0 = 0.0f;
+  if (PD && ks == 1 && !a.scale) rw0 = ldo(a.rrw + P.pxy, o);
   if (ks > 1) {
     // the flux through a segment's lowest face
     float rw = ldo(a.rrw + (size_t)ks * P.pxy, o);
     if (a.scale) rw = rw * P.rf0[ks];
+    if (PD) rw0 = rw;
     const float wm = val(ks - 3);
     auto S = [=](int kk) -> float {
       const int q = kk - ks;  // -3..2
@@ -320,7 +344,7 @@ __device__ __forceinline__ void advs_col(const KP &P, const AdvsArgs &a, const C
   }
   for (int k = ks; k <= ke; k++) {
     const AdvLevel L = nx;
-    if (k < ke) advs_load<WENO, TH>(P, a, o, k + 1, nx);
+    if (k < ke) advs_load<PD, TH>(P, a, o, k + 1, nx);
     const size_t kb = (size_t)k * P.pxy;
     const float tem = sadd ? (P.th0[k] - th0r) : 0.0f;
     auto H = [=](float v) -> float { return sadd ? tem + v : v; };
@@ -365,20 +389,29 @@ __device__ __forceinline__ void advs_col(const KP &P, const AdvsArgs &a, const C
     if (k == 1) az = -fz_hi * P.rdz * P.mh[1];
     else if (k == nk) az = +fz_lo * P.rdz * P.mh[nk];
     else az = -(fz_hi - fz_lo) * P.rdz * P.mh[k];
-    if (MODE1) {
+    if (PD) {
       sto(a.advx + kb, o, ax);
       sto(a.advy + kb, o, ay);
       sto(a.advz + kb, o, az);
-    } else {
-      float st = L.st0;
-      if (TH) st = st - L.t11v * L.thtv;
-      st = st + ((ax + ay) + az + sc * L.dv) * P.rr0[k];
-      if (a.out_sten) sto(a.out_sten + kb, o, st);
-      if (a.out_new) {
-        float v = L.sv0 + a.dt * st;
-        if (a.smeps_flush && fabsf(v) < P.K.smeps) v = 0.0f;
-        sto(a.out_new + kb, o, v);
-      }
+      // pdef_dum of the three directions from what the column holds
+      const float r0s0 = P.rho0[k] * L.sv0;
+      float dx = r0s0 + a.dt * (ax + sc * (ru1 - ru0) * P.rdx);
+      float dy = r0s0 + a.dt * (ay + sc * (rv1 - rv0) * P.rdy);
+      const float dz = r0s0 + a.dt * (az + sc * (L.rw1 - rw0) * P.rdz * P.mh[k]);
+      if ((doitw && i == 1 && ru0 >= 0.0f) || (doite && i == ni && ru1 <= 0.0f)) dx = r0s0;
+      if ((doits && j == 1 && rv0 >= 0.0f) || (doitn && j == nj && rv1 <= 0.0f)) dy = r0s0;
+      const unsigned long long neg = __ballot(dx < 0.0f || dy < 0.0f || dz < 0.0f);
+      if ((threadIdx.x & 63) == 0) a.marks[((size_t)(k - 1) * nj + (j - 1)) * a.gx + ((i - 1) >> 6)] = neg;
+      rw0 = L.rw1;
+    }
+    float st = L.st0;
+    if (TH) st = st - L.t11v * L.thtv;
+    st = st + ((ax + ay) + az + sc * L.dv) * P.rr0[k];
+    if (a.out_sten) sto(a.out_sten + kb, o, st);
+    if (a.out_new) {
+      float v = L.sv0 + a.dt * st;
+      if (a.smeps_flush && fabsf(v) < P.K.smeps) v = 0.0f;
+      sto(a.out_new + kb, o, v);
     }
     fz_lo = fz_hi;
     wv0 = wv1;
@@ -398,10 +431,12 @@ __device__ __forceinline__ void advs_col(const KP &P, const AdvsArgs &a, const C
 // sten0 = thten1, thterm_div[0] = t11 and thterm_div[1] = thterm.
 // out_new, if given, receives s0 + dt*tendency with the smeps flush
 // (src/solve2.F:1416-1426, :1518-1528).
-template <bool WENO, bool SADD, bool TH, bool MODE1>
+template <bool WENO, bool SADD, bool TH, bool PD>
 static void advs_launch(cm1g_model *m, const KP &P, const AdvsArgs &a, const ColGrid &cg) {
-  launch<256>(m, col_blocks(cg), col_threads(cg),
-              [=] __device__(int bx, int, int) { advs_col<WENO, SADD, TH, MODE1>(P, a, cg, bx); });
+  // (the WENO form with marks takes 97 registers uncapped, four wavefronts a
+  // SIMD; five: 578 -> 522 us at 512 x 512 x 128.  Six for the other: no gain)
+  launch<256, PD && WENO ? 5 : 0>(m, col_blocks(cg), col_threads(cg),
+                                  [=] __device__(int bx, int, int) { advs_col<WENO, SADD, TH, PD>(P, a, cg, bx); });
 }
 
 void advs_run(cm1g_model *m, int nrk, const float *s_in, float sadd, const float *s0,
@@ -434,15 +469,14 @@ void advs_run(cm1g_model *m, int nrk, const float *s_in, float sadd, const float
   g.pdefweno = pdefweno;
   g.weps = weps;
   // compile-time variants: theta (offset form, with or without the t11
-  // term), any other scalar in the plain or the pdef (advx/advy/advz) pass
+  // term), any other scalar in the plain or the positive-definite pass
   const bool sadd_on = (sadd != 0.0f), th_on = (thterm_div != nullptr);
   using Launcher = void (*)(cm1g_model *, const KP &, const AdvsArgs &, const ColGrid &);
-  auto pick = [&](bool mode1) -> Launcher {
-    if (sadd_on && th_on && !mode1) return weno ? advs_launch<true, true, true, false> : advs_launch<false, true, true, false>;
-    if (sadd_on && !th_on && !mode1) return weno ? advs_launch<true, true, false, false> : advs_launch<false, true, false, false>;
-    if (!sadd_on && !th_on && !mode1) return weno ? advs_launch<true, false, false, false> : advs_launch<false, false, false, false>;
-    if (!sadd_on && th_on && !mode1) return weno ? advs_launch<true, false, true, false> : advs_launch<false, false, true, false>;
-    // the pdef pass: advx/advy/advz only (the t11 term is added by pdef_z)
+  auto pick = [&](bool pd) -> Launcher {
+    if (sadd_on && th_on && !pd) return weno ? advs_launch<true, true, true, false> : advs_launch<false, true, true, false>;
+    if (sadd_on && !th_on && !pd) return weno ? advs_launch<true, true, false, false> : advs_launch<false, true, false, false>;
+    if (!sadd_on && !th_on && !pd) return weno ? advs_launch<true, false, false, false> : advs_launch<false, false, false, false>;
+    if (!sadd_on && th_on && !pd) return weno ? advs_launch<true, false, true, false> : advs_launch<false, false, true, false>;
     return weno ? advs_launch<true, false, false, true> : advs_launch<false, false, false, true>;
   };
   ColGrid cg = col_grid(ni, nj, m->tile_rows);
@@ -453,16 +487,20 @@ void advs_run(cm1g_model *m, int nrk, const float *s_in, float sadd, const float
   const bool inplace = (out_new != nullptr && out_new == s_in);
   if (inplace) g.out_new = m->thb;
   if (pdef != 1) {
-    g.mode = 0;
     pick(false)(m, P, g, cg);
   } else {
     // the positive-definite pass reads the advected values themselves
     // (never the theta offset form: pdef is for moisture and tracers)
-    if (sadd != 0.0f) {
+    if (sadd != 0.0f || th_on) {
       cm1g_set_error("advs: pdef with an offset field is not supported");
       return;
     }
-    g.mode = 1;
+    // a tendency asked for may be the array its initial value stands in, which
+    // pdef_fix reads again: it is formed in a work array
+    float *const ten = g.out_sten;
+    if (ten) g.out_sten = m->sy;
+    g.marks = (unsigned long long *)m->sx;
+    g.gx = cg.gx;
     pick(true)(m, P, g, cg);
     PdefArgs pa;
     pa.rru = g.rru;
@@ -474,23 +512,30 @@ void advs_run(cm1g_model *m, int nrk, const float *s_in, float sadd, const float
     pa.advz = m->tz;
     pa.s0 = s0;
     pa.s = s_in;
-    pa.ax_out = m->sx;
-    pa.ay_out = m->sy;
     pa.sten0 = sten0;
-    pa.t11 = thterm_div;
-    pa.thterm = g.thterm;
     pa.divx = g.divx;
-    pa.out_sten = out_sten;
+    pa.marks = g.marks;
+    pa.gx = g.gx;
+    pa.out_sten = g.out_sten;
     pa.out_new = g.out_new;
     pa.dt = dt;
     pa.smeps_flush = smeps_flush;
-    launch<256>(m, dim3((ni + 63) / 64, (nj + 3) / 4, nk), dim3(64, 4, 1),
-                [=] __device__(int bx, int by, int bz) { pdef_xy(P, pa, bx, by, bz); });
-    // (a segment's start costs pdef_z five evaluations of dum: large grids
-    // stay uncut, 848 against 901 us at 1024 x 1024 x 96)
-    ColGrid cz = col_grid(ni, nj, m->tile_rows);
-    col_split(m, cz, nk, false);
-    launch<256>(m, col_blocks(cz), col_threads(cz), [=] __device__(int bx, int, int) { pdef_z(P, pa, cz, bx); });
+    // levels a workgroup: visited levels follow one another (two barriers and
+    // their loads' latency each), so a small grid takes fewer of them, down
+    // to one, until there are 4096 workgroups (eight levels against these: 64 x
+    // 64 x 40 25.6 -> 8.5 us; 301 x 227 x 63 37 -> 29 us, at 2048 37).
+    const long rows = m->plan_tiles > 0 ? m->plan_tiles : (long)cg.gx * cg.gy * cg.ty;
+    const long lev = rows / 4 * nk / 4096;
+    pa.lev = (int)(lev < 1 ? 1 : lev > PDEF_L ? PDEF_L : lev);
+    launch<256>(m, dim3((ni + 63) / 64, (nj + 3) / 4, (nk + pa.lev - 1) / pa.lev), dim3(64, 4, 1),
+                [=] __device__(int bx, int by, int bz) { pdef_fix(P, pa, bx, by, bz); });
+    if (ten) {
+      const float *w = m->sy;
+      for3(m, 1, ni, 1, nj, 1, nk, [=] __device__(int i, int j, int k) {
+        const int c = IXD(P, i, j, k);
+        ten[c] = w[c];
+      });
+    }
   }
   if (inplace) {
     // the partner now holds the new field: exchange the two buffers
