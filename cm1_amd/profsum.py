@@ -34,8 +34,10 @@ def short(name):
     if h:
         host = h.group(1).split("::")[-1]
         names = {("sound_run", "1"): "sound_coef", ("sound_run", "2"): "sound_sub",
-                 ("advs_run", "1"): "pdef_xy", ("advs_run", "2"): "pdef_z",
-                 ("cm1g_solve2", "2"): "massflux_div", ("advm_run", "1"): "ten_edges"}
+                 ("advs_run", "1"): "pdef_fix", ("cm1g_solve2", "2"): "massflux_div",
+                 ("sounde_run", "2"): "sounde_col", ("sounde_run", "3"): "sounde_col"}
+        if host == "kess_cols_run":
+            return "kess_cols"
         return names.get((host, h.group(2)), f"{host} λ{h.group(2)}")
     return body.split("(")[0]
 
