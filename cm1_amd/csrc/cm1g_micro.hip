@@ -502,9 +502,11 @@ static void fallout_run(cm1g_model *m) {
 // the workgroup, and the finished ones sit them out.
 //
 // A column marched by one lane is bound by the latency of a load per level;
-// here large grids are bound by memory (4 arrays read, 2 written).
+// here a large grid is bound by the phases of a workgroup, which follow one
+// another: the LDS of a CU holds two workgroups up to 64 levels and one above
+// (2.4 GB at 2.4 TB/s at 96 levels).
 // Measured, both passes before -> this: 64 x 64 x 40 76 -> 10 us, 301 x 227 x 63
-// 166 -> 42 us, eight 128 x 128 x 64 ensemble members in one launch 230 -> 91
+// 166 -> 42 us, eight supercell members (11 M cells) in one launch 230 -> 91
 // us, 1024 x 1024 x 96 (one workgroup per CU fits) 1.17 -> 1.05 ms.
 struct KessArgs {
   const float *rho;

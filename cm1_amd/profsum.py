@@ -43,25 +43,34 @@ def short(name):
 
 
 def trace(path):
-    rows = list(csv.DictReader(open(path)))
-    tot = sum(float(r["TotalDurationNs"]) for r in rows)
+    # the variants of a kernel that share a short name are one row
+    per = defaultdict(lambda: [0, 0.0])
+    for r in csv.DictReader(open(path)):
+        e = per[short(r["Name"])]
+        e[0] += int(r["Calls"])
+        e[1] += float(r["TotalDurationNs"])
+    tot = sum(ns for _, ns in per.values())
     print("| kernel | dispatches | total ms | avg us | share |")
     print("|---|---:|---:|---:|---:|")
-    for r in sorted(rows, key=lambda r: -float(r["TotalDurationNs"])):
-        print(f"| `{short(r['Name'])}` | {r['Calls']} | {float(r['TotalDurationNs']) / 1e6:.2f} | "
-              f"{float(r['AverageNs']) / 1e3:.1f} | {100.0 * float(r['TotalDurationNs']) / tot:.1f}% |")
+    for name, (calls, ns) in sorted(per.items(), key=lambda e: -e[1][1]):
+        print(f"| `{name}` | {calls} | {ns / 1e6:.2f} | {ns / calls / 1e3:.1f} | {100.0 * ns / tot:.1f}% |")
     print(f"\nWhole process kernel time {tot / 1e6:.1f} ms.")
 
 
 def counters(path):
-    per = defaultdict(list)
+    """Values per kernel, the variants that share a short name together, and the model's own kernels."""
+    per, model = defaultdict(list), set()
     for r in csv.DictReader(open(path)):
-        per[r["Kernel_Name"]].append(float(r["Counter_Value"]))
-    return per
+        n = r["Kernel_Name"]
+        if "k_one" in n:
+            n = short(n)
+            model.add(n)
+        per[n].append(float(r["Counter_Value"]))
+    return per, model
 
 
 def pmc(fpath, wpath):
-    f, w = counters(fpath), counters(wpath)
+    (f, model), (w, _) = counters(fpath), counters(wpath)
     gib = 1024.0 ** 3
     # calibration: the copies of 1 GiB the bench ran first
     cf = [v for n, vs in f.items() if "copyBuffer" in n for v in vs if v * 1024 > 0.25 * gib]
@@ -73,11 +82,11 @@ def pmc(fpath, wpath):
           f"(KiB counters x 1024).\n")
     rows = []
     for n in f:
-        if n not in w or "k_one" not in n:
+        if n not in w or n not in model:
             continue
         rd = sum(f[n]) / len(f[n]) * 1024 * rf / 1e9
         wr = sum(w[n]) / len(w[n]) * 1024 * rw / 1e9
-        rows.append((short(n), len(f[n]), rd, wr))
+        rows.append((n, len(f[n]), rd, wr))
     print("| kernel | dispatches | read GB | write GB | traffic GB / dispatch |")
     print("|---|---:|---:|---:|---:|")
     for n, c, rd, wr in sorted(rows, key=lambda r: -(r[2] + r[3])):
