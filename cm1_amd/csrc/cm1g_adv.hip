@@ -7,6 +7,7 @@
 // Every flux is evaluated with the reference's operation order in FP32
 // without contraction, so results are bitwise those of the reference.
 #include "cm1g_adv_common.h"
+#include "cm1g_pdef_visit.h"
 
 // ------------------------------------------------------------------ pdef
 // The positive-definite correction (pdscheme=1, src/pdef.F:15-581), per
@@ -70,14 +71,6 @@ __device__ __forceinline__ float pdef_dum(const KP &P, int dir, const float *vel
     if (P.nbc == 2 && P.ibn == 1 && j == P.nj && hi <= 0.0f) d = P.rho0[k] * s0[c];
   }
   return d;
-}
-
-// halo point of the horizontal fill (bcs, src/bc.F:180-364) -> the
-// interior point whose value it holds
-__device__ __forceinline__ int pdef_wrap(int m, int n, bool periodic) {
-  if (m < 1) return periodic ? max(m + n, 1) : 1;
-  if (m > n) return periodic ? min(m - n, n) : n;  // (past the halo: any point)
-  return m;
 }
 
 // the corrected tendency of one cell from dum at offsets -2..2 along the
@@ -159,9 +152,9 @@ __device__ __forceinline__ void pdef_fix(const KP &P, const PdefArgs &a, int bx,
       if (k >= 1 && k <= nk && a.marks[((size_t)(k - 1) * nj + (jj - 1)) * a.gx + bx])
         m = (r == 0 || r == 5) ? (b >= 0 ? 1u << b : 0u) : (7u << (b + 1)) >> 2;
     } else if (t < own + 8 * lev) {
-      // columns i0-1 and i0+64 of rows j0..j0+3
+      // the columns on either side, rows j0..j0+3
       const int u = t - own, b = u >> 3, k = k0 + b;
-      const int ii = pdef_wrap((u & 1) ? i0 + 64 : i0 - 1, ni, perx);
+      const int ii = pdef_side_col(i0, ni, u & 1, perx);
       const int jj = pdef_wrap(j0 + ((u >> 1) & 3), nj, pery);
       if (k <= nk &&
           ((a.marks[((size_t)(k - 1) * nj + (jj - 1)) * a.gx + ((ii - 1) >> 6)] >> ((ii - 1) & 63)) & 1ULL))
