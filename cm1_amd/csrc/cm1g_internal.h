@@ -4,6 +4,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <type_traits>
 #include <string>
 #include <vector>
@@ -137,10 +138,12 @@ struct cm1g_model {
   // pinned host staging of cm1g_put_array / cm1g_get_array
   float *pin;
   size_t pin_cap;
-  // pinned chunks that box_move's kernels read and write from the device,
-  // and the event of each chunk's last kernel (allocated on first use)
+  // pinned chunks that box_move's kernels read and write from the device (at
+  // most 8 MiB, allocated on first use, freed with the model), and the event
+  // of each chunk's last kernel; one move at a time holds them (xfer_mu)
   float *xfer[2];
   hipEvent_t xfer_ev[2];
+  std::mutex xfer_mu;
 };
 
 // zeroed device allocation of n floats

@@ -422,8 +422,10 @@ __global__ void __launch_bounds__(256) k_box_unpack(float *__restrict__ dev, int
 }
 
 // dev: the box's first element; rows of w = ni + 7 floats.  Waits until the
-// host array is read (written) and the device array written (read).
+// host array is read (written) and the device array written (read).  Threads
+// that move fields of one model take turns: its chunks serve one move.
 static int box_move(cm1g_model *m, float *dev, void *host, bool to_host) {
+  const std::lock_guard<std::mutex> hold(m->xfer_mu);
   const int w = m->P.ni + 7, pitch = m->P.px;
   const size_t total = (size_t)w * (size_t)m->P.py * (size_t)(m->P.nk + 3);  // the same for every field
   const size_t nch = (total + XFER_FLOATS - 1) / XFER_FLOATS;

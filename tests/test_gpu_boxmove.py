@@ -20,3 +20,32 @@ def test_put_get_round_trip(require_gpu, ni, nj, nk):
         assert np.array_equal(m.get("dum1"), a)
         assert np.array_equal(m.get("dum2"), b)
     m.close()
+
+
+@pytest.mark.parametrize("ni,nj,nk", [(57, 40, 20), (401, 230, 70)])
+def test_fetches_from_several_threads(require_gpu, ni, nj, nk):
+    """Fields of one model fetched (and one stored again) by threads side by
+    side: every thread gets its own field's bytes."""
+    import threading
+
+    m = model.Model(model.make_config(ni=ni, nj=nj, nk=nk))
+    rng = np.random.default_rng(ni)
+    want = {n: rng.standard_normal((m.pz, m.py, ni + 7)).astype(np.float32) for n in ("dum1", "dum2", "dum3")}
+    for n, a in want.items():
+        m.put(n, a)
+    bad = []
+
+    def work(n, store):
+        for q in range(10):
+            if not np.array_equal(m.get(n), want[n]):
+                bad.append((n, q))
+            if store:
+                m.put(n, want[n])
+
+    threads = [threading.Thread(target=work, args=(n, n == "dum3")) for n in want]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    m.close()
+    assert not bad, bad
