@@ -51,6 +51,7 @@ __device__ __host__ __forceinline__ int IX2D(const KP &P, int i, int j) {
 enum { BC_S = 0, BC_P = 1, BC_U = 2, BC_V = 3, BC_W1 = 4, BC_W0 = 5 };
 
 struct cm1g_model {
+  int dev;  // the device that was current in cm1g_create: the model's arrays and stream are on it
   cm1g_config c;
   KP P;                         // kernel parameters (device pointers inside)
   float *f[CM1G_NFIELDS];       // 3-D device fields
@@ -144,6 +145,21 @@ struct cm1g_model {
   float *xfer[2];
   hipEvent_t xfer_ev[2];
   std::mutex xfer_mu;
+};
+
+// Makes a device current for a scope (the null stream is the current
+// device's), and the caller's again after it.
+struct DeviceScope {
+  int prev = -1;
+  explicit DeviceScope(int dev) {
+    int d = dev;
+    if (hipGetDevice(&d) == hipSuccess && d != dev && hipSetDevice(dev) == hipSuccess) prev = d;
+  }
+  ~DeviceScope() {
+    if (prev >= 0) hipSetDevice(prev);
+  }
+  DeviceScope(const DeviceScope &) = delete;
+  DeviceScope &operator=(const DeviceScope &) = delete;
 };
 
 // zeroed device allocation of n floats

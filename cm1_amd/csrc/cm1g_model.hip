@@ -136,7 +136,7 @@ extern "C" int cm1g_create(const cm1g_config *cfg, cm1g_model **out) {
   const int pz = cfg->nk + 3;
   m->ntot = (size_t)P.pxy * pz;
   int rc = 0;
-  if (hipStreamCreate(&m->stream) != hipSuccess) {
+  if (hipGetDevice(&m->dev) != hipSuccess || hipStreamCreate(&m->stream) != hipSuccess) {
     cm1g_set_error("hipStreamCreate failed");
     delete m;
     return CM1G_E_HIP;
@@ -401,9 +401,10 @@ static float *box_origin(const cm1g_model *m, int id) { return m->f[id] + (CM1G_
 // of) pinned host memory, in two chunks of 4 MiB that alternate between the
 // kernel and the host's copy to or from the caller's array: a get of 64 x 64
 // x 40 0.07 ms, of 301 x 227 x 63 1.8 ms (0.8 ms into memory the host has
-// touched), of 1024 x 1024 x 96 32 ms.  The kernels run on the null stream, as
-// the copy did: after everything queued on any of the library's streams, and
-// before what is queued on them next.
+// touched), of 1024 x 1024 x 96 32 ms.  The kernels run on the null stream of
+// the model's device, as the copy did whichever device was current: after
+// everything queued on any of the library's streams there, and before what is
+// queued on them next.
 constexpr size_t XFER_FLOATS = (size_t)1 << 20;
 
 __global__ void __launch_bounds__(256) k_box_pack(const float *__restrict__ dev, int pitch, int w, size_t first,
@@ -426,6 +427,7 @@ __global__ void __launch_bounds__(256) k_box_unpack(float *__restrict__ dev, int
 // that move fields of one model take turns: its chunks serve one move.
 static int box_move(cm1g_model *m, float *dev, void *host, bool to_host) {
   const std::lock_guard<std::mutex> hold(m->xfer_mu);
+  const DeviceScope on(m->dev);
   const int w = m->P.ni + 7, pitch = m->P.px;
   const size_t total = (size_t)w * (size_t)m->P.py * (size_t)(m->P.nk + 3);  // the same for every field
   const size_t nch = (total + XFER_FLOATS - 1) / XFER_FLOATS;

@@ -49,3 +49,17 @@ def test_fetches_from_several_threads(require_gpu, ni, nj, nk):
         t.join()
     m.close()
     assert not bad, bad
+
+
+def test_move_with_another_device_current(require_gpu):
+    import torch
+
+    if torch.cuda.device_count() < 2:
+        pytest.skip("needs two GPUs")
+    m = model.Model(model.make_config(ni=57, nj=40, nk=20))
+    a = np.random.default_rng(3).standard_normal((m.pz, m.py, 64)).astype(np.float32)
+    with torch.cuda.device(1):
+        m.put("dum1", a)
+        assert np.array_equal(m.get("dum1"), a)
+        assert torch.cuda.current_device() == 1
+    m.close()
