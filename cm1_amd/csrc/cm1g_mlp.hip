@@ -142,8 +142,11 @@ __device__ __forceinline__ void sum16(const floatx4 (&z)[8], float &r0, float &r
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// acc (pre-activations) -> x = SiLU in BF16, d = SiLU'.  The derivative uses
-// the sigmoid the activation was formed with.
+// acc (pre-activations) -> x = SiLU in BF16, in inference's form, d = SiLU'.
+// The derivative reaches the bias gradients unrounded, so its sigmoid is a
+// single-precision one: the hardware forms' error, which BF16 activations do
+// not show, grows with |z| (3e-6 of the derivative at z = -80, 5e-7 here; k_train
+// 37 us with them, 54 so).
 __device__ __forceinline__ void silu_both(const floatx4 (&acc)[1][8], bf16x4 (&x)[1][8], floatx4 (&d)[8]) {
 #pragma unroll
   for (int nt = 0; nt < 8; nt++) {
@@ -151,12 +154,12 @@ __device__ __forceinline__ void silu_both(const floatx4 (&acc)[1][8], bf16x4 (&x
 #pragma unroll
     for (int t = 0; t < 4; t++) {
       const float z = acc[0][nt][t];
-      const float sg = __builtin_amdgcn_rcpf(1.0f + __expf(-z));
-      h[t] = z * sg;
+      h[t] = silu_f(z);
+      const float sg = 1.0f / (1.0f + expf(-z));
       d[nt][t] = sg * (1.0f + z * (1.0f - sg));
     }
     x[0][nt] = mlp_pack(h[0], h[1], h[2], h[3]);
-    if (nt & 1) __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 // acc += W x, 128 x 128 in four 32-deep steps (one step's weight fragments at
@@ -181,8 +184,8 @@ __device__ __forceinline__ void mlp_prod(floatx4 (&acc)[1][8], const bf16x4 (&x)
 // holds.  The operands of the weight gradients (the layers' inputs and
 // pre-activation gradients, BF16) leave through a small LDS transpose, 25.6 KB
 // a group; bias gradients are summed from the FP32 gradients.  Bound by the
-// vector unit (exponential and reciprocal per hidden value) and by those
-// stores: 40 us for 65536 rows, k_wgrad 32, k_grad_final 7; the separate
+// vector unit (two exponentials, a reciprocal and a division per hidden value)
+// and by those stores: 54 us for 65536 rows, k_wgrad 32, k_grad_final 7; the separate
 // products and element-wise passes they replace (FP32 activations through
 // memory, column sums by one workgroup each) took 1390 us.
 __global__ void __launch_bounds__(512) k_train(const MlpPack *__restrict__ pk, const float *__restrict__ prm,

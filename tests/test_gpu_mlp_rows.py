@@ -41,3 +41,37 @@ def test_gradients_and_forward(require_gpu, rows):
         assert rel(y, R.forward(p, x.astype(np.float64), rnd=True)[0]) < TOL
         net.train(xd, td, steps=1, batch=rows)
     net.close()
+
+
+def test_silu_derivative_in_single_precision(require_gpu):
+    """One row through a network whose third layer sees its biases alone (all
+    hidden weights 0) and whose output weights and output error make that
+    layer's bias gradient SiLU's derivative at those biases, unrounded.
+
+    Tolerance, with u = 2^-24: exp within an ulp (2u), the sum and the division
+    rounded (u each), so the sigmoid s is within 4u of itself; q = 1 + z(1 - s)
+    takes in 4us|z| from s and 2u|z| from two roundings, and rounds itself (u
+    |q|), as the product s q does."""
+    import torch
+    z = np.linspace(-80.0, 20.0, R.NH).astype(np.float32)
+    z[-1] = 0.0
+    net = S.Net(seed=1)
+    w = {name: np.zeros(shape) for name, shape in R.SIZES}
+    w["b3"] = z
+    w["W4"][:, 0] = 1.0
+    net.set_params(R.pack(w))
+    x = torch.ones((1, 8), device="cuda")
+    t = net.forward(x)
+    t[0, 0] -= 2.0  # 2 (y - t) / 4 = 1
+    _, g = net.loss_grad(x, t, want_grad=True)
+    at = sum(int(np.prod(s)) for _, s in R.SIZES[:5])
+    d = g[at:at + R.NH].astype(np.float64)
+    net.close()
+    z = z.astype(np.float64)
+    s = 1.0 / (1.0 + np.exp(-z))
+    # (z < 0: 1 - s without its cancellation)
+    q = 1.0 + z / (1.0 + np.exp(z))
+    u = 2.0 ** -24
+    tol = s * (4 * u * np.abs(q) + np.abs(z) * (4 * u * s + 2 * u) + 2 * u * np.abs(q)) + 2.0 ** -149
+    assert d[-1] == 0.5
+    assert (np.abs(d - s * q) <= tol).all(), np.max(np.abs(d - s * q) / tol)
