@@ -75,8 +75,9 @@ __global__ void __launch_bounds__(256) k_pack(const float *__restrict__ p, MlpPa
 // the summed index).
 constexpr int T_X = 0, T_H1 = 1, T_H2 = 9, T_H3 = 17, T_D1 = 25, T_D2 = 33, T_D3 = 41, T_DY = 49, T_N = 50;
 constexpr int T_ELEM = 256;
-constexpr int TP_N = 392;  // one workgroup's partial sums: 3 x 128 + 4 bias gradients, the loss
+constexpr int TP_N = 392;  // one workgroup's partial sums: 3 x 128 + 4 bias gradients, the loss (a double)
 constexpr int TP_LOSS = 3 * MLP_H + MLP_OUT;
+static_assert(TP_N % 2 == 0 && TP_LOSS % 2 == 0 && TP_LOSS + 2 <= TP_N, "the loss's place");
 
 // (the caller's rows may start on any float)
 typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -198,7 +199,8 @@ __global__ void __launch_bounds__(512) k_train(const MlpPack *__restrict__ pk, c
   mlp_stage_bias(S.b, prm, tid);
   __syncthreads();
   const int64_t count = rows * MLP_OUT;
-  float lsum = 0.0f, bs[3][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}, {0.0f, 0.0f}};
+  double lsum = 0.0;  // (a lane adds 2048 squares at the largest batch)
+  float bs[3][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}, {0.0f, 0.0f}};
   floatx4 b4 = {0.0f, 0.0f, 0.0f, 0.0f};
   const floatx4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
   for (int64_t g = (int64_t)blockIdx.x * MLP_WAVES + w; g < ngroups; g += (int64_t)gridDim.x * MLP_WAVES) {
@@ -254,7 +256,7 @@ __global__ void __launch_bounds__(512) k_train(const MlpPack *__restrict__ pk, c
       for (int t = 0; t < 4; t++) {
         const float e = (y[t] + S.b[3 * MLP_H + t]) - tv[t];
         dy[t] = 2.0f * e / (float)count;
-        lsum += e * e;
+        lsum += (double)e * (double)e;
       }
       b4 += dy;
     }
@@ -309,6 +311,7 @@ __global__ void __launch_bounds__(512) k_train(const MlpPack *__restrict__ pk, c
   }
   __syncthreads();
   float *red = (float *)&S.tr[0][0][0];  // 8 x TP_N floats fit the transposes' space
+  static_assert(offsetof(TrainLds, tr) % 8 == 0, "k_train: the loss's place");
   static_assert(MLP_WAVES * TP_N * sizeof(float) <= sizeof(S.tr), "k_train: partial sums");
   const int f = 2 * (l & 15);  // this lane's two values of sum16: 16nt + 4(l/16) + t
 #pragma unroll
@@ -320,13 +323,17 @@ __global__ void __launch_bounds__(512) k_train(const MlpPack *__restrict__ pk, c
     }
   if (l == 0) {
     for (int t = 0; t < 4; t++) red[w * TP_N + 3 * MLP_H + t] = b4[t];
-    red[w * TP_N + TP_LOSS] = lsum;
+    *(double *)(red + w * TP_N + TP_LOSS) = lsum;
   }
   __syncthreads();
-  if (tid <= TP_LOSS) {
+  if (tid < TP_LOSS) {
     float s = 0.0f;
     for (int q = 0; q < MLP_WAVES; q++) s += red[q * TP_N + tid];
     part[(int64_t)blockIdx.x * TP_N + tid] = s;
+  } else if (tid == TP_LOSS) {
+    double s = 0.0;
+    for (int q = 0; q < MLP_WAVES; q++) s += *(const double *)(red + q * TP_N + tid);
+    *(double *)(part + (int64_t)blockIdx.x * TP_N + tid) = s;
   }
 }
 
@@ -426,7 +433,7 @@ __global__ void __launch_bounds__(256) k_grad_final(const float *__restrict__ wp
   if (blockIdx.x == 0) {
     __shared__ double d[256];
     const int q = (int)threadIdx.x;  // nwg <= 256
-    const double t = block_reduce256(q < nwg ? (double)part[(int64_t)q * TP_N + TP_LOSS] : 0.0, d, OpAdd());
+    const double t = block_reduce256(q < nwg ? *(const double *)(part + (int64_t)q * TP_N + TP_LOSS) : 0.0, d, OpAdd());
     if (q == 0) loss[0] = (float)(t / (double)count);
   }
 }

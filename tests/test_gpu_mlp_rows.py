@@ -75,3 +75,37 @@ def test_silu_derivative_in_single_precision(require_gpu):
     tol = s * (4 * u * np.abs(q) + np.abs(z) * (4 * u * s + 2 * u) + 2 * u * np.abs(q)) + 2.0 ** -149
     assert d[-1] == 0.5
     assert (np.abs(d - s * q) <= tol).all(), np.max(np.abs(d - s * q) / tol)
+
+
+def test_loss_adds_up_over_many_groups(require_gpu):
+    """All weights 0: every squared error is that of the target, whose sum over
+    a wavefront's many groups would drift in single precision.  Tolerance: a
+    square, three sums of a sample's four and the result rounded to single."""
+    import torch
+    rows, c = 2 ** 21 + 3, np.float32(0.7325)
+    drift = np.cumsum(np.full(256, c * c, np.float32), dtype=np.float32)[-1] / (256 * float(c) ** 2) - 1.0
+    assert abs(drift) > 1.0e-6
+    net = S.Net(seed=2)
+    net.set_params(np.zeros(R.NPARAM, np.float32))
+    x = torch.ones((rows, 8), device="cuda")
+    t = torch.full((rows, 4), float(c), device="cuda")
+    loss = net.loss_grad(x, t)
+    net.close()
+    assert abs(loss / float(c) ** 2 - 1.0) <= 5 * 2.0 ** -24
+
+
+def test_many_groups_a_wavefront(require_gpu):
+    """Eight 16-sample groups for most wavefronts, a last one that is not full."""
+    import torch
+    rows = 2 ** 18 + 5
+    rng = np.random.default_rng(rows)
+    net = S.Net(seed=3)
+    x = rng.standard_normal((rows, 8)).astype(np.float32)
+    t = rng.standard_normal((rows, 4)).astype(np.float32)
+    loss, g = net.loss_grad(torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda(), want_grad=True)
+    loss_r, g_r = R.loss_grad(net.params().astype(np.float64), x.astype(np.float64), t.astype(np.float64), rnd=True)
+    net.close()
+    assert abs(loss - loss_r) <= TOL * loss_r, (loss, loss_r)
+    offs = np.cumsum([0] + [int(np.prod(s)) for _, s in R.SIZES])
+    for (name, _), a, b in zip(R.SIZES, offs[:-1], offs[1:]):
+        assert rel(g[a:b], g_r[a:b]) < TOL, name
