@@ -679,15 +679,20 @@ static void slab_launch(cm1g_model *m, int v, dim3 grd, dim3 blk, const KP &P, c
   else a.first ? slab_go<4, true>(m, grd, blk, P, a, sg) : slab_go<4, false>(m, grd, blk, P, a, sg);
 }
 
-// Which kernel runs the substep (0: sound_sub, one thread per column, for
-// columns too deep for a workgroup's LDS and fields of 4 GiB and more).  Up
-// to 64 levels 8 per wavefront, unless the grid is too small to fill the
-// chip: under 1024 tiles (four workgroups per CU) 4 per wavefront put more
-// wavefronts on a column.
+// Which kernel runs the substep (0: sound_sub, one thread per column).
+// sound_sub takes columns too deep for a workgroup's LDS, fields of 4 GiB and
+// more, and shallow columns of a wide grid: a slab workgroup is then one to
+// three wavefronts, and its LDS lets a CU hold three of them, while a thread
+// per column fills the chip.  Six substeps, sound_sub / slabs of 8 levels:
+// 1024 x 1024 x 7 1127 / 1778 us, x 16 2490 / 2805, x 20 3150 / 3188, x 24
+// 3823 / 3535; 512 x 512 x 9 359 / 529, x 20 841 / 923; 100 x 2000 x 18 761 / 901;
+// 512 x 256 x 8 225 / 280, x 12 291 / 316, x 16 369 / 349; 512 x 384 x 16 547 /
+// 526; 384 x 256 x 8 192 / 218, x 12 257 / 246.
 static int slab_variant(const cm1g_model *m) {
   const int nk = m->plan_nk > m->P.nk ? m->plan_nk : m->P.nk;
   const long tiles = m->plan_tiles > 0 ? m->plan_tiles : (long)((m->P.ni + 63) / 64) * m->P.nj;
   if (nk > 192 || m->ntot >= ((size_t)1 << 30)) return 0;
+  if (tiles >= (nk <= 12 ? 2048 : 3840) && nk <= 20) return 0;
   if (nk <= 64) return tiles < 1024 ? 1 : 2;
   return nk <= 96 ? 3 : 4;
 }

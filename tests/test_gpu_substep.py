@@ -37,6 +37,32 @@ def test_substep_edges_match_oracle(require_gpu, ni, nj, nk, nsound, bc):
 
 
 @pytest.mark.parametrize("ni,nj,nk,nsound,bc", [
+    (64, 2047, 7, 4, 1),    # slabs, one tile short of the line
+    (64, 2048, 7, 4, 2),    # one thread per column
+    (65, 1024, 6, 2, 1),    # the fewest levels, single-substep stages
+    (64, 2048, 12, 6, 1),
+    (64, 2048, 13, 6, 2),   # slabs
+    (130, 1279, 20, 6, 1),  # slabs, three tiles short of the second line
+    (130, 1280, 20, 6, 2),  # one thread per column
+    (130, 1280, 21, 4, 1),  # slabs
+])
+def test_shallow_wide_grids_match_oracle(require_gpu, ni, nj, nk, nsound, bc):
+    """Either side of the rule that sends shallow columns of wide grids to the
+    one-thread-per-column kernel."""
+    cfgd, cols, fields = case(ni=ni, nj=nj, nk=nk, nsound=nsound, bc=bc, dz=15000.0 / nk, dt=0.4 * nsound, amp=2.0)
+    g = make_gpu(cfgd, cols, fields)
+    o = make_oracle(cfgd, cols, fields)
+    for n in (1, 1):  # the first step and one that starts from exchanged buffers
+        g.step(n)
+        o.step(n)
+        for name, stag in PROG + [("ppx", None)]:
+            a = g.interior(name, stag)
+            b = interior(o.f(name), nk, nj, ni, stag)
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), name
+    g.close()
+
+
+@pytest.mark.parametrize("ni,nj,nk,nsound,bc", [
     (8, 8, 6, 2, 2),       # single-substep stages
     (9, 8, 7, 5, 2),       # an odd count
     (65, 9, 30, 7, 1),
