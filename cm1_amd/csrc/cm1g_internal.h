@@ -390,8 +390,9 @@ inline ColGrid col_grid_box(int ilo, int ihi, int jlo, int jhi, int ty = 4) {
 // by a wavefront of its own that first forms what the level below its first
 // one would have left it (about two levels' work).  A column's levels take
 // their loads' latency one after the other (1 to 2 us a level), so a grid
-// with few columns is cut until 16384 wavefronts run (16 per SIMD), with no
-// segment under 4 levels.  Measured per step, uncut -> cut: 64 x 64 x 40 2.57
+// with few columns is cut until 16384 wavefronts run (16 per SIMD), into at
+// most nk/4 segments; their length is rounded up, so the last one is shorter,
+// down to one level (nk = 21: 5, 5, 5, 5, 1).  Measured per step, uncut -> cut: 64 x 64 x 40 2.57
 // -> 1.10 ms, 301 x 227 x 63 4.9 -> 4.0 ms; 4096 or 8192 wavefronts 3 to 10%
 // slower at 301 x 227 x 63 and 512 x 512 x 128, at least 8 levels 10% slower
 // at 64 x 64 x 40, 3 levels within 3%.  With `even`, larger grids are cut
@@ -507,6 +508,7 @@ void advs_run(cm1g_model *m, int nrk, const float *s_in, float sadd, const float
               int pdef, int pdefweno, float dt, double weps, int smeps_flush);
 // acoustic (cm1g_sound.hip)
 void sound_run(cm1g_model *m, int nrk, bool fold1 = false);
+const char *sound_kernel(const cm1g_model *m);  // the kernel its substeps run
 void sounde_run(cm1g_model *m, int nrk, bool fold1 = false);
 void getdiv_both(cm1g_model *m, int want_t11, int want_divx = 1, float *div = nullptr);
 void scale_mass_fluxes(cm1g_model *m);

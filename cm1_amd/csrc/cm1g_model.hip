@@ -1736,7 +1736,7 @@ extern "C" int cm1g_ktimer_stop(cm1g_model *m, double *total_ms, int64_t *launch
     // piadv, pk1, pk2, qk, mm read (11).  The kernel evaluates pk1, pk2, qk
     // and mm on the fly instead of reading them, so it touches 23 of them.
     fields = 27.0;
-    nm = "sound_sub";
+    nm = sound_kernel(m);
   }
   *total_ms = tot;
   *launches = (int64_t)npair;

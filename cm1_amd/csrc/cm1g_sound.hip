@@ -392,7 +392,7 @@ __device__ __forceinline__ void sound_sub(const KP &P, const SubArgs &a, const C
 // for sound_sub; 7.5 + 2.8 GB to and from memory (10.7 + 4.2 before), 5.0
 // TB/s, what a plain copy reaches.  On small grids a column's levels are in
 // flight together instead of one after the other: 256 x 256 x 64 104 us
-// against 201, 64 x 64 x 40 see slab_variant.  12 levels per wavefront is
+// against 201, 64 x 64 x 40 20 us against 85.  12 levels per wavefront is
 // the most that 128 registers hold (two workgroups of 8 wavefronts per CU):
 // 6 and 8 levels (one workgroup of 16 or 12) 2.50 and 2.48 ms, 16 levels
 // 3.04 ms; loading the next level's centre values ahead, paid for with a
@@ -688,6 +688,13 @@ static void slab_launch(cm1g_model *m, int v, dim3 grd, dim3 blk, const KP &P, c
 // 3823 / 3535; 512 x 512 x 9 359 / 529, x 20 841 / 923; 100 x 2000 x 18 761 / 901;
 // 512 x 256 x 8 225 / 280, x 12 291 / 316, x 16 369 / 349; 512 x 384 x 16 547 /
 // 526; 384 x 256 x 8 192 / 218, x 12 257 / 246.
+// Up to 64 levels 8 per wavefront, and under 1024 tiles (four workgroups per
+// CU) 4, which put more wavefronts on a column.  Six substeps, 4 / 8 levels:
+// 64 x 64 x 40 122 / 161 us, x 64 160 / 191; 256 x 128 x 20 148 / 170, but x 40
+// 261 / 218; 256 x 256 x 24 247 / 288, x 64 817 / 658.  Above 64 levels there are
+// 12 per wavefront for any grid: a workgroup's 16 wavefronts of 4 levels end
+// there, and fewer than 12 lost on the large grid (above); on a small one only
+// sound_sub was compared (64 x 64 x 96 1266 us, with 12 levels 247).
 static int slab_variant(const cm1g_model *m) {
   const int nk = m->plan_nk > m->P.nk ? m->plan_nk : m->P.nk;
   const long tiles = m->plan_tiles > 0 ? m->plan_tiles : (long)((m->P.ni + 63) / 64) * m->P.nj;
@@ -696,6 +703,8 @@ static int slab_variant(const cm1g_model *m) {
   if (nk <= 64) return tiles < 1024 ? 1 : 2;
   return nk <= 96 ? 3 : 4;
 }
+
+const char *sound_kernel(const cm1g_model *m) { return slab_variant(m) ? "sound_slab" : "sound_sub"; }
 
 // the arguments that do not change over a stage, and its substep count
 static void sub_args(cm1g_model *m, int nrk, SubArgs &a, int *nloop) {

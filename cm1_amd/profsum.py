@@ -27,7 +27,7 @@ def short(name):
         return f"{f.group(1)}<{f.group(2).split('::')[-1]} λ{f.group(3)}>"
     t = re.match(r"(\w+)<([^>]*)>\(", body)
     if t and t.group(1) == "slab_go":
-        return "sound_sub"
+        return "sound_slab"
     if t and t.group(1) in ("advs_launch", "advm_launch"):
         return {"advs_launch": "advs_col", "advm_launch": "advm_col"}[t.group(1)] + f"<{t.group(2)}>"
     h = re.match(r"([\w:]+)(?:\(.*?\))?::\{lambda\(int, int(?:, int)?\)#(\d+)\}", body)
@@ -94,8 +94,8 @@ def pmc(fpath, wpath):
             continue
         print(f"| `{n}` | {c} | {rd:.3f} | {wr:.3f} | {rd + wr:.3f} |")
     for n, c, rd, wr in rows:
-        if n == "sound_sub":
-            print(f"\ntraffic sound_sub bytes_per_launch={(rd + wr) * 1e9:.1f}")
+        if n in ("sound_slab", "sound_sub"):
+            print(f"\ntraffic {n} bytes_per_launch={(rd + wr) * 1e9:.1f}")
 
 
 if __name__ == "__main__":

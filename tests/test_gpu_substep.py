@@ -90,3 +90,17 @@ def test_explicit_substep_matches_oracle(require_gpu, ni, nj, nk, nsound, bc, he
             b = interior(o.f(name), nk, nj, ni, stag)
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (n, name)
     g.close()
+
+
+@pytest.mark.parametrize("nk,kernel", [(40, "sound_slab"), (193, "sound_sub")])
+def test_timer_names_the_kernel_that_runs(require_gpu, nk, kernel):
+    import ctypes as C
+    from cm1_amd import _native as N
+    cfgd, cols, fields = case(ni=8, nj=8, nk=nk, dz=15000.0 / nk, dt=2.0, amp=2.0)
+    g = make_gpu(cfgd, cols, fields)
+    N.check(g.L.cm1g_ktimer_start(g.h, N.KT_SOUND_SUBSTEP), "cm1g_ktimer_start")
+    g.step(1)
+    ms, n, b, name = C.c_double(), C.c_int64(), C.c_double(), C.create_string_buffer(64)
+    N.check(g.L.cm1g_ktimer_stop(g.h, C.byref(ms), C.byref(n), C.byref(b), name, 64), "cm1g_ktimer_stop")
+    assert name.value.decode() == kernel and n.value == 2 + 3 + 6
+    g.close()
