@@ -115,3 +115,20 @@ def test_mismatched_members_refused(require_gpu):
     assert np.array_equal(a.get("ua"), before)
     a.step(1)
     e.close()
+
+
+def test_shallow_members_take_the_ensembles_substep_kernel(require_gpu):
+    """Members whose tiles together reach the line where shallow columns go to
+    the one-thread-per-column substep, while each alone stays below it."""
+    cases = [case(ni=ni, nj=nj, nk=nk, dz=15000.0 / nk, dt=4.0, amp=2.0, seed=nk)
+             for ni, nj, nk in ((64, 900, 8), (130, 300, 12), (24, 400, 6))]
+    ens_models = [make_gpu(*c) for c in cases]
+    solo = [make_gpu(*c) for c in cases]
+    e = model.Ensemble(ens_models)
+    for _ in range(2):
+        e.step(1)
+        for s in solo:
+            s.step(1)
+        e.sync()
+        check_equal(ens_models, solo, NAMES)
+    e.close()
