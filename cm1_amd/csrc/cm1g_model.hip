@@ -400,11 +400,11 @@ static float *box_origin(const cm1g_model *m, int id) { return m->f[id] + (CM1G_
 // 64 x 64 x 40).  Here a kernel packs (or unpacks) the rows straight into (out
 // of) pinned host memory, in two chunks of 4 MiB that alternate between the
 // kernel and the host's copy to or from the caller's array: a get of 64 x 64
-// x 40 0.07 ms, of 301 x 227 x 63 1.8 ms (0.8 ms into memory the host has
-// touched), of 1024 x 1024 x 96 32 ms.  The kernels run on the null stream of
-// the model's device, as the copy did whichever device was current: after
-// everything queued on any of the library's streams there, and before what is
-// queued on them next.
+// x 40 0.05 ms, of 301 x 227 x 63 1.9 ms (0.8 ms into memory the host has
+// touched; a put 0.7 ms), of 1024 x 1024 x 96 32 ms.  The kernels run on the
+// null stream of the model's device, as the copy did whichever device was
+// current: after everything queued on any of the library's streams there, and
+// before what is queued on them next.
 constexpr size_t XFER_FLOATS = (size_t)1 << 20;
 
 __global__ void __launch_bounds__(256) k_box_pack(const float *__restrict__ dev, int pitch, int w, size_t first,
