@@ -1009,11 +1009,48 @@ __device__ __forceinline__ void sounde_col(const KP &P, const SubArgs &a, const 
   }
 }
 
+// The part of those copies that lies outside the points the substeps write:
+// point r of the border i = 0, ni+1 or j = 0, nj+1 at level k.  rru, rrv, rrw
+// are 0, and u3d, v3d the state's, at i = 0 and j = 0; w3d and pp3d are the
+// state's on the whole border (copy: where the reference copies).
+struct SoundeBorder {
+  float *u, *v, *w, *p, *rru, *rrv, *rrw;
+  const float *ua, *va, *wa, *ppi;
+  int npts, copy;
+};
+__device__ __forceinline__ void sounde_border(const KP &P, const SoundeBorder &b, int q) {
+  const int k = 1 + q / b.npts, ni = P.ni, nj = P.nj;
+  if (k > P.nk) return;
+  int r = q % b.npts, i, j;
+  if (r < 2 * (ni + 2)) {
+    j = (r < ni + 2) ? 0 : nj + 1;
+    i = (r < ni + 2) ? r : r - (ni + 2);
+  } else {
+    r -= 2 * (ni + 2);
+    i = (r < nj) ? 0 : ni + 1;
+    j = 1 + ((r < nj) ? r : r - nj);
+  }
+  const int c = IXD(P, i, j, k);
+  if (i == 0 || j == 0) {
+    b.rru[c] = 0.0f;
+    b.rrv[c] = 0.0f;
+    b.rrw[c] = 0.0f;
+    if (b.copy) {
+      b.u[c] = b.ua[c];
+      b.v[c] = b.va[c];
+    }
+  }
+  if (b.copy) {
+    b.w[c] = b.wa[c];
+    b.p[c] = b.ppi[c];
+  }
+}
+
 // Explicit acoustic substeps, psolver=2 (sounde, src/sounde.F:10-1026;
 // Cartesian, no terrain).  The copies the reference makes before the substeps
 // (u3d=ua, ..., ppd=ppx, src/sounde.F:181-233) are folded into the first one
 // (fold: from the second stage on, or where the caller says that u3d..pp3d
-// equal ua..ppi).
+// equal ua..ppi); the border around its points is set with the coefficients.
 void sounde_run(cm1g_model *m, int nrk, bool fold1) {
   const KP P = m->P;
   const int ni = P.ni, nj = P.nj, nk = P.nk;
@@ -1022,10 +1059,22 @@ void sounde_run(cm1g_model *m, int nrk, bool fold1) {
   sub_args(m, nrk, a, &nloop);
   a.expl = 1;
   const bool fold = (nrk >= 2) || fold1;
+  float *u3d = m->f[CM1G_U3D], *v3d = m->f[CM1G_V3D], *w3d = m->f[CM1G_W3D], *pp3d = m->f[CM1G_PP3D];
+  const float *ua = m->f[CM1G_UA], *va = m->f[CM1G_VA], *wa = m->f[CM1G_WA], *ppi = m->f[CM1G_PPI];
   {
     float *cf = m->scoef;
     const float dts = a.dts, rdz = P.rdz, cp = P.K.cp;
-    launch<64>(m, dim3((nk + 63) / 64), dim3(64), [=] __device__(int bx, int, int) {
+    SoundeBorder bd = {u3d, v3d, w3d, pp3d, a.rru, a.rrv, a.rrw, ua, va, wa, ppi};
+    bd.npts = 2 * (ni + 2) + 2 * nj;
+    // (the first stage steps from u3d.. as they are, unless an exchanging
+    // solve3 has left the previous step in them)
+    bd.copy = nrk >= 2 || m->swapped;
+    const int nkb = (nk + 63) / 64;
+    launch<64>(m, dim3(nkb + (bd.npts * nk + 63) / 64), dim3(64), [=] __device__(int bx, int, int) {
+      if (bx >= nkb) {
+        sounde_border(P, bd, (bx - nkb) * 64 + (int)threadIdx.x);
+        return;
+      }
       const int k = 1 + bx * 64 + (int)threadIdx.x;
       if (k > nk) return;
       float *o = cf + 8 * k;
@@ -1047,9 +1096,7 @@ void sounde_run(cm1g_model *m, int nrk, bool fold1) {
   dim3 grd = col_blocks(cg);
   a.nring = ((ni + nj + 1) * nk + (int)blk.x - 1) / (int)blk.x;
   grd.x += a.nring;
-  float *u3d = m->f[CM1G_U3D], *v3d = m->f[CM1G_V3D], *w3d = m->f[CM1G_W3D], *pp3d = m->f[CM1G_PP3D];
   float *ppx = m->f[CM1G_PPX], *ppdb[2] = {m->f[CM1G_DUM7], m->tx};
-  const float *ua = m->f[CM1G_UA], *va = m->f[CM1G_VA], *wa = m->f[CM1G_WA], *ppi = m->f[CM1G_PPI];
   float *us = m->scr1, *vs = m->scr2, *ws = m->ty;
   const float *up = nullptr, *vp = nullptr, *wp = nullptr;
   a.wring = fold ? wa : w3d;

@@ -104,3 +104,52 @@ def test_timer_names_the_kernel_that_runs(require_gpu, nk, kernel):
     N.check(g.L.cm1g_ktimer_stop(g.h, C.byref(ms), C.byref(n), C.byref(b), name, 64), "cm1g_ktimer_stop")
     assert name.value.decode() == kernel and n.value == 2 + 3 + 6
     g.close()
+
+
+BOX = ["u3d", "v3d", "w3d", "pp3d", "ppx", "rru", "rrv", "rrw"]
+
+
+@pytest.mark.parametrize("we,sn", [(1, 1), (2, 2), (1, 2), (2, 1)], ids=["periodic", "open", "we-periodic", "sn-periodic"])
+@pytest.mark.parametrize("ni,nj,nk,nsound", [(8, 9, 6, 2), (13, 8, 9, 5), (70, 11, 8, 10)])
+def test_explicit_routine_whole_boxes(require_gpu, ni, nj, nk, nsound, we, sn):
+    """sounde as a routine, every stage, from arrays that differ everywhere
+    (borders too): whole boxes equal the oracle's."""
+    import ctypes as C
+
+    import pyoracle
+    from cm1_amd import _native as N
+    cfgd, cols, fields = case(ni=ni, nj=nj, nk=nk, nsound=nsound, dz=15000.0 / nk, dt=0.25 * nsound, amp=2.0, psolver=2)
+    cfgd.update(wbc=we, ebc=we, sbc=sn, nbc=sn)
+    g = make_gpu(cfgd, cols, fields)
+    o = make_oracle(cfgd, cols, fields)
+    g.step(1)  # (the open sides' radiation speeds)
+    o.step(1)
+    rng = np.random.default_rng(ni)
+    noise = ("ua", "va", "wa", "ppi", "u3d", "v3d", "w3d", "pp3d", "ppx", "rru", "rrv", "rrw")
+    for nrk in (1, 2, 3):
+        for n in noise:
+            o.f(n)[:] = (rng.standard_normal(o.f(n).shape) * 0.1).astype(np.float32)
+        for n in pyoracle.FIELDS:
+            g.put(n, np.ascontiguousarray(o.f(n)))
+        dttmp = C.c_float(np.float32(cfgd["dt"]) / np.float32(4 - nrk))
+        N.check(g.L.cm1g_sound(g.h, nrk, dttmp), "cm1g_sound")
+        o.L.cm1o_sound(o.h, nrk, dttmp)
+        for n in BOX:
+            assert np.array_equal(g.get(n).view(np.uint32), o.f(n).view(np.uint32)), (nrk, n)
+    g.close()
+
+
+@pytest.mark.parametrize("we,sn", [(1, 1), (2, 2), (1, 2), (2, 1)], ids=["periodic", "open", "we-periodic", "sn-periodic"])
+def test_explicit_step_whole_boxes(require_gpu, we, sn):
+    """Whole steps with the explicit solver: what the halo fills leave in the
+    corners comes from the border the substeps start from."""
+    cfgd, cols, fields = case(ni=13, nj=9, nk=8, nsound=10, dz=15000.0 / 8, dt=2.0, amp=2.0, psolver=2)
+    cfgd.update(wbc=we, ebc=we, sbc=sn, nbc=sn)
+    g = make_gpu(cfgd, cols, fields)
+    o = make_oracle(cfgd, cols, fields)
+    for _ in range(3):  # from equal arrays, then from exchanged buffers
+        g.step(1)
+        o.step(1)
+        for n in ("u3d", "v3d", "w3d", "pp3d"):
+            assert np.array_equal(g.get(n).view(np.uint32), o.f(n).view(np.uint32)), n
+    g.close()
